@@ -153,6 +153,7 @@ static void derive_params(gf::Params& P)
     P.crit2 = std::sqrt(P.crit);
     P.critsq = P.crit * P.crit;
     P.inv16g = 1.0 / (16.0 * P.grav);
+    P.fast = gf::step_params_in_range(P.grav, P.dry_tolerance);
 }
 
 struct Lib {

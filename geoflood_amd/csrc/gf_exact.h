@@ -1,0 +1,142 @@
+// gf_exact.h -- correctly rounded quotients and square roots of the step's
+// inner loops, without the range handling of the general operations.
+//
+// The step kernel is bound by VALU issue, and its ~50 divisions and ~10
+// square roots per cell were a third of the instructions: `a / b` costs 11
+// (two scalings, the quarter-rate reciprocal, two Newton steps, the quotient
+// with its residual correction, and the unscaling and special-case fixups),
+// sqrt about 17.  Two things make them cheaper without changing a bit:
+//
+//  * inside the range below nothing can overflow or lose bits to underflow,
+//    so the scaling and fixup steps have nothing to do;
+//  * quotients with one denominator share its reciprocal: each further one is
+//    a product and one residual correction (3 instructions).
+//
+// Correct rounding.  y is the reciprocal of b after two Newton steps from a
+// seed good to 20 bits or better: its error before the last rounding is below
+// 2^-80, so y is 1/b rounded (or a neighbour of a tie).  q0 = a y is then
+// within one ulp of a/b, the residual r = a - b q0 is exact in one FMA, and
+// q = q0 + r y rounds to the correctly rounded a/b (P. Markstein, "Computation
+// of elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
+// Dev. 34, 1990; J.-M. Muller et al., Handbook of Floating-Point Arithmetic,
+// 2nd ed., 2018, sections 4.7 and 4.8, also for the square root: a Goldschmidt
+// step and two residual corrections).  The residual is exact when
+// |a| >= 2^-960 or a = 0.  A zero quotient loses the sign of its zero.
+//
+// Range.  step_cell_in_range bounds a tile's cells, and
+// step_params_in_range bounds the parameters; a tile that holds anything else
+// (a NaN, a momentum of 1e-80, 10^9 m of water) takes the same step with the
+// general operations.  Write m = 2^-240 for the smallest non-zero momentum or
+// bathymetry.  A non-zero sum of two values is at least 2^-52 of the smaller,
+// so, with drytol >= 2^-14, 2^-4 <= g <= 2^8, h <= 2^30, |hu|, |hv| <= 2^20:
+//   u, v in {0} or [m 2^-30, 2^34]; c = sqrt(g h) in [2^-9, 2^19];
+//   |u| / c <= 2^20 drytol^-3/2 g^-1/2 <= 2^43, so the differences of wave
+//   speeds that divide (s2 - s0, sE2 - sE1, lam0 - lam2) never vanish;
+//   speeds in {0} or [2^-68, 2^36]; |delb| in {0} or [m 2^-52, 2^31];
+//   deldelh >= m 2^-205, hstarHLL (sE2 - sE1) >= m 2^-240,
+//   delh - deldelh >= m 2^-354, the numerators of beta >= m 2^-714 = 2^-954,
+// and every product stays below 2^800.  Two families of numerators have no
+// such bound, because they multiply waves with waves: the limiter's dot
+// products and rpt2's.  They are tested one by one (quotients_tiny) and
+// divided in the general way when they are too small.
+#pragma once
+
+#include <cmath>
+
+#ifndef GF_DEVICE
+#define GF_DEVICE __device__ __forceinline__
+#endif
+
+namespace gf {
+
+GF_DEVICE unsigned long long bits_of(double x) { return __builtin_bit_cast(unsigned long long, x); }
+
+// smallest non-zero |hu|, |hv|, |b| of a fast tile: 2^-240 (zero_or_within)
+constexpr double STEP_MAX_Q = 0x1p20;    // largest |hu|, |hv|
+constexpr double STEP_MAX_H = 0x1p30;    // largest h, |b|
+constexpr int QUOT_MIN_EXP = -900;       // numerators and denominators below 2^-901 divide in the general way
+
+inline bool step_params_in_range(double grav, double drytol)
+{
+    return grav >= 0x1p-4 && grav <= 0x1p8 && drytol >= 0x1p-14 && drytol <= 0x1p10;
+}
+
+// |x| is 0 or lies in [2^-240, hi], by its high word (hi a power of two).
+GF_DEVICE bool zero_or_within(double x, double hi)
+{
+    constexpr unsigned lo = (1023u - 240u) << 20;
+    const unsigned top = (unsigned)(bits_of(hi) >> 32);
+    return x == 0.0 || ((unsigned)(bits_of(x) >> 32) & 0x7fffffffu) - lo < top - lo;
+}
+
+// A cell after b4step2 that the fast quotients are made for.
+GF_DEVICE bool step_cell_in_range(double h, double hu, double hv, double b)
+{
+    return h <= STEP_MAX_H && zero_or_within(hu, STEP_MAX_Q) && zero_or_within(hv, STEP_MAX_Q) &&
+           zero_or_within(b, STEP_MAX_H);
+}
+
+#ifndef GF_SEED_FUNCTIONS
+GF_DEVICE double rcp_seed(double b) { return __builtin_amdgcn_rcp(b); }
+GF_DEVICE double rsq_seed(double b) { return __builtin_amdgcn_rsq(b); }
+GF_DEVICE int exponent_of(double a) { return __builtin_amdgcn_frexp_exp(a); }  // 0 for 0, NaN and Inf
+#endif
+
+// A denominator with its refined reciprocal.
+struct Recip {
+    double b, y;
+};
+
+template <bool FAST>
+GF_DEVICE Recip recip(double b)
+{
+    if (!FAST) return Recip{b, 0.0};
+    double y = rcp_seed(b);
+    y = ::fma(y, ::fma(-b, y, 1.0), y);
+    y = ::fma(y, ::fma(-b, y, 1.0), y);
+    return Recip{b, y};
+}
+
+template <bool FAST>
+GF_DEVICE double quot(double a, const Recip& d)
+{
+    if (!FAST) return a / d.b;
+    const double q = a * d.y;
+    return ::fma(::fma(-d.b, q, a), d.y, q);
+}
+
+template <bool FAST>
+GF_DEVICE double quot(double a, double b)
+{
+    return quot<FAST>(a, recip<FAST>(b));
+}
+
+// sqrt(x); FAST: x = 0 or 2^-700 <= x <= 2^700.
+template <bool FAST>
+GF_DEVICE double root(double x)
+{
+    if (!FAST) return ::sqrt(x);
+    const double y = rsq_seed(::fmax(x, 0x1p-700));
+    double s = x * y, h = 0.5 * y;
+    const double r = ::fma(-h, s, 0.5);
+    s = ::fma(s, r, s);
+    h = ::fma(h, r, h);
+    s = ::fma(::fma(-s, s, x), h, s);
+    return ::fma(::fma(-s, s, x), h, s);
+}
+
+// Maximum and minimum as LLVM Flang evaluates MAX and MIN.  FAST: the
+// operands are numbers and the sign of a zero result does not matter, and one
+// instruction does it instead of a compare and two selects.
+template <bool FAST>
+GF_DEVICE double vmax(double a, double b)
+{
+    return FAST ? ::fmax(a, b) : (a > b ? a : b);
+}
+template <bool FAST>
+GF_DEVICE double vmin(double a, double b)
+{
+    return FAST ? ::fmin(a, b) : (a < b ? a : b);
+}
+
+}  // namespace gf

@@ -57,45 +57,33 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-// Compressed f-waves of one face: wave 1 (3), normal momentum of wave 2 (1),
-// wave 3 (3).  The other two components of wave 2 are exact zeros
-// (geoclaw_riemann_utils.f:289-299: fw(1,2) = beta(2)*r(2,2) = 0, fw(3,2) = 0).
-__device__ __forceinline__ void compress(const double w[3][3], double c[7])
-{
-    c[0] = w[0][0]; c[1] = w[0][1]; c[2] = w[0][2];
-    c[3] = w[1][1];
-    c[4] = w[2][0]; c[5] = w[2][1]; c[6] = w[2][2];
-}
-
 // Dot product of two 3-vectors given in direction-local order (h, n, t),
 // summed in the reference's physical component order (h, hu, hv):
 // x-direction (h, n, t) = (h, hu, hv); y-direction (h, n, t) = (h, hv, hu).
 template <int DIR>
-__device__ __forceinline__ double pdot(double a0, double a1, double a2, double b0, double b1, double b2)
+__device__ __forceinline__ double pdot(const double* a, const double* b)
 {
-    if (DIR == 0) return a0 * b0 + a1 * b1 + a2 * b2;
-    return a0 * b0 + a2 * b2 + a1 * b1;
+    if (DIR == 0) return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
+    return a[0] * b[0] + a[2] * b[2] + a[1] * b[1];
 }
 
 // Limiter, second-order correction and fluctuation split of one face
 // (geoclaw_flux2fw_fort.f:143-224 with geoclaw_limiter_fort.f:34-58 and
-// philim.f).  wc: own compressed unlimited waves; wl / wr: those of the faces
+// philim.f).  w: own compressed unlimited waves; wl / wr: those of the faces
 // before / after along the sweep.  Outputs in direction-local order: faddm,
 // faddp (flux increments) and amdq*, apdq* (fluctuations handed to rpt2).
 // DEF: the default method (order 2, transverse 2, MC limiter on all three
 // families) fixed at compile time; otherwise the method is read from P.
-template <int DIR, bool DEF>
-__device__ __forceinline__ void face_second_order(const double wc[7], const double s[3],
+template <int DIR, bool DEF, bool FAST>
+__device__ __forceinline__ void face_second_order(const double w[7], const double s[3],
                                                   const double wl[7], const double wr[7],
                                                   double dtdx, const Params& P,
                                                   double faddm[3], double faddp[3],
                                                   double amq[3], double apq[3])
 {
-    double w[3][3] = {{wc[0], wc[1], wc[2]}, {0.0, wc[3], 0.0}, {wc[4], wc[5], wc[6]}};
     double amdq[3], apdq[3];
     fluctuations(s, w, amdq, apdq);
     const int order = DEF ? 2 : P.order;
-    const int lim0 = DEF ? 4 : P.mthlim[0], lim1 = DEF ? 4 : P.mthlim[1], lim2 = DEF ? 4 : P.mthlim[2];
     if (order == 1) {
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -106,70 +94,41 @@ __device__ __forceinline__ void face_second_order(const double wc[7], const doub
         }
         return;
     }
-    // limiter on the three wave families with the unlimited neighbours
-    {
-        // wave 1
-        if (lim0 != 0) {
-            const double wn2 = pdot<DIR>(wc[0], wc[1], wc[2], wc[0], wc[1], wc[2]);
-            if (wn2 != 0.0) {
-                const double dotl = pdot<DIR>(wl[0], wl[1], wl[2], wc[0], wc[1], wc[2]);
-                const double dotr = pdot<DIR>(wc[0], wc[1], wc[2], wr[0], wr[1], wr[2]);
-                const double lim = philim(wn2, s[0] > 0.0 ? dotl : dotr, lim0);
-                w[0][0] = lim * w[0][0]; w[0][1] = lim * w[0][1]; w[0][2] = lim * w[0][2];
-            }
-        }
-        // wave 2 (only its normal-momentum component is non-zero)
-        if (lim1 != 0) {
-            const double wn2 = wc[3] * wc[3];
-            if (wn2 != 0.0) {
-                const double dotl = wl[3] * wc[3];
-                const double dotr = wc[3] * wr[3];
-                const double lim = philim(wn2, s[1] > 0.0 ? dotl : dotr, lim1);
-                w[1][1] = lim * w[1][1];
-            }
-        }
-        // wave 3
-        if (lim2 != 0) {
-            const double wn2 = pdot<DIR>(wc[4], wc[5], wc[6], wc[4], wc[5], wc[6]);
-            if (wn2 != 0.0) {
-                const double dotl = pdot<DIR>(wl[4], wl[5], wl[6], wc[4], wc[5], wc[6]);
-                const double dotr = pdot<DIR>(wc[4], wc[5], wc[6], wr[4], wr[5], wr[6]);
-                const double lim = philim(wn2, s[2] > 0.0 ? dotl : dotr, lim2);
-                w[2][0] = lim * w[2][0]; w[2][1] = lim * w[2][1]; w[2][2] = lim * w[2][2];
-            }
-        }
-    }
-    double c[3];
+    // limiter on the three wave families with the unlimited neighbour on the
+    // side the wave comes from (wave 2 has its normal momentum only): the
+    // ratios b / a of the dot products, then the factor of each family (1
+    // where the wave vanishes or its family is not limited)
+    const double a[3] = {pdot<DIR>(w, w), w[3] * w[3], pdot<DIR>(w + 4, w + 4)};
+    const double b[3] = {s[0] > 0.0 ? pdot<DIR>(wl, w) : pdot<DIR>(w, wr),
+                         s[1] > 0.0 ? wl[3] * w[3] : w[3] * wr[3],
+                         s[2] > 0.0 ? pdot<DIR>(wl + 4, w + 4) : pdot<DIR>(w + 4, wr + 4)};
+    double r[3];
 #pragma unroll
-    for (int mw = 0; mw < 3; mw++) c[mw] = copysign(1.0, s[mw]) * (1.0 - fabs(s[mw]) * dtdx);
+    for (int mw = 0; mw < 3; mw++) r[mw] = quot<FAST>(b[mw], a[mw]);
+    const double ab[6] = {a[0], a[1], a[2], b[0], b[1], b[2]};
+    if (FAST && quotients_tiny(ab)) {
+#pragma unroll
+        for (int mw = 0; mw < 3; mw++) r[mw] = b[mw] / a[mw];
+    }
+    double lim[3], c[3];
+#pragma unroll
+    for (int mw = 0; mw < 3; mw++) {
+        const int meth = DEF ? 4 : P.mthlim[mw];
+        lim[mw] = a[mw] != 0.0 && (DEF || meth != 0) ? philim<FAST>(r[mw], meth) : 1.0;
+        c[mw] = copysign(1.0, s[mw]) * (1.0 - fabs(s[mw]) * dtdx);
+    }
     double cq[3];
-    cq[0] = c[0] * w[0][0] + c[2] * w[2][0];
-    cq[1] = c[0] * w[0][1] + c[1] * w[1][1] + c[2] * w[2][1];
-    cq[2] = c[0] * w[0][2] + c[2] * w[2][2];
+    cq[0] = c[0] * (lim[0] * w[0]) + c[2] * (lim[2] * w[4]);
+    cq[1] = c[0] * (lim[0] * w[1]) + c[1] * (lim[1] * w[3]) + c[2] * (lim[2] * w[5]);
+    cq[2] = c[0] * (lim[0] * w[2]) + c[2] * (lim[2] * w[6]);
     const bool fold = DEF ? true : (P.transverse == 2);
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        faddm[k] = amdq[k] + 0.5 * cq[k];
-        faddp[k] = -apdq[k] + 0.5 * cq[k];
+        const double hq = 0.5 * cq[k];
+        faddm[k] = amdq[k] + hq;
+        faddp[k] = -apdq[k] + hq;
         amq[k] = fold ? amdq[k] + cq[k] : amdq[k];
         apq[k] = fold ? apdq[k] - cq[k] : apdq[k];
-    }
-}
-
-// Transverse increments of one cell from the two normal fluctuations that
-// its state splits (geoclaw_flux2fw_fort.f:232-265): G1 (below/left) and G2
-// (above/right), direction-local order, hd = dt/dx / 2.
-__device__ __forceinline__ void cell_transverse(const Rpt2Cell& C, const double am_next[3],
-                                                const double ap_own[3], double hd,
-                                                double G1[3], double G2[3])
-{
-    double bm1[3], bp1[3], bm2[3], bp2[3];
-    rpt2_apply(C, am_next, bm1, bp1);
-    rpt2_apply(C, ap_own, bm2, bp2);
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        G1[k] = -(hd * bm1[k]) - hd * bm2[k];
-        G2[k] = -(hd * bp1[k]) - hd * bp2[k];
     }
 }
 
@@ -215,162 +174,20 @@ __device__ __forceinline__ void block_max2(double& a, double& b, double* red, in
     }
 }
 
-// The whole step of one tile of a patch by one workgroup of NT threads.  A
-// tile is the TX x TY block of interior cells at offset (ox, oy) of an
-// MX x MY patch (TX = MX, TY = MY: the whole patch) with its own 2-cell
-// halo: the update of an interior cell reaches two cells in each direction
-// (limiter and transverse corrections), so a tile computes exactly what the
-// whole-patch step computes for its cells.  q_src / q_dst are the pool's
-// source and destination buffers (q_dst == q_src updates in place).  With
-// PULL the halo cells outside the patch are gathered from the neighbours'
-// interiors in q_src (same-level exchange and physical sides fused into the
-// load); otherwise the stored ghost cells are used; halo cells inside the
-// patch are its own interior.  Thread 0 receives the tile's maximum CFL
-// number (uncapped) and the maximum interior depth after the step.
-//
-// A workgroup may step several patches at once, one per group of NT
-// threads (ltid: the thread's index in its group; T, E, F, red: the group's
-// slices of LDS).  The groups pass every barrier together, so the all-dry
-// fast path is taken only when every group's tile is dry (the full path
-// gives the same values on a dry tile).  A group without a patch (valid
-// false: the last item of the work list) computes on a zero tile and writes
-// nothing.  FREG: the x-face flux increments stay in the owning thread's
-// registers between the x and the y phase (the thread that forms a face's
-// increments is the one that reads them back) instead of in LDS -- the "LDS
-// split" of a step variant.
-//
-// Hook: called by thread NT-1 (of group 0) right after the tile is in LDS:
-// that thread has no position in the last slot, so its wave has slack in
-// the phases that follow.
-struct NoHook {
-    __device__ void operator()() const {}
-};
-
-template <int MX, int MY, int TX, int TY, int NT, bool PULL, bool DEF, bool FREG = false, typename Hook = NoHook>
-__device__ __forceinline__ void step_patch(double* T, double* E, double* F, double* red, const PatchDesc* dptr, int patch,
-                           int ox, int oy, const double* q_src, double* q_dst, const double* aux,
-                           double dt, const Params& P, double& cfl_res, double& hmax_res,
-                           int ltid, bool valid, const Hook& hook = Hook())
+// The step of one tile in LDS (T: h, hu, hv, b after b4step2, at least one
+// cell wet), by a group of NT threads; arguments as in step_patch.  FAST: every
+// cell and parameter lies in the range of gf_exact.h.
+template <int MX, int MY, int TX, int TY, int NT, bool DEF, bool FREG, bool FAST>
+__device__ __forceinline__ void step_tile(const double* T, double* E, double* F, double* red, int ox, int oy,
+                                          double* dst, double dtdx, double dtdy, double dt, const Params& P,
+                                          double& cfl_res, double& hmax_res, int tid, bool valid)
 {
     using G = Geo<TX, TY>;   // tile geometry (LDS)
     using GP = Geo<MX, MY>;  // patch geometry (HBM)
-    constexpr int NXP = G::NXP, NP2 = G::NP2, PX = G::PX, NPOS = G::NPOS;
+    constexpr int NP2 = G::NP2, PX = G::PX, NPOS = G::NPOS;
     constexpr int PNP2 = GP::NP2;
     constexpr int SLOTS = (NPOS + NT - 1) / NT;
-    // Opaque copy of the thread index: inside the persistent loop this stops
-    // the compiler from hoisting every index computation of the body out of
-    // the loop, which would keep them live in registers across iterations.
-    int tid = ltid;
-    asm volatile("" : "+v"(tid));
-    const double* src = q_src + (size_t)patch * 3 * PNP2;
-    double* dst = q_dst + (size_t)patch * 3 * PNP2;
-    const double* auxp = aux + (size_t)patch * PNP2;
     const double g = P.grav, drytol = P.dry_tolerance;
-    const double dtdx = dt / dptr->dx;
-    const double dtdy = dt / dptr->dy;
-
-    // ---- tile load (+ halo gather) + b4step2 (geoclaw_b4step2_fort.f90:153-156) ----
-    // Addresses of every cell this thread loads first, then all loads, then
-    // the LDS stores: one memory round trip per tile instead of one per cell
-    // group.
-    constexpr int LS = (NP2 + NT - 1) / NT;
-    const double* lbase[LS];
-    int lk[LS], lpc[LS];
-    bool lok[LS], lnu[LS], lnv[LS];
-#pragma unroll
-    for (int r = 0; r < LS; r++) {
-        const int c = tid + r * NT;
-        lok[r] = valid && c < NP2;
-        const int cc = lok[r] ? c : 0;
-        const int fi = ox + cc % NXP - 1, fj = oy + cc / NXP - 1;  // patch Fortran indices
-        const int pc = GP::ti(fi, fj);
-        const double* base = src;
-        int k = pc;
-        bool nu = false, nv = false;
-        if (PULL) {
-            const bool interior = (fi >= 1 && fi <= MX && fj >= 1 && fj <= MY);
-            int sp = patch, si = fi, sj = fj;
-            if (!interior && ghost_source<MX, MY>(dptr->nbr, patch, fi, fj, sp, si, sj, nu, nv)) {
-                base = q_src + (size_t)sp * 3 * PNP2;
-                k = GP::ti(si, sj);
-            }
-        }
-        lbase[r] = base;
-        lk[r] = k;
-        lpc[r] = pc;
-        lnu[r] = nu;
-        lnv[r] = nv;
-    }
-    double lh[LS], lhu[LS], lhv[LS], lb[LS];
-#pragma unroll
-    for (int r = 0; r < LS; r++) {
-        if (lok[r]) {
-            lh[r] = lbase[r][lk[r]];
-            lhu[r] = lbase[r][PNP2 + lk[r]];
-            lhv[r] = lbase[r][2 * PNP2 + lk[r]];
-            lb[r] = auxp[lpc[r]];
-        }
-    }
-    int wet = 0;
-#pragma unroll
-    for (int r = 0; r < LS; r++) {
-        if (lok[r]) {
-            const int c = tid + r * NT;
-            double h = lh[r], hu = lnu[r] ? -lhu[r] : lhu[r], hv = lnv[r] ? -lhv[r] : lhv[r];
-            if (h < drytol) {
-                h = fmaxf64(h, 0.0);
-                hu = 0.0;
-                hv = 0.0;
-            }
-            T[c] = h;
-            T[NP2 + c] = hu;
-            T[2 * NP2 + c] = hv;
-            T[3 * NP2 + c] = lb[r];
-            wet |= (h > drytol);
-        } else if (!valid && tid + r * NT < NP2) {
-            const int c = tid + r * NT;  // a group without a patch: a dry zero tile
-            T[c] = 0.0;
-            T[NP2 + c] = 0.0;
-            T[2 * NP2 + c] = 0.0;
-            T[3 * NP2 + c] = 0.0;
-        }
-    }
-    const int anywet = __syncthreads_or(wet);
-    static_assert(NT - 1 + NT * (SLOTS - 1) >= G::NPOS || SLOTS == 1,
-                  "the hook thread must have no position in the last slot");
-    if (threadIdx.x == NT - 1) hook();
-
-    if (!anywet) {
-        // Every face of the tile is dry on both sides: all fluctuations, waves
-        // and transverse splits are zero and the update leaves q unchanged, so
-        // the step reduces to b4step2 + src2 on the interior and CFL = 0.
-        double hm = 0.0;
-        bool bad = false;
-        for (int c = tid; c < TX * TY; c += NT) {
-            const int i = c % TX + 1, j = c / TX + 1;
-            const int k = G::ti(i, j);
-            const int pk = GP::ti(ox + i, oy + j);
-            double h = T[k], hu = T[NP2 + k], hv = T[2 * NP2 + k];
-            if (P.src_term > 0) src2_cell(h, hu, hv, T[3 * NP2 + k], dt, P);
-            if (valid) {
-                dst[pk] = h;
-                dst[PNP2 + pk] = hu;
-                dst[2 * PNP2 + pk] = hv;
-            }
-            hm = fmaxf64(hm, h);
-            bad |= !finite3(h, hu, hv);
-        }
-        // a non-finite cell (a NaN depth is neither wet nor dry) makes the
-        // tile's CFL number NaN, which stops the scenario
-        if (bad) hm = quiet_nan();
-        hm = block_max<NT>(hm, red, tid);
-        if (tid == 0) {
-            cfl_res = hm != hm ? quiet_nan() : 0.0;
-            hmax_res = hm;
-        }
-        return;
-    }
-
     int pi[SLOTS], pj[SLOTS];
     bool in[SLOTS];
 #pragma unroll
@@ -381,7 +198,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
         pj[s] = p / PX;
     }
 
-    double cfl = 0.0;
+    double smax = 0.0;  // largest |s| of the direction's faces: max |s| dt/dx = (max |s|) dt/dx, rounded too
     // A face's own compressed waves go to LDS for its neighbours' limiter and
     // are read back from there by the face itself, so that they do not stay
     // in registers while the other slots solve their Riemann problems.
@@ -393,18 +210,14 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     // the extra registers are free (up to 168 at three waves per SIMD), while
     // the other variants' occupancy is set by registers.
     constexpr bool OWN = TX >= 32 && TY >= 32 && NT <= 768;
-    double CU[SLOTS], CV[SLOTS], CS[SLOTS];
+    CellVel C[SLOTS];
 #pragma unroll
     for (int s = 0; s < SLOTS; s++) {
-        CU[s] = 0.0; CV[s] = 0.0; CS[s] = 0.0;
+        C[s] = CellVel{0.0, 0.0, 0.0, 0.0};
         if (OWN) {
             const int k = G::ti(pi[s], pj[s]);
             const double h = in[s] ? T[k] : 0.0;
-            if (h > drytol) {
-                CU[s] = T[NP2 + k] / h;
-                CV[s] = T[2 * NP2 + k] / h;
-                CS[s] = sqrt(g * h);
-            }
+            if (h > drytol) C[s] = cell_velocity<FAST>(h, T[NP2 + k], T[2 * NP2 + k], g);
         }
     }
     double AP[SLOTS][3], AM[SLOTS][3], GA[SLOTS][3], GB[SLOTS][3];
@@ -415,21 +228,14 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     for (int s = 0; s < SLOTS; s++) {
         const int i = pi[s], j = pj[s];
         double sw[3] = {0.0, 0.0, 0.0};
-        double w[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+        double wc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (in[s] && j <= TY + 1) {
             const int kL = G::ti(i - 1, j), kR = G::ti(i, j);
-            rpn2_face<OWN>(T[kL], T[NP2 + kL], T[2 * NP2 + kL], T[3 * NP2 + kL],
-                           T[kR], T[NP2 + kR], T[2 * NP2 + kR], T[3 * NP2 + kR], P, sw, w,
-                           RightCell{CU[s], CV[s], CS[s]});
+            rpn2_face<FAST, OWN>(T[kL], T[NP2 + kL], T[2 * NP2 + kL], T[3 * NP2 + kL],
+                                 T[kR], T[NP2 + kR], T[2 * NP2 + kR], T[3 * NP2 + kR], P, sw, wc, C[s]);
 #pragma unroll
-            for (int mw = 0; mw < 3; mw++) {
-                const double v = dtdx * sw[mw];
-                cfl = fmaxf64(cfl, v);
-                cfl = fmaxf64(cfl, -v);
-            }
+            for (int mw = 0; mw < 3; mw++) smax = vmax<FAST>(smax, fabs(sw[mw]));
         }
-        double wc[7];
-        compress(w, wc);
         Sr[s][0] = sw[0]; Sr[s][1] = sw[1]; Sr[s][2] = sw[2];
         if (in[s]) {
             const int p = tid + s * NT;
@@ -438,6 +244,9 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
         }
     }
     __syncthreads();
+
+    double cfl = dtdx * smax;
+    smax = 0.0;
 
     // ================= x-faces: limiter + corrections =================
 #pragma unroll
@@ -453,7 +262,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
                 wr[k] = E[k * NPOS + p + 1];
             }
             double fxm[3], fxp[3];
-            face_second_order<0, DEF>(wc, Sr[s], wl, wr, dtdx, P, fxm, fxp, AM[s], AP[s]);
+            face_second_order<0, DEF, FAST>(wc, Sr[s], wl, wr, dtdx, P, fxm, fxp, AM[s], AP[s]);
             if constexpr (FREG) {
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
@@ -494,13 +303,11 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
         for (int k = 0; k < 3; k++) { GA[s][k] = 0.0; GB[s][k] = 0.0; }
         if (transverse && in[s] && i >= 1 && i <= TX && j <= TY + 1) {
             const int kc = G::ti(i, j);
-            const Rpt2Cell C =
-                OWN ? rpt2_setup_c(T[kc], CU[s], CV[s], CS[s], T[3 * NP2 + kc], T[3 * NP2 + G::ti(i, j - 1)],
-                                   T[3 * NP2 + G::ti(i, j + 1)], drytol)
-                    : rpt2_setup(T[kc], T[NP2 + kc], T[2 * NP2 + kc], T[3 * NP2 + kc], T[3 * NP2 + G::ti(i, j - 1)],
-                                 T[3 * NP2 + G::ti(i, j + 1)], g, drytol);
+            const CellVel V = OWN ? C[s] : cell_velocity<FAST>(T[kc], T[NP2 + kc], T[2 * NP2 + kc], g);
+            const Rpt2Cell R = rpt2_setup(T[kc], V.u, V.v, V.sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i, j - 1)],
+                                          T[3 * NP2 + G::ti(i, j + 1)], drytol);
             const double amn[3] = {E[p + 1], E[NPOS + p + 1], E[2 * NPOS + p + 1]};
-            cell_transverse(C, amn, AP[s], hdx, GA[s], GB[s]);  // GA = G1 (below), GB = G2 (above)
+            cell_transverse<FAST>(R, amn, AP[s], hdx, GA[s], GB[s]);  // GA = G1 (below), GB = G2 (above)
         }
     }
     __syncthreads();
@@ -533,22 +340,16 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     for (int s = 0; s < SLOTS; s++) {
         const int i = pi[s], j = pj[s];
         double sw[3] = {0.0, 0.0, 0.0};
-        double w[3][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
+        double wc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (in[s] && i <= TX + 1) {
             const int kL = G::ti(i, j - 1), kR = G::ti(i, j);
             // direction-local order for y: (h, hv, hu)
-            rpn2_face<OWN>(T[kL], T[2 * NP2 + kL], T[NP2 + kL], T[3 * NP2 + kL],
-                           T[kR], T[2 * NP2 + kR], T[NP2 + kR], T[3 * NP2 + kR], P, sw, w,
-                           RightCell{CV[s], CU[s], CS[s]});
+            rpn2_face<FAST, OWN>(T[kL], T[2 * NP2 + kL], T[NP2 + kL], T[3 * NP2 + kL],
+                                 T[kR], T[2 * NP2 + kR], T[NP2 + kR], T[3 * NP2 + kR], P, sw, wc,
+                                 CellVel{C[s].v, C[s].u, C[s].sg, C[s].y});
 #pragma unroll
-            for (int mw = 0; mw < 3; mw++) {
-                const double v = dtdy * sw[mw];
-                cfl = fmaxf64(cfl, v);
-                cfl = fmaxf64(cfl, -v);
-            }
+            for (int mw = 0; mw < 3; mw++) smax = vmax<FAST>(smax, fabs(sw[mw]));
         }
-        double wc[7];
-        compress(w, wc);
         Sr[s][0] = sw[0]; Sr[s][1] = sw[1]; Sr[s][2] = sw[2];
         if (in[s]) {
             const int p = tid + s * NT;
@@ -574,7 +375,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
                 wc[k] = E[k * NPOS + p];
                 wr[k] = E[k * NPOS + p + PX];
             }
-            face_second_order<1, DEF>(wc, Sr[s], wl, wr, dtdy, P, fm, fp, AM[s], AP[s]);
+            face_second_order<1, DEF, FAST>(wc, Sr[s], wl, wr, dtdy, P, fm, fp, AM[s], AP[s]);
             // gm = GT + faddm in physical order (h, hu, hv) = local (0, 2, 1)
             GMr[s][0] = GT[s][0] + fm[0];
             GMr[s][1] = GT[s][1] + fm[2];
@@ -604,13 +405,11 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
         for (int k = 0; k < 3; k++) { GA[s][k] = 0.0; GB[s][k] = 0.0; }
         if (transverse && in[s] && i <= TX + 1 && j >= 1 && j <= TY) {
             const int kc = G::ti(i, j);
-            const Rpt2Cell C =
-                OWN ? rpt2_setup_c(T[kc], CV[s], CU[s], CS[s], T[3 * NP2 + kc], T[3 * NP2 + G::ti(i - 1, j)],
-                                   T[3 * NP2 + G::ti(i + 1, j)], drytol)
-                    : rpt2_setup(T[kc], T[2 * NP2 + kc], T[NP2 + kc], T[3 * NP2 + kc], T[3 * NP2 + G::ti(i - 1, j)],
-                                 T[3 * NP2 + G::ti(i + 1, j)], g, drytol);
+            const CellVel V = OWN ? C[s] : cell_velocity<FAST>(T[kc], T[NP2 + kc], T[2 * NP2 + kc], g);
+            const Rpt2Cell R = rpt2_setup(T[kc], V.v, V.u, V.sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i - 1, j)],
+                                          T[3 * NP2 + G::ti(i + 1, j)], drytol);
             const double amn[3] = {E[p + PX], E[NPOS + p + PX], E[2 * NPOS + p + PX]};
-            cell_transverse(C, amn, AP[s], hdy, GA[s], GB[s]);  // GA = left (side 1), GB = right (side 2)
+            cell_transverse<FAST>(R, amn, AP[s], hdy, GA[s], GB[s]);  // GA = left (side 1), GB = right (side 2)
         }
     }
     __syncthreads();
@@ -676,7 +475,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
                 const double gmt = E[(3 + m) * NPOS + p + PX];
                 qn[m] = T[m * NP2 + k] - dtdx * (fmr - FPr[s][m]) - dtdy * (gmt - GPr[s][m]);
             }
-            if (P.src_term > 0) src2_cell(qn[0], qn[1], qn[2], T[3 * NP2 + k], dt, P);
+            if (P.src_term > 0) src2_cell<FAST>(qn[0], qn[1], qn[2], T[3 * NP2 + k], dt, P);
             dst[pk] = qn[0];
             dst[PNP2 + pk] = qn[1];
             dst[2 * PNP2 + pk] = qn[2];
@@ -688,12 +487,178 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     // ================= CFL and depth reductions =================
     // (the per-patch MAXCFL_CAP is applied by the caller, once per patch; a
     // non-finite new state makes the CFL number NaN, which the cap keeps)
+    cfl = fmaxf64(cfl, dtdy * smax);
     double v = bad ? quiet_nan() : cfl, hmx = hm;
     block_max2<NT>(v, hmx, red, tid);
     if (tid == 0) {
         cfl_res = v;
         hmax_res = hmx;
     }
+}
+
+// The whole step of one tile of a patch by one workgroup of NT threads.  A
+// tile is the TX x TY block of interior cells at offset (ox, oy) of an
+// MX x MY patch (TX = MX, TY = MY: the whole patch) with its own 2-cell
+// halo: the update of an interior cell reaches two cells in each direction
+// (limiter and transverse corrections), so a tile computes exactly what the
+// whole-patch step computes for its cells.  q_src / q_dst are the pool's
+// source and destination buffers (q_dst == q_src updates in place).  With
+// PULL the halo cells outside the patch are gathered from the neighbours'
+// interiors in q_src (same-level exchange and physical sides fused into the
+// load); otherwise the stored ghost cells are used; halo cells inside the
+// patch are its own interior.  Thread 0 receives the tile's maximum CFL
+// number (uncapped) and the maximum interior depth after the step.
+//
+// A workgroup may step several patches at once, one per group of NT
+// threads (ltid: the thread's index in its group; T, E, F, red: the group's
+// slices of LDS).  The groups pass every barrier together, so the all-dry
+// fast path is taken only when every group's tile is dry (the full path
+// gives the same values on a dry tile).  A group without a patch (valid
+// false: the last item of the work list) computes on a zero tile and writes
+// nothing.  FREG: the x-face flux increments stay in the owning thread's
+// registers between the x and the y phase (the thread that forms a face's
+// increments is the one that reads them back) instead of in LDS -- the "LDS
+// split" of a step variant.
+//
+// Hook: called by thread NT-1 (of group 0) right after the tile is in LDS:
+// that thread has no position in the last slot, so its wave has slack in
+// the phases that follow.
+struct NoHook {
+    __device__ void operator()() const {}
+};
+
+template <int MX, int MY, int TX, int TY, int NT, bool PULL, bool DEF, bool FREG = false, typename Hook = NoHook>
+__device__ __forceinline__ void step_patch(double* T, double* E, double* F, double* red, const PatchDesc* dptr, int patch,
+                           int ox, int oy, const double* q_src, double* q_dst, const double* aux,
+                           double dt, const Params& P, double& cfl_res, double& hmax_res,
+                           int ltid, bool valid, const Hook& hook = Hook())
+{
+    using G = Geo<TX, TY>;   // tile geometry (LDS)
+    using GP = Geo<MX, MY>;  // patch geometry (HBM)
+    constexpr int NXP = G::NXP, NP2 = G::NP2, PX = G::PX, NPOS = G::NPOS;
+    constexpr int PNP2 = GP::NP2;
+    constexpr int SLOTS = (NPOS + NT - 1) / NT;
+    // Opaque copy of the thread index: inside the persistent loop this stops
+    // the compiler from hoisting every index computation of the body out of
+    // the loop, which would keep them live in registers across iterations.
+    int tid = ltid;
+    asm volatile("" : "+v"(tid));
+    const double* src = q_src + (size_t)patch * 3 * PNP2;
+    double* dst = q_dst + (size_t)patch * 3 * PNP2;
+    const double* auxp = aux + (size_t)patch * PNP2;
+    const double drytol = P.dry_tolerance;
+    const double dtdx = dt / dptr->dx;
+    const double dtdy = dt / dptr->dy;
+
+    // ---- tile load (+ halo gather) + b4step2 (geoclaw_b4step2_fort.f90:153-156) ----
+    // Addresses of every cell this thread loads first, then all loads, then
+    // the LDS stores: one memory round trip per tile instead of one per cell
+    // group.
+    constexpr int LS = (NP2 + NT - 1) / NT;
+    const double* lbase[LS];
+    int lk[LS], lpc[LS];
+    bool lok[LS], lnu[LS], lnv[LS];
+#pragma unroll
+    for (int r = 0; r < LS; r++) {
+        const int c = tid + r * NT;
+        lok[r] = valid && c < NP2;
+        const int cc = lok[r] ? c : 0;
+        const int fi = ox + cc % NXP - 1, fj = oy + cc / NXP - 1;  // patch Fortran indices
+        const int pc = GP::ti(fi, fj);
+        const double* base = src;
+        int k = pc;
+        bool nu = false, nv = false;
+        if (PULL) {
+            const bool interior = (fi >= 1 && fi <= MX && fj >= 1 && fj <= MY);
+            int sp = patch, si = fi, sj = fj;
+            if (!interior && ghost_source<MX, MY>(dptr->nbr, patch, fi, fj, sp, si, sj, nu, nv)) {
+                base = q_src + (size_t)sp * 3 * PNP2;
+                k = GP::ti(si, sj);
+            }
+        }
+        lbase[r] = base;
+        lk[r] = k;
+        lpc[r] = pc;
+        lnu[r] = nu;
+        lnv[r] = nv;
+    }
+    double lh[LS], lhu[LS], lhv[LS], lb[LS];
+#pragma unroll
+    for (int r = 0; r < LS; r++) {
+        if (lok[r]) {
+            lh[r] = lbase[r][lk[r]];
+            lhu[r] = lbase[r][PNP2 + lk[r]];
+            lhv[r] = lbase[r][2 * PNP2 + lk[r]];
+            lb[r] = auxp[lpc[r]];
+        }
+    }
+    // bit 0: a wet cell; bit 1: a cell, a parameter or a step size outside the
+    // range of the fast quotients (gf_exact.h)
+    int wet = 0;
+    if (!(P.fast && dtdx >= 0x1p-100 && dtdx <= 0x1p100 && dtdy >= 0x1p-100 && dtdy <= 0x1p100)) wet = 2;
+#pragma unroll
+    for (int r = 0; r < LS; r++) {
+        if (lok[r]) {
+            const int c = tid + r * NT;
+            double h = lh[r], hu = lnu[r] ? -lhu[r] : lhu[r], hv = lnv[r] ? -lhv[r] : lhv[r];
+            if (h < drytol) {
+                h = fmaxf64(h, 0.0);
+                hu = 0.0;
+                hv = 0.0;
+            }
+            T[c] = h;
+            T[NP2 + c] = hu;
+            T[2 * NP2 + c] = hv;
+            T[3 * NP2 + c] = lb[r];
+            wet |= (h > drytol) | (step_cell_in_range(h, hu, hv, lb[r]) ? 0 : 2);
+        } else if (!valid && tid + r * NT < NP2) {
+            const int c = tid + r * NT;  // a group without a patch: a dry zero tile
+            T[c] = 0.0;
+            T[NP2 + c] = 0.0;
+            T[2 * NP2 + c] = 0.0;
+            T[3 * NP2 + c] = 0.0;
+        }
+    }
+    const int flags = __syncthreads_or(wet);
+    static_assert(NT - 1 + NT * (SLOTS - 1) >= G::NPOS || SLOTS == 1,
+                  "the hook thread must have no position in the last slot");
+    if (threadIdx.x == NT - 1) hook();
+
+    if (!(flags & 1)) {
+        // Every face of the tile is dry on both sides: all fluctuations, waves
+        // and transverse splits are zero and the update leaves q unchanged, so
+        // the step reduces to b4step2 + src2 on the interior and CFL = 0.
+        double hm = 0.0;
+        bool bad = false;
+        for (int c = tid; c < TX * TY; c += NT) {
+            const int i = c % TX + 1, j = c / TX + 1;
+            const int k = G::ti(i, j);
+            const int pk = GP::ti(ox + i, oy + j);
+            double h = T[k], hu = T[NP2 + k], hv = T[2 * NP2 + k];
+            if (P.src_term > 0) src2_cell<false>(h, hu, hv, T[3 * NP2 + k], dt, P);
+            if (valid) {
+                dst[pk] = h;
+                dst[PNP2 + pk] = hu;
+                dst[2 * PNP2 + pk] = hv;
+            }
+            hm = fmaxf64(hm, h);
+            bad |= !finite3(h, hu, hv);
+        }
+        // a non-finite cell (a NaN depth is neither wet nor dry) makes the
+        // tile's CFL number NaN, which stops the scenario
+        if (bad) hm = quiet_nan();
+        hm = block_max<NT>(hm, red, tid);
+        if (tid == 0) {
+            cfl_res = hm != hm ? quiet_nan() : 0.0;
+            hmax_res = hm;
+        }
+        return;
+    }
+
+    if (flags & 2)
+        step_tile<MX, MY, TX, TY, NT, DEF, FREG, false>(T, E, F, red, ox, oy, dst, dtdx, dtdy, dt, P, cfl_res, hmax_res, tid, valid);
+    else
+        step_tile<MX, MY, TX, TY, NT, DEF, FREG, true>(T, E, F, red, ox, oy, dst, dtdx, dtdy, dt, P, cfl_res, hmax_res, tid, valid);
 }
 
 // Tile decomposition of an MX x MY patch into TX x TY tiles.
@@ -940,7 +905,7 @@ __device__ __forceinline__ void dry_item(const BatchArgs* pa, int k, int next, i
             P.manning_n = c->manning_n;
             hu = src[NP2 + kk[r]];
             hv = src[2 * NP2 + kk[r]];
-            if (P.src_term > 0) src2_cell(h, hu, hv, a.aux[(size_t)pt * NP2 + kk[r]], c->dt, P);
+            if (P.src_term > 0) src2_cell<false>(h, hu, hv, a.aux[(size_t)pt * NP2 + kk[r]], c->dt, P);
             // a NaN depth lands here too: it sets the scenario's CFL maximum
             // to NaN, which stops the scenario at the controller
             if (!finite3(h, hu, hv))
