@@ -1905,7 +1905,7 @@ try {
         p->wet_grid = 0;
         double tot = 0.0;
         for (int r = 0; r <= reps; r++) {  // the first run warms up
-            HIPCHK(hipMemsetAsync(p->counters + gf::NEXT_WET, 0, sizeof(int), g.stream));
+            HIPCHK(hipMemsetAsync(p->counters + gf::CURSOR_LINE, 0, gf::CURSOR_LINE * gf::QUEUES * sizeof(int), g.stream));
             HIPCHK(hipEventRecord(g.ev_tune[0], g.stream));
             HIPCHK(gf::launch_all(p->mx, p->my, v, gf::default_method(g.P), p->d_args, wet_grid(p), g.stream));
             HIPCHK(hipEventRecord(g.ev_tune[1], g.stream));

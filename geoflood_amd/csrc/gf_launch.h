@@ -108,8 +108,14 @@ struct InflowArgs {
 // Dry-list entries carry the patch's current buffer: patch | cur << 30.
 constexpr int DRY_CUR_SHIFT = 30;
 
-// Device counters of the batched path (BatchArgs::counters).
-enum { CNT_WET = 0, CNT_DRY = 1, NEXT_WET = 2, CNT_SKIP = 3, NCOUNTERS = 4 };
+// Device counters of the batched path (BatchArgs::counters): the list lengths,
+// then one cursor per item queue of the persistent step kernel, each in a
+// 128-byte line of its own.  Workgroup b serves queue b % QUEUES, which is its
+// XCD under the round-robin dispatch, and its first item is b itself: atomics
+// on one cursor were served one at a time, 20-50 ns each, by the 512-2,048
+// workgroups of a launch at once (a launch over 64 8x8 patches took 110 us of
+// which the work is a quarter).
+enum { CNT_WET = 0, CNT_DRY = 1, CNT_SKIP = 2, CURSOR_LINE = 32, QUEUES = 8, NCOUNTERS = CURSOR_LINE * (1 + QUEUES) };
 
 // Steady dry patches.  A dry patch whose cells are all below dry_tolerance
 // steps to (max(h,0), 0, 0), which is idempotent: after two such steps into

@@ -174,12 +174,17 @@ __device__ __forceinline__ void block_max2(double& a, double& b, double* red, in
     }
 }
 
+// Device memory named as such: an access through a pointer that was itself
+// read from memory would otherwise be a flat one, which also waits for LDS.
+using gdouble = __attribute__((address_space(1))) double;
+using gint = __attribute__((address_space(1))) int;
+
 // The step of one tile in LDS (T: h, hu, hv, b after b4step2, at least one
 // cell wet), by a group of NT threads; arguments as in step_patch.  FAST: every
 // cell and parameter lies in the range of gf_exact.h.
 template <int MX, int MY, int TX, int TY, int NT, bool DEF, bool FREG, bool FAST>
 __device__ __forceinline__ void step_tile(const double* T, double* E, double* F, double* red, int ox, int oy,
-                                          double* dst, double dtdx, double dtdy, double dt, const Params& P,
+                                          gdouble* dst, double dtdx, double dtdy, double dt, const Params& P,
                                           double& cfl_res, double& hmax_res, int tid, bool valid)
 {
     using G = Geo<TX, TY>;   // tile geometry (LDS)
@@ -496,6 +501,28 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
     }
 }
 
+// A value that is the same in every lane of the wave, in scalar registers:
+// what an item reads from LDS or through the argument block would otherwise
+// hold vector registers through the whole step.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uniform(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)uniform((int)b), hi = (unsigned)uniform((int)(b >> 32));
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+__device__ __forceinline__ Params uniform(const Params& p)
+{
+    constexpr int W = sizeof(Params) / sizeof(int);
+    int w[W];
+    __builtin_memcpy(w, &p, sizeof(Params));
+#pragma unroll
+    for (int k = 0; k < W; k++) w[k] = uniform(w[k]);
+    Params u;
+    __builtin_memcpy(&u, w, sizeof(Params));
+    return u;
+}
+
 // The whole step of one tile of a patch by one workgroup of NT threads.  A
 // tile is the TX x TY block of interior cells at offset (ox, oy) of an
 // MX x MY patch (TX = MX, TY = MY: the whole patch) with its own 2-cell
@@ -529,7 +556,7 @@ struct NoHook {
 
 template <int MX, int MY, int TX, int TY, int NT, bool PULL, bool DEF, bool FREG = false, typename Hook = NoHook>
 __device__ __forceinline__ void step_patch(double* T, double* E, double* F, double* red, const PatchDesc* dptr, int patch,
-                           int ox, int oy, const double* q_src, double* q_dst, const double* aux,
+                           int ox, int oy, const gdouble* q_src, gdouble* q_dst, const gdouble* aux,
                            double dt, const Params& P, double& cfl_res, double& hmax_res,
                            int ltid, bool valid, const Hook& hook = Hook())
 {
@@ -543,19 +570,19 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     // the loop, which would keep them live in registers across iterations.
     int tid = ltid;
     asm volatile("" : "+v"(tid));
-    const double* src = q_src + (size_t)patch * 3 * PNP2;
-    double* dst = q_dst + (size_t)patch * 3 * PNP2;
-    const double* auxp = aux + (size_t)patch * PNP2;
+    const gdouble* src = q_src + (size_t)patch * 3 * PNP2;
+    gdouble* dst = q_dst + (size_t)patch * 3 * PNP2;
+    const gdouble* auxp = aux + (size_t)patch * PNP2;
     const double drytol = P.dry_tolerance;
-    const double dtdx = dt / dptr->dx;
-    const double dtdy = dt / dptr->dy;
+    const double dtdx = uniform(dt / dptr->dx);
+    const double dtdy = uniform(dt / dptr->dy);
 
     // ---- tile load (+ halo gather) + b4step2 (geoclaw_b4step2_fort.f90:153-156) ----
     // Addresses of every cell this thread loads first, then all loads, then
     // the LDS stores: one memory round trip per tile instead of one per cell
     // group.
     constexpr int LS = (NP2 + NT - 1) / NT;
-    const double* lbase[LS];
+    const gdouble* lbase[LS];
     int lk[LS], lpc[LS];
     bool lok[LS], lnu[LS], lnv[LS];
 #pragma unroll
@@ -565,7 +592,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
         const int cc = lok[r] ? c : 0;
         const int fi = ox + cc % NXP - 1, fj = oy + cc / NXP - 1;  // patch Fortran indices
         const int pc = GP::ti(fi, fj);
-        const double* base = src;
+        const gdouble* base = src;
         int k = pc;
         bool nu = false, nv = false;
         if (PULL) {
@@ -710,11 +737,11 @@ __global__ void __launch_bounds__(NT) k_step(StepArgs a)
     const int patch = a.first + bid / TL::NTILES;
     int ox, oy;
     TL::origin(bid % TL::NTILES, ox, oy);
-    const double* src = a.cur ? a.q1 : a.q0;
-    double* dst = a.q1 ? (a.cur ? a.q0 : a.q1) : a.q0;
+    const gdouble* src = (const gdouble*)(a.cur ? a.q1 : a.q0);
+    gdouble* dst = (gdouble*)(a.q1 ? (a.cur ? a.q0 : a.q1) : a.q0);
     double cfl = 0.0, hm = 0.0;
-    step_patch<MX, MY, TX, TY, NT, false, DEF, FREG>(T, E, F, red, a.desc + patch, patch, ox, oy, src, dst, a.aux,
-                                                     a.dt, a.P, cfl, hm, threadIdx.x, true);
+    step_patch<MX, MY, TX, TY, NT, false, DEF, FREG>(T, E, F, red, a.desc + patch, patch, ox, oy, src, dst,
+                                                     (const gdouble*)a.aux, a.dt, a.P, cfl, hm, threadIdx.x, true);
     if (threadIdx.x == 0) {
         bool last = true;
         if (TL::NTILES > 1) last = tile_fold(a.tile_cfl, a.tile_h, a.tile_cnt, patch, TL::NTILES, cfl, hm);
@@ -758,18 +785,28 @@ __device__ __forceinline__ void load_head(const BatchArgs& a, int patch, ItemHea
     h->manning = c.manning_n;
 }
 
+// The item after the workgroup's first ones: the next of its queue (items x,
+// x + nq, x + 2 nq, ... of queue x), or `limit` when every item is some
+// workgroup's first.
+__device__ __forceinline__ int next_item(int* counters, int limit)
+{
+    const int grid = (int)gridDim.x, nq = grid % QUEUES == 0 ? QUEUES : 1, x = (int)blockIdx.x % nq;
+    if (grid + x >= limit) return limit;
+    return grid + x + nq * atomicAdd(&counters[CURSOR_LINE * (1 + x)], 1);
+}
+
 // Run by one thread of the current active item: takes the next item from
-// the cursor, publishes it, and when it is active fills its ItemHeads (one
+// the queue, publishes it, and when it is active fills its ItemHeads (one
 // per patch of the item: entries next*NPP .. of the active tile list).
 template <int NTILES, int NPP>
 struct ItemPrefetch {
     const BatchArgs* pa;
     int* next_slot;
     ItemHead* next_head;
-    int nwet;
+    int nwet, limit;
     __device__ void operator()() const
     {
-        const int next = atomicAdd(&pa->counters[NEXT_WET], 1);
+        const int next = next_item(pa->counters, limit);
         *next_slot = next;
 #pragma unroll
         for (int g = 0; g < NPP; g++) {
@@ -793,7 +830,7 @@ struct ItemPrefetch {
 // idx*NPP .. idx*NPP+NPP-1 of the active list, one per group of NT threads.
 template <int MX, int MY, int TX, int TY, int NT, int NPP, bool FREG, bool DEF>
 __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const ItemHead* head, ItemHead* next_head,
-                                         int* next_slot, int nwet)
+                                         int* next_slot, int nwet, int limit)
 {
     using G = Geo<TX, TY>;
     using TL = Tiling<MX, MY, TX, TY>;
@@ -809,22 +846,23 @@ __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const Ite
     const bool valid = NPP == 1 || entry < nwet;
     // a group without a patch computes on a zero tile with group 0's header
     const ItemHead* hd = valid ? head + grp : head;
-    const int patch = hd->patch;
+    // (a group is whole waves, so these are uniform in each wave)
+    const int patch = uniform(hd->patch);
     int ox, oy;
-    TL::origin(entry % TL::NTILES, ox, oy);
-    const int scen = hd->d.scen;
-    const int cur = hd->cur;
-    const double dt = hd->dt;
-    const double* src = cur ? a.q1 : a.q0;
-    double* dst = cur ? a.q0 : a.q1;
-    Params P = a.P;
-    P.manning_n = hd->manning;
+    TL::origin(uniform(entry % TL::NTILES), ox, oy);
+    const int scen = uniform(hd->d.scen);
+    const int cur = uniform(hd->cur);
+    const double dt = uniform(hd->dt);
+    const gdouble* src = (const gdouble*)(cur ? a.q1 : a.q0);
+    gdouble* dst = (gdouble*)(cur ? a.q0 : a.q1);
+    Params P = uniform(a.P);
+    P.manning_n = uniform(hd->manning);
     if (ltid == 0 && valid) a.dry_age[patch] = 0;
     double cfl = 0.0, hm = 0.0;
-    const ItemPrefetch<TL::NTILES, NPP> pf{pa, next_slot, next_head, nwet};
+    const ItemPrefetch<TL::NTILES, NPP> pf{pa, next_slot, next_head, nwet, limit};
     step_patch<MX, MY, TX, TY, NT, true, DEF, FREG>(T + grp * 4 * G::NP2, E + grp * 7 * G::NPOS,
                                                     F + (FREG ? 0 : grp * 6 * G::NF), red + grp * 2 * (NT / 64),
-                                                    &hd->d, patch, ox, oy, src, dst, a.aux, dt, P, cfl, hm, ltid,
+                                                    &hd->d, patch, ox, oy, src, dst, (const gdouble*)a.aux, dt, P, cfl, hm, ltid,
                                                     valid, pf);
     if (ltid == 0 && valid) {
         bool last = true;
@@ -836,7 +874,11 @@ __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const Ite
             // doubles, but -0.0 (which the CFL maximum can return for a patch
             // with no waves) sorts above them all: zeros are left out (the
             // scenario's maximum starts at +0.0).  NaN still propagates.
-            if (cfl != 0.0) atomicMax(a.cflbits + scen, (unsigned long long)__double_as_longlong(cfl));
+            // Most patches do not raise it: a look first leaves the one address
+            // that all of a scenario's patches share mostly unwritten.
+            const unsigned long long bits = (unsigned long long)__double_as_longlong(cfl);
+            if (cfl != 0.0 && bits > __hip_atomic_load(a.cflbits + scen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                atomicMax(a.cflbits + scen, bits);
         }
     }
     __syncthreads();
@@ -874,51 +916,71 @@ __device__ __forceinline__ void dry_item(const BatchArgs* pa, int k, int next, i
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));
     const double tol = a.P.dry_tolerance;
+    const gint* list = (const gint*)a.list_dry;
+    gdouble* q0 = (gdouble*)a.q0;
+    gdouble* q1 = (gdouble*)a.q1;
     // entries (patch | cur << DRY_CUR_SHIFT), then h, then the stores: two
     // dependent memory round trips per item
-    int ent[PER], kk[PER];
+    int ent[PER];
+    double h0[PER];
 #pragma unroll
     for (int r = 0; r < PER; r++) {
         const int e = tid + NT * r;
         const int j = first + e / CELLS;
-        ent[r] = (e < DPI * CELLS && j < count) ? a.list_dry[j] : -1;
-        const int c = e % CELLS;
-        kk[r] = G::ti(c % MX + 1, c / MX + 1);
+        ent[r] = (e < DPI * CELLS && j < count) ? list[j] : -1;
     }
-    double h0[PER];
 #pragma unroll
-    for (int r = 0; r < PER; r++)
-        if (ent[r] >= 0) h0[r] = ((ent[r] >> DRY_CUR_SHIFT) ? a.q1 : a.q0)[(size_t)(ent[r] & PMASK) * 3 * NP2 + kk[r]];
+    for (int r = 0; r < PER; r++) {
+        const int c = (tid + NT * r) % CELLS;
+        const size_t k = (size_t)(ent[r] & PMASK) * 3 * NP2 + G::ti(c % MX + 1, c / MX + 1);
+        if (ent[r] >= 0) h0[r] = ((ent[r] >> DRY_CUR_SHIFT) ? q1 : q0)[k];
+    }
+    unsigned wetter = 0;  // the cells with h >= dry_tolerance, or NaN
 #pragma unroll
     for (int r = 0; r < PER; r++) {
         if (ent[r] < 0) continue;
+        const int c = (tid + NT * r) % CELLS;
         const int pt = ent[r] & PMASK, cur = ent[r] >> DRY_CUR_SHIFT;
-        const double* src = (cur ? a.q1 : a.q0) + (size_t)pt * 3 * NP2;
-        double* dst = (cur ? a.q0 : a.q1) + (size_t)pt * 3 * NP2;
-        double h = h0[r], hu = 0.0, hv = 0.0;
-        if (h < tol) {
-            h = fmaxf64(h, 0.0);
-        } else {
-            atomicOr(&unsteady[(tid + NT * r) / CELLS], 1);
-            const ScenCtrl* c = a.ctrl + a.desc[pt].scen;
-            Params P = a.P;
-            P.manning_n = c->manning_n;
-            hu = src[NP2 + kk[r]];
-            hv = src[2 * NP2 + kk[r]];
-            if (P.src_term > 0) src2_cell<false>(h, hu, hv, a.aux[(size_t)pt * NP2 + kk[r]], c->dt, P);
-            // a NaN depth lands here too: it sets the scenario's CFL maximum
-            // to NaN, which stops the scenario at the controller
-            if (!finite3(h, hu, hv))
-                atomicMax(a.cflbits + a.desc[pt].scen, (unsigned long long)__double_as_longlong(quiet_nan()));
+        if (c == 0) a.hmax[(size_t)(cur ^ 1) * a.capacity + pt] = 0.0;
+        if (!(h0[r] < tol)) {
+            wetter |= 1u << r;
+            continue;
         }
-        dst[kk[r]] = h;
-        dst[NP2 + kk[r]] = hu;
-        dst[2 * NP2 + kk[r]] = hv;
-        if ((tid + NT * r) % CELLS == 0) a.hmax[(size_t)(cur ^ 1) * a.capacity + pt] = 0.0;
+        gdouble* dst = (cur ? q0 : q1) + (size_t)pt * 3 * NP2 + G::ti(c % MX + 1, c / MX + 1);
+        dst[0] = fmaxf64(h0[r], 0.0);
+        dst[NP2] = 0.0;
+        dst[2 * NP2] = 0.0;
+    }
+    // the rare cells at dry_tolerance, one at a time (unrolled with the rest,
+    // their friction term set the registers of the whole kernel, 142 instead of
+    // 120 VGPRs at 16x16: three waves a SIMD instead of four)
+    while (wetter) {
+        const int e = tid + NT * (__ffs(wetter) - 1), c = e % CELLS;
+        wetter &= wetter - 1;
+        const int en = list[first + e / CELLS];
+        const int pt = en & PMASK, cur = en >> DRY_CUR_SHIFT;
+        const size_t k = (size_t)pt * 3 * NP2 + G::ti(c % MX + 1, c / MX + 1);
+        const gdouble* src = (cur ? q1 : q0) + k;
+        gdouble* dst = (cur ? q0 : q1) + k;
+        atomicOr(&unsteady[e / CELLS], 1);
+        const ScenCtrl* sc = a.ctrl + a.desc[pt].scen;
+        Params P = a.P;
+        P.manning_n = sc->manning_n;
+        const double h = src[0];
+        double hu = src[NP2], hv = src[2 * NP2];
+        if (P.src_term > 0)
+            src2_cell<false>(h, hu, hv, a.aux[(size_t)pt * NP2 + G::ti(c % MX + 1, c / MX + 1)], sc->dt, P);
+        // a NaN depth lands here too: it sets the scenario's CFL maximum
+        // to NaN, which stops the scenario at the controller
+        if (!finite3(h, hu, hv))
+            atomicMax(a.cflbits + a.desc[pt].scen, (unsigned long long)__double_as_longlong(quiet_nan()));
+        dst[0] = h;
+        dst[NP2] = hu;
+        dst[2 * NP2] = hv;
     }
     __syncthreads();
     if (threadIdx.x < DPI && first + (int)threadIdx.x < count) {
-        const int e = a.list_dry[first + threadIdx.x];
+        const int e = list[first + threadIdx.x];
         const int pt = e & PMASK, dstbuf = (e >> DRY_CUR_SHIFT) ^ 1;
         const int old = a.dry_age[pt];
         int age = old & 3;
@@ -933,7 +995,7 @@ __device__ __forceinline__ void dry_item(const BatchArgs* pa, int k, int next, i
 
 // Unified persistent step of an attempt: the active patches' tiles first
 // (wet_item), then the dry patches in items of dry_per_item (dry_item), from
-// one atomic cursor.  The streaming dry items fill the tail that the
+// the item queues.  The streaming dry items fill the tail that the
 // compute-bound active items leave when the list runs out.
 // 8x8 patches: the register budget for three waves per SIMD (the kernels
 // need 170 VGPRs, two waves, without it; no spills at 167) is 8% faster at
@@ -949,14 +1011,16 @@ __global__ void __launch_bounds__(NT * NPP, (MX == 8 ? 3 : 1)) k_all(const Batch
     __shared__ int unsteady[DPI];  // per dry patch of an item: a cell at dry_tolerance
     const int nwet = pa->counters[CNT_WET] * TL::NTILES;  // active tiles
     const int witems = (nwet + NPP - 1) / NPP;             // active items
+    const int limit = witems + (pa->counters[CNT_DRY] + DPI - 1) / DPI;
+    if ((int)blockIdx.x >= limit) return;
     if (threadIdx.x == 0) {
-        item[0] = atomicAdd(&pa->counters[NEXT_WET], 1);
+        item[0] = (int)blockIdx.x;
         for (int g = 0; g < NPP; g++)
-            if (item[0] * NPP + g < nwet) load_head(*pa, pa->list_wet[(item[0] * NPP + g) / TL::NTILES], &head[0][g]);
+            if ((int)blockIdx.x * NPP + g < nwet)
+                load_head(*pa, pa->list_wet[((int)blockIdx.x * NPP + g) / TL::NTILES], &head[0][g]);
     }
     if (threadIdx.x < DPI) unsteady[threadIdx.x] = 0;
     __syncthreads();
-    const int limit = witems + (pa->counters[CNT_DRY] + DPI - 1) / DPI;
     for (int it = 0;; it++) {
         const int idx = item[it & 1];
         if (idx >= limit) break;
@@ -964,10 +1028,10 @@ __global__ void __launch_bounds__(NT * NPP, (MX == 8 ? 3 : 1)) k_all(const Batch
             // active items come first in the cursor's order, so an active
             // item's successor's heads are always prefetched by an active item
             wet_item<MX, MY, TX, TY, NT, NPP, FREG, DEF>(pa, idx, head[it & 1], head[(it + 1) & 1],
-                                                         &item[(it + 1) & 1], nwet);
+                                                         &item[(it + 1) & 1], nwet, limit);
         } else {
             int next = 0;
-            if (threadIdx.x == 0) next = atomicAdd(&pa->counters[NEXT_WET], 1);
+            if (threadIdx.x == 0) next = next_item(pa->counters, limit);
             dry_item<MX, MY, NB>(pa, idx - witems, next, &item[(it + 1) & 1], unsteady);
         }
     }
@@ -1296,7 +1360,9 @@ __global__ void __launch_bounds__(64) k_batch_control(const BatchArgs* pa)
         a.stats[1] += a.counters[CNT_DRY] + a.counters[CNT_SKIP];
         a.stats[2] += 1;
         a.stats[3] += a.counters[CNT_SKIP];
-        for (int k = 0; k < NCOUNTERS; k++) a.counters[k] = 0;
+        for (int k = 0; k <= CNT_SKIP; k++) a.counters[k] = 0;
+    } else if (s <= QUEUES) {
+        a.counters[CURSOR_LINE * s] = 0;
     }
     if (s >= a.nscen) return;
     ScenCtrl* c = a.ctrl + s;
