@@ -185,15 +185,14 @@ Lib g;
 
 constexpr size_t kChunk = 1024;  // patches per upload/download chunk
 
-// Resident AMR: refinement levels 0 .. kMaxLevels-1; device ranges
-// [lo, hi) of the stored links (all, then the interpolation links of each
-// coarse level) and of the inflow list's entries per level.
+// Resident AMR: refinement levels 0 .. kMaxLevels-1, and the workgroups of a
+// level's ghost update (one per patch with finer neighbours or a hydrograph
+// side, grid-stride).
 constexpr int kMaxLevels = 16;
-constexpr int kRanges = 2 * (1 + 2 * kMaxLevels);
-inline int range_links() { return 0; }
-inline int range_interp(int l) { return 2 + 2 * l; }
-inline int range_inflow(int l) { return 2 + 2 * kMaxLevels + 2 * l; }
-constexpr int kLinkGrid = 1024;  // workgroups of a resident coarse/fine transfer (one wave per link, grid-stride)
+constexpr int kGhostGrid = 1024;
+constexpr int kLinkBlocks = 256;   // workgroups of the averaging (four links each at a time)
+constexpr int kHydroBlocks = 4;    // and of the hydrograph look-ups (four scenarios each at a time)
+constexpr int kAmrHead = 32;       // ints before the links of gf_pool::d_amr
 
 // Maximum in which a NaN operand wins, as the device reductions fold CFL
 // numbers: a patch whose new state is not finite reports a NaN CFL number.
@@ -272,22 +271,23 @@ struct gf_pool {
     hipGraphExec_t graph_exec = nullptr;
     bool graph_dirty = true;
     // Resident AMR (gf_pool_set_levels, gf_pool_set_cf_links): every attempt
-    // starts with the multi-level ghost update -- fine -> coarse averaging
-    // over all links, then level by level the hydrograph sides and the
-    // coarse -> fine interpolation -- whose link and inflow ranges live in
-    // device memory, so a regrid changes them without a new graph.  The
-    // graph holds only the passes whose ranges are not empty (a forest that
-    // occupies levels 3-4 launches no pass for levels 0-2); it is captured
-    // again when that set changes, which a regrid that keeps the occupied
-    // levels does not.
+    // starts with the multi-level ghost update, one launch per level that has
+    // patches with finer neighbours or a hydrograph side.  The items and links
+    // of the levels and their ranges live in device memory, so a regrid changes
+    // them without a new graph; it is captured again when the set of levels
+    // with a launch changes, which a regrid that keeps the occupied levels does
+    // not.
     bool amr = false;
     std::vector<int> h_level;              // [capacity] refinement level per slot (0 when not set)
-    int nlev = 1;                          // levels the ghost update walks (max level + 1)
-    int* d_links = nullptr;                // [4][link_cap]: coarse, fine, side, igrid by the coarse level
+    std::vector<int> h_links, h_link_level; // the links as given, [n][coarse, fine, side, igrid], and their coarse levels
+    std::vector<int> h_inflow;             // the slots of inflow_list
+    std::vector<int> slot_item;            // [capacity] scratch of rebuild_ghost_items, -1 between calls
+    // one device block: the numbers of items per level and of links, [5][link_cap]
+    // coarse, fine, side, igrid, scenario in item order, then the items by level
+    int* d_amr = nullptr;
     int link_cap = 0, nlinks = 0;
-    unsigned inflow_levels = 0;            // bit l: level l has hydrograph patches (its k_inflow pass runs)
-    unsigned interp_levels = 0;            // bit l: links with a level-l coarse patch (its interpolation runs)
-    int* d_ranges = nullptr;               // [kRanges]: see range_links / range_interp / range_inflow
+    int level_items[kMaxLevels + 1] = {};  // first item of each level in the block (a multiple of 64 apart)
+    unsigned ghost_levels = 0;             // bit l: level l has items
 };
 
 static void default_params()
@@ -480,6 +480,89 @@ static void free_hydrographs(gf_pool* p)
     }
 }
 
+// Rebuild the device items of the resident ghost update from the pool's links
+// and hydrograph patches: one item per patch, level by level, each with its
+// links in one run.
+static int rebuild_ghost_items(gf_pool* p)
+{
+    const int nl = (int)p->h_link_level.size();
+    struct Entry {
+        int patch, level, links, inflow;
+    };
+    std::vector<Entry> e;
+    p->slot_item.resize(p->capacity, -1);
+    std::vector<int> item_of(nl);
+    for (int k = 0; k < nl; k++) {
+        int& i = p->slot_item[p->h_links[4 * k]];
+        if (i < 0) {
+            i = (int)e.size();
+            e.push_back({p->h_links[4 * k], p->h_link_level[k], 0, 0});
+        }
+        e[i].links++;
+        item_of[k] = i;
+    }
+    const size_t linked = e.size();
+    for (int s : p->h_inflow) {
+        const int i = p->slot_item[s];
+        if (i >= 0 && e[i].level == p->h_level[s]) e[i].inflow = 1;
+        else e.push_back({s, p->h_level[s], 0, 1});
+    }
+    for (size_t i = 0; i < linked; i++) p->slot_item[e[i].patch] = -1;
+    // the place of each level's items in the block is part of the captured
+    // graph: it is kept while every level's items fit
+    int count[kMaxLevels] = {};
+    for (const Entry& x : e) count[x.level]++;
+    bool fits = p->d_amr != nullptr && nl <= p->link_cap;
+    for (int l = 0; l < kMaxLevels; l++) fits = fits && count[l] <= p->level_items[l + 1] - p->level_items[l];
+    if (!fits) {
+        const int lc = nl > p->link_cap ? std::max(nl, 2 * p->link_cap) : p->link_cap;
+        int first[kMaxLevels + 1] = {};
+        for (int l = 0; l < kMaxLevels; l++) {
+            const int had = p->level_items[l + 1] - p->level_items[l];
+            first[l + 1] = first[l] + (count[l] > had ? (2 * count[l] + 63) / 64 * 64 : had);
+        }
+        int* d = nullptr;
+        HIPCHK(hipMalloc(&d, sizeof(int) * (kAmrHead + 5 * (size_t)lc) + sizeof(gf::GhostItem) * (size_t)(first[kMaxLevels] + 1)));
+        HIPCHK(hipStreamSynchronize(g.stream));
+        HIPCHK(hipFree(p->d_amr));
+        p->d_amr = d;
+        p->link_cap = lc;
+        std::copy(first, first + kMaxLevels + 1, p->level_items);
+        p->graph_dirty = true;  // the graph holds the block's addresses
+    }
+    std::vector<int> h(kAmrHead + 5 * (size_t)p->link_cap + sizeof(gf::GhostItem) / sizeof(int) * (size_t)p->level_items[kMaxLevels], 0);
+    unsigned levels = 0;
+    int next[kMaxLevels];
+    for (int l = 0; l < kMaxLevels; l++) {
+        h[l] = count[l];
+        if (count[l]) levels |= 1u << l;
+        next[l] = p->level_items[l];
+    }
+    h[kMaxLevels] = nl;
+    int* links = h.data() + kAmrHead;
+    gf::GhostItem* items = reinterpret_cast<gf::GhostItem*>(links + 5 * (size_t)p->link_cap);
+    std::vector<int> cursor(e.size());
+    int off = 0;
+    for (size_t i = 0; i < e.size(); i++) {
+        items[next[e[i].level]++] = {e[i].patch, p->h_desc[e[i].patch].scen, off, off + e[i].links, e[i].inflow};
+        cursor[i] = off;
+        off += e[i].links;
+    }
+    for (int k = 0; k < nl; k++) {
+        const int at = cursor[item_of[k]]++;
+        for (int m = 0; m < 4; m++) links[(size_t)m * p->link_cap + at] = p->h_links[4 * k + m];
+        links[4 * (size_t)p->link_cap + at] = p->h_desc[p->h_links[4 * k]].scen;
+    }
+    if (levels != p->ghost_levels || nl != p->nlinks) {
+        if (levels != p->ghost_levels || (nl > 0) != (p->nlinks > 0)) p->graph_dirty = true;
+        p->ghost_levels = levels;
+        p->nlinks = nl;
+    }
+    HIPCHK(hipMemcpyAsync(p->d_amr, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice, g.stream));
+    HIPCHK(hipStreamSynchronize(g.stream));
+    return GF_OK;
+}
+
 // Rebuild the device list of patches with a hydrograph side, and check that
 // every scenario with such patches has a table and uses one side only.
 static int rebuild_inflow(gf_pool* p)
@@ -509,29 +592,11 @@ static int rebuild_inflow(gf_pool* p)
         p->has_inflow = n > 0;
         p->graph_dirty = true;
     }
-    if (p->amr) {
-        // level by level: the ghost update fills a level's hydrograph sides
-        // before interpolating from it to the next finer level
-        std::stable_sort(list.begin(), list.end(), [&](int a, int b) { return p->h_level[a] < p->h_level[b]; });
-        std::vector<int> rng(2 * kMaxLevels);
-        unsigned levels = 0;
-        for (int l = 0, k = 0; l < kMaxLevels; l++) {
-            rng[2 * l] = k;
-            while (k < n && p->h_level[list[k]] == l) k++;
-            rng[2 * l + 1] = k;
-            if (k > rng[2 * l]) levels |= 1u << l;
-        }
-        if (levels != p->inflow_levels) {
-            p->inflow_levels = levels;
-            p->graph_dirty = true;
-        }
-        HIPCHK(hipMemcpyAsync(p->d_ranges + range_inflow(0), rng.data(), sizeof(int) * rng.size(),
-                              hipMemcpyHostToDevice, g.stream));
-    }
     if (n) HIPCHK(hipMemcpyAsync(p->inflow_list, list.data(), sizeof(int) * n, hipMemcpyHostToDevice, g.stream));
     HIPCHK(hipMemcpyAsync(p->inflow_n, &n, sizeof(int), hipMemcpyHostToDevice, g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
-    return GF_OK;
+    p->h_inflow = std::move(list);
+    return p->amr ? rebuild_ghost_items(p) : GF_OK;
 }
 
 gf_pool* gf_pool_create(int mx, int my, int mbc, int capacity)
@@ -653,8 +718,7 @@ try {
     hipFree(p->tag_buf);
     hipFree(p->inflow_list);
     hipFree(p->inflow_n);
-    hipFree(p->d_links);
-    hipFree(p->d_ranges);
+    hipFree(p->d_amr);
     for (double* m : p->hyd_mem) hipFree(m);
     if (p->h_stage) hipHostFree(p->h_stage);
     if (p->h_cfl) hipHostFree(p->h_cfl);
@@ -1288,47 +1352,46 @@ static int wet_grid(gf_pool* p)
     return p->wet_grid;
 }
 
-// The multi-level ghost update of a resident AMR pool, in ForestClaw's order
-// (fclaw2d_ghost_update with time_interp off, as restated for resident
-// patches): the coarse ghost cells that finer neighbours cover, averaged from
-// them (all links at once: they read fine interiors only); then for each
-// level from coarse to fine its hydrograph sides, and the next finer level's
-// ghost cells interpolated from it.  Same-level copies and walls need no
-// pass: every reader takes them from the neighbours (ghost_source).  buf < 0:
-// each scenario's current buffer and time, inactive scenarios skipped (the
-// form captured in the attempt graph); otherwise buffer buf at time t.
-static int enqueue_ghost_update(gf_pool* p, int buf, double t)
+// The multi-level ghost update of a resident AMR pool, which leaves what
+// ForestClaw's order leaves (fclaw2d_ghost_update with time_interp off): the
+// coarse ghost cells that finer neighbours cover, averaged from them; then for
+// each level from coarse to fine its hydrograph sides, and the next finer
+// level's ghost cells interpolated from it (k_ghost_begin, k_ghost_level).
+// classify: the attempt's classification shares the first launch (buf < 0;
+// p->d_args is up to date).  Same-level copies and
+// walls need no pass: every reader takes them from the neighbours
+// (ghost_source).  buf < 0: each scenario's current buffer and time, inactive
+// scenarios skipped (the form captured in the attempt graph); otherwise buffer
+// buf at time t.
+static int enqueue_ghost_update(gf_pool* p, int buf, double t, bool classify)
 {
-    gf::RegridArgs a{};
+    gf::GhostLevelArgs a{};
+    const int* links = p->d_amr + kAmrHead;
+    const gf::GhostItem* items = reinterpret_cast<const gf::GhostItem*>(links + 5 * (size_t)p->link_cap);
+    a.links.desc = p->desc;
+    a.links.aux = p->aux;
+    a.links.cs = links;
+    a.links.fs = links + p->link_cap;
+    a.links.side = links + 2 * (size_t)p->link_cap;
+    a.links.igrid = links + 3 * (size_t)p->link_cap;
+    a.links.dry_tolerance = g.P.dry_tolerance;
+    a.link_scen = links + 4 * (size_t)p->link_cap;
     a.desc = p->desc;
+    a.ctrl = p->ctrl;
+    a.q0 = p->q[0];
+    a.q1 = p->q[1];
     a.aux = p->aux;
-    a.cs = p->d_links;
-    a.fs = p->d_links + p->link_cap;
-    a.side = p->d_links + 2 * p->link_cap;
-    a.igrid = p->d_links + 3 * p->link_cap;
-    a.n = kLinkGrid;
-    a.dry_tolerance = g.P.dry_tolerance;
-    if (buf < 0) {
-        a.q = p->q[0];
-        a.q1 = p->q[1];
-        a.ctrl = p->ctrl;
-    } else {
-        a.q = p->q[buf];
-    }
-    if (p->nlinks > 0) {
-        a.range = p->d_ranges + range_links();
-        HIPCHK(gf::launch_average_ghost(p->mx, p->my, a, g.stream));
-    }
-    for (int l = 0; l < p->nlev; l++) {
-        if (p->has_inflow && (p->inflow_levels >> l & 1u)) {
-            gf::InflowArgs ia = inflow_args(p, 0, p->capacity, buf, t);
-            ia.range = p->d_ranges + range_inflow(l);
-            HIPCHK(gf::launch_inflow(p->mx, p->my, ia, inflow_grid(), g.stream));
-        }
-        if (l + 1 < p->nlev && p->nlinks > 0 && (p->interp_levels >> l & 1u)) {
-            a.range = p->d_ranges + range_interp(l);
-            HIPCHK(gf::launch_interpolate_ghost(p->mx, p->my, a, g.stream));
-        }
+    a.buf = buf;
+    a.t = t;
+    a.P = g.P;
+    a.count = p->d_amr + kMaxLevels;
+    HIPCHK(gf::launch_ghost_begin(p->mx, p->my, a, buf < 0 ? p->d_args : nullptr, classify ? p->capacity : 0,
+                                  p->nlinks > 0 ? kLinkBlocks : 0, buf < 0 && p->has_inflow ? kHydroBlocks : 0, g.stream));
+    for (int l = 0; l < kMaxLevels; l++) {
+        if (!(p->ghost_levels >> l & 1u)) continue;
+        a.items = items + p->level_items[l];
+        a.count = p->d_amr + l;
+        HIPCHK(gf::launch_ghost_level(p->mx, p->my, a, kGhostGrid, g.stream));
     }
     return GF_OK;
 }
@@ -1341,11 +1404,13 @@ static int enqueue_ghost_update(gf_pool* p, int buf, double t)
 static int enqueue_attempt(gf_pool* p, int k)
 {
     if (p->amr) {
-        if (int r = enqueue_ghost_update(p, -1, 0.0)) return r;
+        if (int r = enqueue_ghost_update(p, -1, 0.0, true)) return r;
     } else if (p->has_inflow) {
-        HIPCHK(gf::launch_inflow(p->mx, p->my, inflow_args(p, 0, p->capacity, -1, 0.0), inflow_grid(), g.stream));
+        HIPCHK(gf::launch_begin(p->mx, p->my, p->d_args, p->capacity, inflow_args(p, 0, p->capacity, -1, 0.0),
+                                inflow_grid(), g.stream));
+    } else {
+        HIPCHK(gf::launch_classify(p->d_args, p->capacity, g.stream));
     }
-    HIPCHK(gf::launch_classify(p->d_args, p->capacity, g.stream));
     if (k >= 0) HIPCHK(hipEventRecord(g.ev_step[2 * k], g.stream));
     HIPCHK(gf::launch_all(p->mx, p->my, p->variant, gf::default_method(g.P), p->d_args, wet_grid(p), g.stream));
     if (k >= 0) HIPCHK(hipEventRecord(g.ev_step[2 * k + 1], g.stream));
@@ -1484,6 +1549,8 @@ try {
     std::vector<ScenCtrl>& hc = p->h_ctrl;
     HIPCHK(hipMemcpyAsync(hc.data(), p->ctrl, sizeof(ScenCtrl) * p->nscen, hipMemcpyDeviceToHost, g.stream));
     if (int r = reset_dry_age(p, 0, p->capacity)) return r;
+    if (p->amr)  // the ghost update reads the scenario count from them
+        if (int r = sync_batch_args(p)) return r;
     HIPCHK(hipStreamSynchronize(g.stream));
     double total_ms = 0.0, step_ms = 0.0;
     int launches = 0;
@@ -1501,7 +1568,7 @@ try {
             // the multi-level ghost update reads each scenario's buffer and
             // time from the device records: bring them up to date first
             HIPCHK(hipMemcpyAsync(p->ctrl, hc.data(), sizeof(ScenCtrl) * p->nscen, hipMemcpyHostToDevice, g.stream));
-            if (int r = enqueue_ghost_update(p, -1, 0.0)) return r;
+            if (int r = enqueue_ghost_update(p, -1, 0.0, false)) return r;
         }
         int e = 0;
         for (int s = 0; s < p->nscen; s++) {
@@ -1881,11 +1948,11 @@ try {
     // Each candidate steps it from the accepted buffer into the other one,
     // which the next attempt overwrites: no scenario advances.
     if (p->amr) {
-        if (int r = enqueue_ghost_update(p, -1, 0.0)) return r;
+        if (int r = enqueue_ghost_update(p, -1, 0.0, true)) return r;
     } else {
         HIPCHK(gf::launch_inflow(p->mx, p->my, inflow_args(p, 0, p->capacity, -1, 0.0), inflow_grid(), g.stream));
+        HIPCHK(gf::launch_classify(p->d_args, p->capacity, g.stream));
     }
-    HIPCHK(gf::launch_classify(p->d_args, p->capacity, g.stream));
     // an inactive scenario (stopped at its target, or between regrids) lists
     // nothing: with every list empty there is no work to time
     int cnt[2] = {0, 0};
@@ -2243,16 +2310,10 @@ try {
 
 static int ensure_amr(gf_pool* p)
 {
-    if (!p->d_ranges) {
-        HIPCHK(hipMalloc(&p->d_ranges, sizeof(int) * kRanges));
-        HIPCHK(hipMemsetAsync(p->d_ranges, 0, sizeof(int) * kRanges, g.stream));
-        HIPCHK(hipStreamSynchronize(g.stream));
-    }
-    if (!p->amr) {
-        p->amr = true;
-        p->graph_dirty = true;
-    }
-    return GF_OK;
+    if (p->amr) return GF_OK;
+    p->amr = true;
+    p->graph_dirty = true;
+    return rebuild_ghost_items(p);
 }
 
 int gf_pool_set_levels(gf_pool* p, int first, int n, const int* level)
@@ -2268,11 +2329,6 @@ try {
     for (int k = 0; k < n; k++) {
         in_scenario |= p->h_desc[first + k].scen >= 0;
         p->h_level[first + k] = level[k];
-    }
-    const int nlev = 1 + *std::max_element(p->h_level.begin(), p->h_level.end());
-    if (nlev != p->nlev) {
-        p->nlev = nlev;
-        p->graph_dirty = true;
     }
     // the hydrograph list holds the slots of scenarios, by level: levels of
     // slots outside every scenario (a regrid's next half) leave it as it is,
@@ -2299,49 +2355,17 @@ try {
         }
     }
     if (int r = ensure_amr(p)) return r;
-    if (n > p->link_cap) {
-        const int cap = std::max(n, 2 * p->link_cap);
-        int* d = nullptr;
-        HIPCHK(hipMalloc(&d, sizeof(int) * 4 * (size_t)cap));
-        HIPCHK(hipStreamSynchronize(g.stream));
-        HIPCHK(hipFree(p->d_links));
-        p->d_links = d;
-        p->graph_dirty = true;  // the graph holds the link arrays' addresses (or had no transfers)
-        p->link_cap = cap;
+    p->h_links.resize(4 * (size_t)n);
+    p->h_link_level.resize(n);
+    for (int l = 0; l < n; l++) {
+        int* k = p->h_links.data() + 4 * (size_t)l;
+        k[0] = coarse[l];
+        k[1] = fine[l];
+        k[2] = side[l];
+        k[3] = side[l] >= 4 ? 0 : igrid[l];
+        p->h_link_level[l] = p->h_level[coarse[l]];
     }
-    // links by the coarse patch's level (stable), so each level's
-    // interpolation links form one range
-    std::vector<int> order(n);
-    for (int l = 0; l < n; l++) order[l] = l;
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return p->h_level[coarse[a]] < p->h_level[coarse[b]]; });
-    std::vector<int> h(4 * (size_t)std::max(p->link_cap, 1), 0);
-    for (int k = 0; k < n; k++) {
-        const int l = order[k];
-        h[k] = coarse[l];
-        h[p->link_cap + k] = fine[l];
-        h[2 * p->link_cap + k] = side[l];
-        h[3 * p->link_cap + k] = side[l] >= 4 ? 0 : igrid[l];
-    }
-    std::vector<int> rng(2 * (1 + kMaxLevels), 0);
-    rng[0] = 0;
-    rng[1] = n;
-    unsigned levels = 0;
-    for (int lv = 0, k = 0; lv < kMaxLevels; lv++) {
-        rng[range_interp(lv)] = k;
-        while (k < n && p->h_level[h[k]] == lv) k++;
-        rng[range_interp(lv) + 1] = k;
-        if (k > rng[range_interp(lv)]) levels |= 1u << lv;
-    }
-    if (levels != p->interp_levels || (n > 0) != (p->nlinks > 0)) {
-        p->interp_levels = levels;
-        p->graph_dirty = true;
-    }
-    if (p->link_cap > 0)
-        HIPCHK(hipMemcpyAsync(p->d_links, h.data(), sizeof(int) * 4 * (size_t)p->link_cap, hipMemcpyHostToDevice, g.stream));
-    HIPCHK(hipMemcpyAsync(p->d_ranges, rng.data(), sizeof(int) * rng.size(), hipMemcpyHostToDevice, g.stream));
-    HIPCHK(hipStreamSynchronize(g.stream));
-    p->nlinks = n;
-    return GF_OK;
+    return rebuild_ghost_items(p);
 } GF_CATCH_STATUS
 
 int gf_pool_ghost_update(gf_pool* p, int buf, double t)
@@ -2351,7 +2375,9 @@ try {
     if (!p->inflow_error.empty()) return fail(GF_EINVAL, "%s", p->inflow_error.c_str());
     if (int r = ensure_amr(p)) return r;
     // stream-ordered: every call that reads the pool afterwards waits for it
-    return enqueue_ghost_update(p, buf, t);
+    if (buf < 0)
+        if (int r = sync_batch_args(p)) return r;
+    return enqueue_ghost_update(p, buf, t, false);
 } GF_CATCH_STATUS
 
 int gf_pool_move(gf_pool* p, int n, const int* src, const int* dst, int buf)

@@ -46,6 +46,7 @@ struct ScenCtrl {
     const double* hyd;   // hydrograph table: hyd[0..rows) times, hyd[rows..2 rows) discharge per unit width
     double hyd_b, hyd_x0, hyd_y0;  // channel width and centre of the inflow strip
     double dt_max;       // upper bound of the next dt (<= 0: none)
+    double hyd_hu;       // the hydrograph's discharge at t, written at the start of a resident forest's attempt
     int hyd_rows;        // 0: no hydrograph
     int status;          // SCEN_OK, or why the scenario stopped (SCEN_NONFINITE)
     int cur;             // index of the q buffer holding the accepted state

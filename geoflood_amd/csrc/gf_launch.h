@@ -52,12 +52,6 @@ struct GaugeArgs {
 // Regrid between levels on resident patches (refinement ratio 2): family f
 // has the coarse patch in slot cs[f] and its children in slots fs[4f + g],
 // g = igrid = 0..3 (x fastest), all in buffer q.
-//
-// Coarse/fine ghost transfers also run in a resident mode (ctrl != nullptr),
-// as nodes of the attempt graph: link l's buffer is the current one of the
-// coarse patch's scenario (q, or q1 when its ``cur`` is 1; links of inactive
-// scenarios are skipped), and the links are [range[0], range[1]) of the
-// arrays, read from device memory, taken grid-stride by n workgroups.
 struct RegridArgs {
     const PatchDesc* desc;
     double* q;
@@ -68,9 +62,6 @@ struct RegridArgs {
     const int* igrid;  // and the fine neighbour's half along a face
     int n;
     double dry_tolerance;
-    double* q1;             // resident mode: the other q buffer
-    const ScenCtrl* ctrl;   // resident mode: per-scenario current buffer
-    const int* range;       // nullable: links [range[0], range[1]) instead of [0, n)
 };
 
 // Time interpolation of the two interior border layers: slot dst[k] of qdst
@@ -102,7 +93,32 @@ struct InflowArgs {
     int buf;
     double t;
     Params P;
-    const int* range;  // nullable: entries [range[0], range[1]) of list (one level) instead of [0, *list_n)
+};
+
+// One patch of a level of a resident forest's ghost update: its scenario, its
+// links to finer patches [first, end) and whether it has a hydrograph side.
+struct GhostItem {
+    int patch, scen, first, end, inflow;
+};
+
+// A resident forest's ghost update (k_ghost_begin, k_ghost_level).  The links,
+// a level's items and their numbers are read from device memory, so that a
+// regrid needs no new graph, and taken grid-stride.  buf < 0: each patch's
+// scenario's current buffer and time, inactive scenarios skipped; otherwise
+// buffer buf at time t.
+struct GhostLevelArgs {
+    RegridArgs links;      // desc, aux and the link arrays; q is set per patch
+    const int* link_scen;  // the coarse patch's scenario, per link
+    const PatchDesc* desc;
+    ScenCtrl* ctrl;
+    double* q0;
+    double* q1;
+    double* aux;
+    const GhostItem* items;
+    const int* count;      // links (k_ghost_begin) or items (k_ghost_level)
+    int buf;
+    double t;
+    Params P;
 };
 
 // Dry-list entries carry the patch's current buffer: patch | cur << 30.
@@ -209,6 +225,11 @@ hipError_t launch_interpolate2fine(int mx, int my, const RegridArgs& a, hipStrea
 hipError_t launch_copy_slots(const double* src, double* dst, const int* slots, int n, int np2, hipStream_t st);
 hipError_t launch_average_ghost(int mx, int my, const RegridArgs& a, hipStream_t st);
 hipError_t launch_interpolate_ghost(int mx, int my, const RegridArgs& a, hipStream_t st);
+hipError_t launch_ghost_level(int mx, int my, const GhostLevelArgs& a, int grid, hipStream_t st);
+hipError_t launch_ghost_begin(int mx, int my, const GhostLevelArgs& a, const BatchArgs* da, int slots, int link_blocks,
+                              int hydro_blocks, hipStream_t st);
+hipError_t launch_begin(int mx, int my, const BatchArgs* da, int slots, const InflowArgs& in, int inflow_blocks,
+                        hipStream_t st);
 hipError_t launch_timeinterp(int mx, int my, const TimeInterpArgs& a, hipStream_t st);
 // hmax[slot] of buffer q for the listed slots; clears their dry_age entries.
 hipError_t launch_hmax_list(int mx, int my, const double* q, double* hmax, int* dry_age, const int* slots, int n,

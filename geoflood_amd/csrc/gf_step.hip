@@ -1093,7 +1093,7 @@ __global__ void __launch_bounds__(256) k_ghost(GhostArgs a)
 // rows/columns and, for the y sides, the ghost columns the x sides wrote;
 // writes only this side's ghost cells.
 template <int MX, int MY>
-__device__ void bc2_side(double* L, int side, int code, const PatchDesc* __restrict__ dp,
+__device__ void bc2_side(double* L, int side, int code, const PatchDesc* dp,
                          const ScenCtrl* __restrict__ c, double hu0, const Params& P)
 {
     using G = Geo<MX, MY>;
@@ -1154,89 +1154,154 @@ __device__ void bc2_side(double* L, int side, int code, const PatchDesc* __restr
     }
 }
 
+// The cells that the side passes read (the ghost ring and the MBC interior
+// rows and columns next to it: mirror and boundary cells), numbered 0 ..
+// RingCells - 1: the lowest and highest 2 MBC rows, then 2 MBC cells at each
+// end of the rows between.
 template <int MX, int MY>
-__global__ void __launch_bounds__(256) k_inflow(InflowArgs a)
+struct Ring {
+    using G = Geo<MX, MY>;
+    static constexpr int W = 2 * MBC, ROWS = 2 * W * G::NXP, CELLS = ROWS + (G::NYP - 2 * W) * 2 * W;
+    __device__ static void cell(int r, int& fi, int& fj)
+    {
+        int i, j;
+        if (r < ROWS) {
+            i = r % G::NXP;
+            j = r / G::NXP;
+            if (j >= W) j += G::NYP - 2 * W;
+        } else {
+            i = (r - ROWS) % (2 * W);
+            j = W + (r - ROWS) / (2 * W);
+            if (i >= W) i += G::NXP - 2 * W;
+        }
+        fi = i - 1;
+        fj = j - 1;
+    }
+};
+
+// Ghost ring of one hydrograph patch (base: the q buffer) by a workgroup of
+// 256 threads.  It is a chain of dependent steps rather than work (a few
+// hundred cells): the last wave looks the discharge up (or takes it from
+// known_hu, looked up before) while the other three load the ring, every load
+// of a thread is in flight before the first is used, and sides that bc2 leaves
+// alone cost no barrier.
+template <int MX, int MY>
+__device__ void inflow_patch(double* L, double* hu_sh, double* base, double* aux, const PatchDesc* dp,
+                             const ScenCtrl* __restrict__ c, int patch, double t, const Params& P,
+                             const double* known_hu = nullptr)
 {
     using G = Geo<MX, MY>;
+    using R = Ring<MX, MY>;
     constexpr int NXP = G::NXP, NP2 = G::NP2;
-    __shared__ double L[4 * NP2];
-    const int lo = a.range ? a.range[0] : 0, n = a.range ? a.range[1] : *a.list_n;
-    for (int k = lo + (int)blockIdx.x; k < n; k += gridDim.x) {
+    constexpr int NL = 192, PER = (R::CELLS + NL - 1) / NL;
+    double* q = base + (size_t)patch * 3 * NP2;
+    double* ax = aux + (size_t)patch * NP2;
+    if (threadIdx.x >= NL && known_hu) {
+        if (threadIdx.x == NL) *hu_sh = *known_hu;
+    } else if (threadIdx.x >= NL) {
+        // the discharge per unit width at time t, when a ghost cell of the
+        // hydrograph side lies in the channel (bc2_side's own test)
+        const int lane = (int)threadIdx.x - NL;
+        bool in = false;
+        for (int side = 0; side < 4; side++) {
+            if (dp->nbr[side] != NB_INFLOW) continue;
+            const bool xs = side < 2;
+            const double lo = xs ? dp->ylo : dp->xlo;
+            const double del = xs ? dp->dy : dp->dx;
+            const double c0 = xs ? c->hyd_y0 : c->hyd_x0;
+            for (int r = lane + 1 - MBC; r <= (xs ? MY : MX) + MBC; r += 64)
+                in |= fabs(lo + ((double)r - 0.5) * del - c0) <= c->hyd_b / 2.0;
+        }
+        const double hu0 = __ballot(in) ? hydro_interpolate(c->hyd, c->hyd + c->hyd_rows, c->hyd_rows, t) : 0.0;
+        if (lane == 0) *hu_sh = hu0;
+    } else {
+        double v[PER][4];
+        bool nu[PER], nv[PER];
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            const int e = (int)threadIdx.x + r * NL;
+            nu[r] = nv[r] = false;
+            if (e >= R::CELLS) continue;
+            int fi, fj;
+            R::cell(e, fi, fj);
+            const int own = G::ti(fi, fj);
+            const double* src = q;
+            int kk = own;
+            if (!(fi >= 1 && fi <= MX && fj >= 1 && fj <= MY)) {
+                int sp, si, sj;
+                if (ghost_source<MX, MY>(dp->nbr, patch, fi, fj, sp, si, sj, nu[r], nv[r])) {
+                    src = base + (size_t)sp * 3 * NP2;
+                    kk = G::ti(si, sj);
+                }
+            }
+            v[r][0] = src[kk];
+            v[r][1] = src[NP2 + kk];
+            v[r][2] = src[2 * NP2 + kk];
+            v[r][3] = ax[own];
+        }
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            const int e = (int)threadIdx.x + r * NL;
+            if (e >= R::CELLS) continue;
+            int fi, fj;
+            R::cell(e, fi, fj);
+            const int own = G::ti(fi, fj);
+            L[own] = v[r][0];
+            L[NP2 + own] = nu[r] ? -v[r][1] : v[r][1];
+            L[2 * NP2 + own] = nv[r] ? -v[r][2] : v[r][2];
+            L[3 * NP2 + own] = v[r][3];
+        }
+    }
+    __syncthreads();
+    const double hu0 = *hu_sh;
+    for (int side = 0; side < 4; side++) {
+        const int code = dp->nbr[side];
+        if (code != NB_WALL && code != NB_EXTRAP && code != NB_INFLOW) continue;
+        bc2_side<MX, MY>(L, side, code, dp, c, hu0, P);
+        __syncthreads();
+    }
+    for (int e = threadIdx.x; e < R::CELLS; e += blockDim.x) {
+        int fi, fj;
+        R::cell(e, fi, fj);
+        if (fi >= 1 && fi <= MX && fj >= 1 && fj <= MY) continue;
+        const int k = G::ti(fi, fj);
+        q[k] = L[k];
+        q[NP2 + k] = L[NP2 + k];
+        q[2 * NP2 + k] = L[2 * NP2 + k];
+        ax[k] = L[3 * NP2 + k];
+    }
+}
+
+// The listed hydrograph patches, by workgroup `first` and every `stride`-th.
+template <int MX, int MY>
+__device__ __forceinline__ void inflow_list(const InflowArgs& a, int first, int stride)
+{
+    __shared__ double L[4 * Geo<MX, MY>::NP2];
+    __shared__ double hu_sh;
+    const int n = *a.list_n;
+    for (int k = first; k < n; k += stride) {
         const int patch = a.list[k];
         if (patch < a.first || patch >= a.last) continue;
         const PatchDesc* dp = a.desc + patch;
         const int scen = dp->scen;
         if (scen < 0) continue;
         const ScenCtrl* c = a.ctrl + scen;
-        int cur;
-        double t;
+        int cur = a.buf;
+        double t = a.t;
         if (a.buf < 0) {
             if (!c->active) continue;
             cur = c->cur;
             t = c->t;
-        } else {
-            cur = a.buf;
-            t = a.t;
         }
-        double* base = cur ? a.q1 : a.q0;
-        double* q = base + (size_t)patch * 3 * NP2;
-        double* ax = a.aux + (size_t)patch * NP2;
         __syncthreads();  // the previous patch's write-back has read L
-        // bc2's side passes read the ghost ring and the MBC interior rows and
-        // columns next to it (mirror and boundary cells): the deeper interior
-        // is never read, and not loaded
-        for (int e = threadIdx.x; e < NP2; e += blockDim.x) {
-            const int fi = e % NXP - 1, fj = e / NXP - 1;
-            if (fi > MBC && fi <= MX - MBC && fj > MBC && fj <= MY - MBC) continue;
-            const double* src = q;
-            int kk = e;
-            bool nu = false, nv = false;
-            if (!(fi >= 1 && fi <= MX && fj >= 1 && fj <= MY)) {
-                int sp, si, sj;
-                if (ghost_source<MX, MY>(dp->nbr, patch, fi, fj, sp, si, sj, nu, nv)) {
-                    src = base + (size_t)sp * 3 * NP2;
-                    kk = G::ti(si, sj);
-                }
-            }
-            const double h = src[kk], hu = src[NP2 + kk], hv = src[2 * NP2 + kk];
-            L[e] = h;
-            L[NP2 + e] = nu ? -hu : hu;
-            L[2 * NP2 + e] = nv ? -hv : hv;
-            L[3 * NP2 + e] = ax[e];
-        }
-        __syncthreads();
-        // the discharge per unit width at time t, once for the patch, when a
-        // ghost cell of its hydrograph side lies in the channel (bc2_side's
-        // own test; every wave takes the same branch and value)
-        int in_channel = 0;
-        for (int side = 0; side < 4; side++) {
-            if (dp->nbr[side] != NB_INFLOW) continue;
-            const bool xs = side < 2;
-            const int r = (int)threadIdx.x + 1 - MBC;  // one row (x sides) or column (y sides) per thread
-            if (r <= (xs ? MY : MX) + MBC) {
-                const double lo = xs ? dp->ylo : dp->xlo;
-                const double del = xs ? dp->dy : dp->dx;
-                const double c0 = xs ? c->hyd_y0 : c->hyd_x0;
-                in_channel |= fabs(lo + ((double)r - 0.5) * del - c0) <= c->hyd_b / 2.0;
-            }
-        }
-        const double hu0 = __syncthreads_or(in_channel)
-                               ? hydro_interpolate(c->hyd, c->hyd + c->hyd_rows, c->hyd_rows, t)
-                               : 0.0;
-        for (int side = 0; side < 4; side++) {
-            const int code = dp->nbr[side];
-            if (code == NB_WALL || code == NB_EXTRAP || code == NB_INFLOW) bc2_side<MX, MY>(L, side, code, dp, c, hu0, a.P);
-            __syncthreads();
-        }
-        for (int e = threadIdx.x; e < NP2; e += blockDim.x) {
-            const int fi = e % NXP - 1, fj = e / NXP - 1;
-            if (fi >= 1 && fi <= MX && fj >= 1 && fj <= MY) continue;
-            q[e] = L[e];
-            q[NP2 + e] = L[NP2 + e];
-            q[2 * NP2 + e] = L[2 * NP2 + e];
-            ax[e] = L[3 * NP2 + e];
-        }
+        inflow_patch<MX, MY>(L, &hu_sh, cur ? a.q1 : a.q0, a.aux, dp, c, patch, t, a.P);
     }
+}
+
+template <int MX, int MY>
+__global__ void __launch_bounds__(256) k_inflow(InflowArgs a)
+{
+    inflow_list<MX, MY>(a, blockIdx.x, gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1300,10 +1365,10 @@ __global__ void __launch_bounds__(256) k_control(ScenCtrl* ctrl, int nscen, cons
 // or a neighbour's maximum interior depth exceeds the tolerance, or a side's
 // ghost cells come from the host.  Active patches go to the wet list (full
 // step), the others to the dry list.  Appends are aggregated per wavefront.
-__global__ void __launch_bounds__(256) k_classify(const BatchArgs* pa)
+// Block b of 256 threads takes slots 256 b to 256 b + 255.
+__device__ __forceinline__ void classify(const BatchArgs& a, int block)
 {
-    const BatchArgs& a = *pa;
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int p = block * 256 + (int)threadIdx.x;
     int kind = -1;  // -1: not stepping, 0: dry, 1: active
     int cur = 0;
     if (p < a.n) {
@@ -1346,6 +1411,17 @@ __global__ void __launch_bounds__(256) k_classify(const BatchArgs* pa)
     const unsigned long long below = lane ? (~0ull >> (64 - lane)) : 0ull;
     if (kind == 1) a.list_wet[bw + __popcll(mw & below)] = p;
     if (kind == 0) a.list_dry[bd + __popcll(md & below)] = p | (cur << DRY_CUR_SHIFT);
+}
+
+__global__ void __launch_bounds__(256) k_classify(const BatchArgs* pa) { classify(*pa, blockIdx.x); }
+
+// The first launch of an attempt of a pool with hydrograph sides: the patches'
+// inflow ghosts and the classification, which do not depend on each other.
+template <int MX, int MY>
+__global__ void __launch_bounds__(256) k_begin(const BatchArgs* pa, InflowArgs in, int inflow_blocks)
+{
+    if ((int)blockIdx.x < inflow_blocks) inflow_list<MX, MY>(in, blockIdx.x, inflow_blocks);
+    else classify(*pa, (int)blockIdx.x - inflow_blocks);
 }
 
 // Controller of the batched path: the per-scenario CFL maximum was folded by
@@ -1581,13 +1657,13 @@ __device__ __forceinline__ double amr_slope(double sl, double sr)
 }
 
 template <int MX, int MY>
-__device__ __forceinline__ double regrid_cell(const RegridArgs& a, int patch, int fi, int fj, int m)
+__device__ __forceinline__ double regrid_cell(const RegridArgs& a, const int* nbr, int patch, int fi, int fj, int m)
 {
     using G = Geo<MX, MY>;
     int sp = patch, si = fi, sj = fj;
     bool nu = false, nv = false;
     const bool interior = fi >= 1 && fi <= MX && fj >= 1 && fj <= MY;
-    if (!interior && !ghost_source<MX, MY>(a.desc[patch].nbr, patch, fi, fj, sp, si, sj, nu, nv)) {
+    if (!interior && !ghost_source<MX, MY>(nbr, patch, fi, fj, sp, si, sj, nu, nv)) {
         sp = patch; si = fi; sj = fj;
     }
     const double v = a.q[(size_t)sp * 3 * G::NP2 + m * G::NP2 + G::ti(si, sj)];
@@ -1599,8 +1675,8 @@ __device__ __forceinline__ double regrid_cell(const RegridArgs& a, int patch, in
 // :117-171, interpolate_corner :351-396), sea_level = 0: qc, slopes gx, gy of
 // eta (dry-limited 3x3 stencil) and of hu, hv.
 template <int MX, int MY>
-__device__ __forceinline__ void reconstruct_coarse(const RegridArgs& a, int cp, const double* __restrict__ ac,
-                                                   int ic, int jc, double qc[3], double gx[3], double gy[3])
+__device__ __forceinline__ void reconstruct_coarse(const RegridArgs& a, const int* nbr, int cp,
+                                                   const double* __restrict__ ac, int ic, int jc, double qc[3], double gx[3], double gy[3])
 {
     using G = Geo<MX, MY>;
     double eb[3][3];
@@ -1608,7 +1684,7 @@ __device__ __forceinline__ void reconstruct_coarse(const RegridArgs& a, int cp, 
     for (int ii = -1; ii <= 1; ii++)
 #pragma unroll
         for (int jj = -1; jj <= 1; jj++) {
-            const double h = regrid_cell<MX, MY>(a, cp, ic + ii, jc + jj, 0);
+            const double h = regrid_cell<MX, MY>(a, nbr, cp, ic + ii, jc + jj, 0);
             const double b = ac[G::ti(ic + ii, jc + jj)];
             eb[ii + 1][jj + 1] = h < a.dry_tolerance ? 0.0 : h + b;
         }
@@ -1617,11 +1693,11 @@ __device__ __forceinline__ void reconstruct_coarse(const RegridArgs& a, int cp, 
     gy[0] = amr_slope(qc[0] - eb[1][0], eb[1][2] - qc[0]);
 #pragma unroll
     for (int mq = 1; mq < 3; mq++) {
-        qc[mq] = regrid_cell<MX, MY>(a, cp, ic, jc, mq);
-        gx[mq] = amr_slope(qc[mq] - regrid_cell<MX, MY>(a, cp, ic - 1, jc, mq),
-                           regrid_cell<MX, MY>(a, cp, ic + 1, jc, mq) - qc[mq]);
-        gy[mq] = amr_slope(qc[mq] - regrid_cell<MX, MY>(a, cp, ic, jc - 1, mq),
-                           regrid_cell<MX, MY>(a, cp, ic, jc + 1, mq) - qc[mq]);
+        qc[mq] = regrid_cell<MX, MY>(a, nbr, cp, ic, jc, mq);
+        gx[mq] = amr_slope(qc[mq] - regrid_cell<MX, MY>(a, nbr, cp, ic - 1, jc, mq),
+                           regrid_cell<MX, MY>(a, nbr, cp, ic + 1, jc, mq) - qc[mq]);
+        gy[mq] = amr_slope(qc[mq] - regrid_cell<MX, MY>(a, nbr, cp, ic, jc - 1, mq),
+                           regrid_cell<MX, MY>(a, nbr, cp, ic, jc + 1, mq) - qc[mq]);
     }
 }
 
@@ -1644,7 +1720,7 @@ __global__ void __launch_bounds__(256) k_interpolate2fine(RegridArgs a)
         const int i = (1 - ig) + c % NI, j = (1 - jg) + c / NI;
         const int ic = i + ig * MX / 2, jc = j + jg * MY / 2;
         double qc[3], gx[3], gy[3];
-        reconstruct_coarse<MX, MY>(a, cp, ac, ic, jc, qc, gx, gy);
+        reconstruct_coarse<MX, MY>(a, a.desc[cp].nbr, cp, ac, ic, jc, qc, gx, gy);
 #pragma unroll
         for (int mq = 0; mq < 3; mq++)
 #pragma unroll
@@ -1678,37 +1754,11 @@ __device__ __forceinline__ void half_origin(int side, int igrid, int& ox, int& o
 
 // fc2d_geoclaw_fort_average_face / _average_corner (fc2d_geoclaw_average_fort.f:
 // 33-480), mcapa = 0: the coarse ghost cells the fine neighbour covers.
-// The buffer of link l: a.q, or in the resident mode the current buffer of
-// the coarse patch's scenario (nullptr: an inactive scenario, skipped).
-__device__ __forceinline__ double* link_buffer(const RegridArgs& a, int l)
-{
-    if (!a.ctrl) return a.q;
-    const int sc = a.desc[a.cs[l]].scen;
-    if (sc < 0) return nullptr;
-    const ScenCtrl& c = a.ctrl[sc];
-    if (!c.active) return nullptr;
-    return c.cur ? a.q1 : a.q;
-}
-
 template <int MX, int MY>
-__device__ __forceinline__ void average_link(const RegridArgs& a, int l, double* q);
-template <int MX, int MY>
-__device__ __forceinline__ void interpolate_link(const RegridArgs& a, int l);
-
-template <int MX, int MY>
-__global__ void __launch_bounds__(64) k_average_ghost(RegridArgs a)
-{
-    const int lo = a.range ? a.range[0] : 0, hi = a.range ? a.range[1] : a.n;
-    for (int l = lo + (int)blockIdx.x; l < hi; l += gridDim.x) {
-        double* q = link_buffer(a, l);
-        if (q) average_link<MX, MY>(a, l, q);
-    }
-}
-
-template <int MX, int MY>
-__device__ __forceinline__ void average_link(const RegridArgs& a, int l, double* q)
+__device__ __forceinline__ void average_link(const RegridArgs& a, int l, int lane)
 {
     using G = Geo<MX, MY>;
+    double* q = a.q;
     const int side = a.side[l], igrid = a.igrid[l];
     int ox, oy;
     half_origin<MX, MY>(side, igrid, ox, oy);
@@ -1717,7 +1767,7 @@ __device__ __forceinline__ void average_link(const RegridArgs& a, int l, double*
     double* qc = q + (size_t)a.cs[l] * 3 * G::NP2;
     const double* ac = a.aux + (size_t)a.cs[l] * G::NP2;
     const int ncell = side >= 4 ? MBC * MBC : MBC * (side < 2 ? MY : MX);
-    for (int c = threadIdx.x; c < ncell; c += 64) {
+    for (int c = lane; c < ncell; c += 64) {
         int ic, jc;
         if (side >= 4) {
             const int ibc = c / MBC + 1, jbc = c % MBC + 1;
@@ -1755,20 +1805,7 @@ __device__ __forceinline__ void average_link(const RegridArgs& a, int l, double*
 // at 0.  Coarse cells outside the coarse interior are read through
 // ghost_source, as the halo pull reads them.
 template <int MX, int MY>
-__global__ void __launch_bounds__(64) k_interpolate_ghost(RegridArgs a)
-{
-    const int lo = a.range ? a.range[0] : 0, hi = a.range ? a.range[1] : a.n;
-    for (int l = lo + (int)blockIdx.x; l < hi; l += gridDim.x) {
-        double* q = link_buffer(a, l);
-        if (!q) continue;
-        RegridArgs b = a;  // the per-cell helpers read the state through b.q
-        b.q = q;
-        interpolate_link<MX, MY>(b, l);
-    }
-}
-
-template <int MX, int MY>
-__device__ __forceinline__ void interpolate_link(const RegridArgs& a, int l)
+__device__ __forceinline__ void interpolate_link(const RegridArgs& a, int l, int lane, const int* nbr)
 {
     using G = Geo<MX, MY>;
     const int side = a.side[l], igrid = a.igrid[l];
@@ -1779,7 +1816,7 @@ __device__ __forceinline__ void interpolate_link(const RegridArgs& a, int l)
     double* qf = a.q + (size_t)a.fs[l] * 3 * G::NP2;
     const double* af = a.aux + (size_t)a.fs[l] * G::NP2;
     const int ncell = side >= 4 ? 1 : MX;
-    for (int c = threadIdx.x; c < ncell; c += 64) {
+    for (int c = lane; c < ncell; c += 64) {
         int ic, jc;
         if (side >= 4) {
             ic = (side - 4) & 1 ? MX : 1;
@@ -1795,7 +1832,7 @@ __device__ __forceinline__ void interpolate_link(const RegridArgs& a, int l)
         // fclaw2d_clawpatch_is_valid_interp: the four cells inside the fine array
         if (side < 4 && !(i0 >= 1 - MBC && i0 + 1 <= MX + MBC && j0 >= 1 - MBC && j0 + 1 <= MY + MBC)) continue;
         double qc[3], gx[3], gy[3];
-        reconstruct_coarse<MX, MY>(a, cp, ac, ic, jc, qc, gx, gy);
+        reconstruct_coarse<MX, MY>(a, nbr, cp, ac, ic, jc, qc, gx, gy);
 #pragma unroll
         for (int mq = 0; mq < 3; mq++)
 #pragma unroll
@@ -1811,6 +1848,91 @@ __device__ __forceinline__ void interpolate_link(const RegridArgs& a, int l)
                     qf[mq * G::NP2 + k] = v;
                 }
             }
+    }
+}
+
+template <int MX, int MY>
+__global__ void __launch_bounds__(64) k_average_ghost(RegridArgs a)
+{
+    if ((int)blockIdx.x < a.n) average_link<MX, MY>(a, blockIdx.x, threadIdx.x);
+}
+
+template <int MX, int MY>
+__global__ void __launch_bounds__(64) k_interpolate_ghost(RegridArgs a)
+{
+    if ((int)blockIdx.x < a.n) interpolate_link<MX, MY>(a, blockIdx.x, threadIdx.x, a.desc[a.cs[blockIdx.x]].nbr);
+}
+
+// The multi-level ghost update of a resident forest.  What bounds it is the
+// chain of dependent loads (600-800 ns each after a launch boundary), not its
+// few hundred patches, so independent parts share a launch:
+//  * k_ghost_begin: the coarse ghost cells under finer neighbours, averaged
+//    from their interiors, of every level; the discharge of every scenario's
+//    hydrograph at its time; and the attempt's classification.
+//  * k_ghost_level, once per level: one workgroup per patch that has finer
+//    neighbours or a hydrograph side fills its hydrograph sides, then the ghost
+//    cells of those neighbours.  All that these read of ghost cells is the
+//    patch's own, so only the levels follow each other (a patch's ghost cells
+//    towards a coarser one are written by the coarser level's launch).
+// On four levels of 16x16 patches (0.9k leaves) the five launches take 50 us;
+// averaging, hydrographs, interpolation and classification as nine launches of
+// their own took 63 us and three more launch gaps.
+__device__ __forceinline__ double* link_buffer(const GhostLevelArgs& a, int scen)
+{
+    if (a.buf >= 0) return a.buf ? a.q1 : a.q0;
+    if (scen < 0) return nullptr;
+    const ScenCtrl* c = a.ctrl + scen;
+    return !c->active ? nullptr : c->cur ? a.q1 : a.q0;
+}
+
+template <int MX, int MY>
+__global__ void __launch_bounds__(256) k_ghost_begin(GhostLevelArgs a, const BatchArgs* pa, int link_blocks, int hydro_blocks)
+{
+    const int b = (int)blockIdx.x, wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    if (b < link_blocks) {
+        const int n = *a.count;
+        RegridArgs r = a.links;
+        for (int l = 4 * b + wave; l < n; l += 4 * link_blocks) {
+            r.q = link_buffer(a, a.link_scen[l]);
+            if (r.q) average_link<MX, MY>(r, l, lane);
+        }
+    } else if (b < link_blocks + hydro_blocks) {
+        const int n = pa->nscen;
+        for (int s = 4 * (b - link_blocks) + wave; s < n; s += 4 * hydro_blocks) {
+            ScenCtrl* c = a.ctrl + s;
+            if (!c->active || c->hyd_rows == 0) continue;
+            const double hu = hydro_interpolate(c->hyd, c->hyd + c->hyd_rows, c->hyd_rows, c->t);
+            if (lane == 0) c->hyd_hu = hu;
+        }
+    } else {
+        classify(*pa, b - link_blocks - hydro_blocks);
+    }
+}
+
+template <int MX, int MY>
+__global__ void __launch_bounds__(256) k_ghost_level(GhostLevelArgs a)
+{
+    __shared__ double L[4 * Geo<MX, MY>::NP2];
+    __shared__ double hu_sh;
+    __shared__ PatchDesc D;
+    const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+    const int n = *a.count;
+    for (int k = (int)blockIdx.x; k < n; k += gridDim.x) {
+        const GhostItem it = a.items[k];
+        RegridArgs r = a.links;
+        r.q = link_buffer(a, it.scen);
+        if (!r.q) continue;
+        __syncthreads();  // the previous patch's links have read D
+        constexpr int W = sizeof(PatchDesc) / sizeof(int);
+        if (threadIdx.x < W) ((int*)&D)[threadIdx.x] = ((const int*)(a.desc + it.patch))[threadIdx.x];
+        __syncthreads();
+        if (it.inflow) {
+            const ScenCtrl* c = a.ctrl + it.scen;
+            inflow_patch<MX, MY>(L, &hu_sh, r.q, a.aux, &D, c, it.patch, a.buf < 0 ? c->t : a.t, a.P,
+                                 a.buf < 0 ? &c->hyd_hu : nullptr);
+            __syncthreads();
+        }
+        for (int l = it.first + wave; l < it.end; l += 4) interpolate_link<MX, MY>(r, l, lane, D.nbr);
     }
 }
 
@@ -2152,6 +2274,35 @@ hipError_t launch_interpolate_ghost(int mx, int my, const RegridArgs& a, hipStre
 #define GF_IG(M, N) k_interpolate_ghost<M, N><<<a.n, 64, 0, st>>>(a)
     GF_SIZES(GF_IG)
 #undef GF_IG
+    return hipGetLastError();
+}
+
+hipError_t launch_ghost_level(int mx, int my, const GhostLevelArgs& a, int grid, hipStream_t st)
+{
+#define GF_GL(M, N) k_ghost_level<M, N><<<grid, 256, 0, st>>>(a)
+    GF_SIZES(GF_GL)
+#undef GF_GL
+    return hipGetLastError();
+}
+
+hipError_t launch_ghost_begin(int mx, int my, const GhostLevelArgs& a, const BatchArgs* da, int slots, int link_blocks,
+                              int hydro_blocks, hipStream_t st)
+{
+    const int grid = link_blocks + hydro_blocks + (da ? (slots + 255) / 256 : 0);
+    if (grid <= 0) return hipSuccess;
+#define GF_GB(M, N) k_ghost_begin<M, N><<<grid, 256, 0, st>>>(a, da, link_blocks, hydro_blocks)
+    GF_SIZES(GF_GB)
+#undef GF_GB
+    return hipGetLastError();
+}
+
+hipError_t launch_begin(int mx, int my, const BatchArgs* da, int slots, const InflowArgs& in, int inflow_blocks,
+                        hipStream_t st)
+{
+    const int grid = inflow_blocks + (slots + 255) / 256;
+#define GF_BE(M, N) k_begin<M, N><<<grid, 256, 0, st>>>(da, in, inflow_blocks)
+    GF_SIZES(GF_BE)
+#undef GF_BE
     return hipGetLastError();
 }
 
