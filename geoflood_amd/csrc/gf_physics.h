@@ -77,16 +77,20 @@ __device__ __forceinline__ void middle_speeds(const Recip& rL, const Recip& rR, 
     const double delu = uR - uL;
     const double F_min = delu + 2.0 * ((left ? sgR : sgL) - (left ? sgL : sgR));
     const double F_max = delu + dh * root<FAST>(quot<FAST>(halfg * (h_max + h_min), h_max * h_min));
-    // The three branches leave hm (and, for two shocks, u1m, u2m); sqrt(g*hm)
-    // and the speeds are formed once after them, so that a wave whose lanes
-    // take different branches pays for the shared part only once.
-    double hm, u1m = 0.0, u2m = 0.0;
-    int kind;  // 0: two rarefactions, 1: two shocks, 2: one shock, one rarefaction
-    if (F_min > 0.0) {
-        const double t = vmax<FAST>(0.0, -delu + 2.0 * (sgL + sgR));
-        hm = P.inv16g * (t * t);
-        kind = 0;
-    } else if (F_max <= 0.0) {
+    // two rarefactions and the shock-rarefaction pair are formed by every lane,
+    // the two-shock case by the lanes that have it: a branch costs a wave more
+    // than the few instructions of the first two
+    const bool rare = F_min > 0.0, shocks = !rare && F_max <= 0.0;
+    // F0 = delu + 2(sqrt(g h0) - sqrt(g h_max)) + (h0 - h_min) sqrt(g/2 (1/h0 + 1/h_min))
+    // at h0 = h_min: the last product is (+0) times a finite positive
+    // whenever g/h_min cannot overflow, so F0 is F_min + 0.0 exactly
+    const double F0 = FAST || (h_min >= 1e-150 && g <= 1e150)
+                          ? F_min
+                          : F_min + 0.0 * sqrt(halfg * (1 / h_min + 1 / h_min));
+    const double tr = vmax<FAST>(0.0, -delu + 2.0 * (sgL + sgR));
+    double hm = rare ? P.inv16g * (tr * tr) : h_min - quot<FAST>(F0, quot<FAST>(F_max - F0, dh));
+    double u1m = 0.0, u2m = 0.0;
+    if (shocks) {
         // one Newton step on sqrt(h) from h0 = h_max.  The side at h0 has a zero
         // (h0 - h) factor: only the other side's terms remain, and 1/h0 is that
         // side's own 1/h
@@ -94,27 +98,16 @@ __device__ __forceinline__ void middle_speeds(const Recip& rL, const Recip& rR, 
         const double i_min = quot<FAST>(1.0, left ? rR : rL);
         const double gs = root<FAST>(halfg * (i_max + i_max));
         const double go = root<FAST>(halfg * (i_max + i_min));
-        const double F0 = delu + dh * go;
+        const double F0s = delu + dh * go;
         const double T = quot<FAST>(g * dh, 4.0 * (h_max * h_max) * go);
         const double dfdh = left ? (gs + go) - T : (go - T) + gs;
         const double rh = root<FAST>(h_max);
         const double slope = 2.0 * rh * dfdh;
-        const double t = rh - quot<FAST>(F0, slope);
+        const double t = rh - quot<FAST>(F0s, slope);
         hm = t * t;
         const double im = quot<FAST>(1.0, hm);
         u1m = uL - (hm - hL) * root<FAST>(halfg * (im + (left ? i_max : i_min)));
         u2m = uR + (hm - hR) * root<FAST>(halfg * (im + (left ? i_min : i_max)));
-        kind = 1;
-    } else {
-        // F0 = delu + 2(sqrt(g h0) - sqrt(g h_max)) + (h0 - h_min) sqrt(g/2 (1/h0 + 1/h_min))
-        // at h0 = h_min: the last product is (+0) times a finite positive
-        // whenever g/h_min cannot overflow, so F0 is F_min + 0.0 exactly
-        const double F0 = FAST || (h_min >= 1e-150 && g <= 1e150)
-                              ? F_min
-                              : F_min + 0.0 * sqrt(halfg * (1 / h_min + 1 / h_min));
-        const double slope = quot<FAST>(F_max - F0, dh);
-        hm = h_min - quot<FAST>(F0, slope);
-        kind = 2;
     }
     const double sghm = root<FAST>(g * hm);
     // two rarefactions:      s1m = (uL + 2 sqrt(g hL)) - 3 sghm, s2m = (uR - 2 sqrt(g hR)) + 3 sghm
@@ -122,16 +115,9 @@ __device__ __forceinline__ void middle_speeds(const Recip& rL, const Recip& rR, 
     //                        else:    a = uR - 2 sqrt(g hR), s2m = a + 3 sghm, s1m = a + sghm
     // two shocks:            s1m = u1m - sghm, s2m = u2m + sghm
     const double A = uL + 2.0 * sgL, B = uR - 2.0 * sgR, s3 = 3.0 * sghm;
-    if (kind == 1) {
-        s1m = u1m - sghm;
-        s2m = u2m + sghm;
-    } else if (kind == 0 || hL > hR) {
-        s1m = A - s3;
-        s2m = kind == 0 ? B + s3 : A - sghm;
-    } else {
-        s1m = B + sghm;
-        s2m = B + s3;
-    }
+    const bool fromL = hL > hR;
+    s1m = shocks ? u1m - sghm : (rare || fromL) ? A - s3 : B + sghm;
+    s2m = shocks ? u2m + sghm : (rare || !fromL) ? B + s3 : A - sghm;
 }
 
 // hm of riemanntype(h, h, u, -u), h > drytol, the wall test of rpn2
@@ -167,50 +153,36 @@ __device__ __forceinline__ double wall_hstar(const Recip& r, double u, double sg
 // speeds s[3] and the f-waves in compressed form, wave 1 (3), the normal
 // momentum of wave 2, wave 3 (3): the other two components of wave 2 are exact
 // zeros (geoclaw_riemann_utils.f:289-299: fw(1,2) = beta(2)*r(2,2) = 0,
-// fw(3,2) = 0).  A face with both sides dry leaves zeros, as the reference
-// does.  With RC, rc holds the right-hand cell's quantities when it is wet.
+// fw(3,2) = 0).  A face with both sides dry gives zeros, as the reference
+// leaves them.  With RC, rc holds the right-hand cell's quantities when it is wet.
 template <bool FAST, bool RC>
 __device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, double bL,
                                           double hR, double huR, double hvR, double bR,
                                           const Params& P, double s[3], double w[7], const CellVel& rc = CellVel{})
 {
     const double g = P.grav, drytol = P.dry_tolerance, halfg = P.halfg;
-#pragma unroll
-    for (int k = 0; k < 3; k++) s[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < 7; k++) w[k] = 0.0;
-    if (hL <= drytol && hR <= drytol) return;
     const bool wetL = hL > drytol, wetR = hR > drytol;
-    double uR, vR, phiR, sgR, uL, vL, phiL, sgL;
-    Recip rL, rR;
-    if (wetR) {
-        if (RC) {
-            rR = Recip{hR, rc.y};
-            uR = rc.u; vR = rc.v; sgR = rc.sg;
-        } else {
-            rR = recip<FAST>(hR);
-            uR = quot<FAST>(huR, rR); vR = quot<FAST>(hvR, rR); sgR = root<FAST>(g * hR);
-        }
-        phiR = halfg * (hR * hR) + quot<FAST>(huR * huR, rR);
-    } else {
-        hR = 0.0; huR = 0.0; hvR = 0.0; uR = 0.0; vR = 0.0; phiR = 0.0; sgR = 0.0;
-        rR = Recip{0.0, 0.0};
-    }
-    if (wetL) {
-        rL = recip<FAST>(hL);
-        uL = quot<FAST>(huL, rL); vL = quot<FAST>(hvL, rL); sgL = root<FAST>(g * hL);
-        phiL = halfg * (hL * hL) + quot<FAST>(huL * huL, rL);
-    } else {
-        hL = 0.0; huL = 0.0; hvL = 0.0; uL = 0.0; vL = 0.0; phiL = 0.0; sgL = 0.0;
-        rL = Recip{0.0, 0.0};
-    }
-
-    // the wall test of whichever side is dry: riemanntype(hL, hL, uL, -uL) or
-    // riemanntype(hR, hR, -uR, uR), one call for both kinds of lane; a dry side
-    // that the water cannot climb is a wall (the wet side mirrored)
-    const bool front = !wetL || !wetR;
+    const bool still = hL <= drytol && hR <= drytol;
+    // Both sides as if wet; the lanes of a wave that have a dry side are put
+    // right below, in code that the other waves skip.
+    Recip rL = recip<FAST>(hL), rR = RC ? Recip{hR, rc.y} : recip<FAST>(hR);
+    double uL = quot<FAST>(huL, rL), vL = quot<FAST>(hvL, rL), sgL = root<FAST>(g * hL);
+    double uR = RC ? rc.u : quot<FAST>(huR, rR), vR = RC ? rc.v : quot<FAST>(hvR, rR);
+    double sgR = RC ? rc.sg : root<FAST>(g * hR);
+    double phiL = halfg * (hL * hL) + quot<FAST>(huL * huL, rL);
+    double phiR = halfg * (hR * hR) + quot<FAST>(huR * huR, rR);
+    const bool front = !(wetL && wetR);
     bool wallL = false, wallR = false;
     if (front) {
+        if (!wetL) {
+            hL = 0.0; huL = 0.0; hvL = 0.0; uL = 0.0; vL = 0.0; phiL = 0.0; sgL = 0.0;
+        }
+        if (!wetR) {
+            hR = 0.0; huR = 0.0; hvR = 0.0; uR = 0.0; vR = 0.0; phiR = 0.0; sgR = 0.0;
+        }
+        // the wall test of whichever side is dry: riemanntype(hL, hL, uL, -uL) or
+        // riemanntype(hR, hR, -uR, uR), one call for both kinds of lane; a dry
+        // side that the water cannot climb is a wall (the wet side mirrored)
         const double hstar = wall_hstar<FAST>(wetL ? rL : rR, wetL ? uL : -uR, wetL ? sgL : sgR, P);
         if (!wetR) {
             const double hstartest = fmaxf64(hL, hstar);
@@ -245,11 +217,10 @@ __device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, dou
     const double delb = bR - bL;
 
     double s1m, s2m;
-    if (fminf64(hR, hL) <= drytol) {
+    middle_speeds<FAST>(rL, rR, uL, uR, sgL, sgR, P, s1m, s2m);
+    if (front && fminf64(hR, hL) <= drytol) {
         s1m = uR + uL - 2.0 * sgR + 2.0 * sgL;
         s2m = s1m;
-    } else {
-        middle_speeds<FAST>(rL, rR, uL, uR, sgL, sgR, P, s1m, s2m);
     }
 
     // (the sign of a zero speed matters to the limiter: Flang's MIN and MAX)
@@ -283,16 +254,10 @@ __device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, dou
         const double hs = hstarHLL * (sE2 - sE1);
         const double q2 = quot<FAST>(hs, sE2);
         const double q1 = quot<FAST>(hs, sE1);
-        if (sE1 < -crit && sE2 > crit) {
-            deldelh = vmin<FAST>(deldelh, q2);
-            deldelh = vmax<FAST>(deldelh, q1);
-        } else if (sE1 >= crit) {
-            deldelh = vmin<FAST>(deldelh, q1);
-            deldelh = vmax<FAST>(deldelh, -hL);
-        } else if (sE2 <= -crit) {
-            deldelh = vmin<FAST>(deldelh, hR);
-            deldelh = vmax<FAST>(deldelh, q2);
-        }
+        const bool sub = sE1 < -crit && sE2 > crit, right = !sub && sE1 >= crit, left = !sub && !right && sE2 <= -crit;
+        const double upper = sub ? q2 : right ? q1 : hR, lower = sub ? q1 : right ? -hL : q2;
+        const double bounded = vmax<FAST>(vmin<FAST>(deldelh, upper), lower);
+        deldelh = (sub || right || left) ? bounded : deldelh;
         deldelphi = sonic ? -g * hbar * delb : quot<FAST>(gn * s1s2tilde, rb);
         deldelphi = vmin<FAST>(deldelphi, g * vmax<FAST>(-hL * delb, -hR * delb));
         deldelphi = vmax<FAST>(deldelphi, g * vmin<FAST>(-hL * delb, -hR * delb));
@@ -313,22 +278,23 @@ __device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, dou
     const double fw00 = beta0 * r10, fw20 = beta2 * r12;
     double fw02 = fw00 * vL, fw22 = fw20 * vR;
     const double rest = hR * uR * vR - hL * uL * vL - fw02 - fw22;
-    if (huL + fw00 <= 0.0)
-        fw02 = fw02 + rest;
-    else
-        fw22 = fw22 + rest;
+    const bool below = huL + fw00 <= 0.0;
+    fw02 = below ? fw02 + rest : fw02;
+    fw22 = below ? fw22 : fw22 + rest;
 
     s[0] = lam0; s[1] = lam1; s[2] = lam2;
     w[0] = fw00; w[1] = beta0 * r20; w[2] = fw02;
     w[3] = beta1;
     w[4] = fw20; w[5] = beta2 * r22; w[6] = fw22;
-    // eliminate ghost fluxes for the wall problem (rpn2_geoclaw.f:303-309)
-    if (wallL || wallR) {
-        const double w0 = wallL ? 0.0 : 1.0, w2 = wallR ? 0.0 : 1.0;
-        s[0] = s[0] * w0; s[1] = s[1] * 0.0; s[2] = s[2] * w2;
-        w[0] = w[0] * w0; w[1] = w[1] * w0; w[2] = w[2] * w0;
-        w[3] = w[3] * 0.0;
-        w[4] = w[4] * w2; w[5] = w[5] * w2; w[6] = w[6] * w2;
+    if (front) {
+        // eliminate ghost fluxes for the wall problem (rpn2_geoclaw.f:303-309);
+        // no waves between dry cells (there the products are of garbage)
+        const double w0 = wallL ? 0.0 : 1.0, w1 = wallL || wallR ? 0.0 : 1.0, w2 = wallR ? 0.0 : 1.0;
+        const double f[3] = {w0, w1, w2};
+#pragma unroll
+        for (int k = 0; k < 3; k++) s[k] = still ? 0.0 : s[k] * f[k];
+#pragma unroll
+        for (int k = 0; k < 7; k++) w[k] = still ? 0.0 : w[k] * f[k / 3 < 1 ? 0 : (k == 3 ? 1 : 2)];
     }
 }
 

@@ -997,11 +997,15 @@ __device__ __forceinline__ void dry_item(const BatchArgs* pa, int k, int next, i
 // (wet_item), then the dry patches in items of dry_per_item (dry_item), from
 // the item queues.  The streaming dry items fill the tail that the
 // compute-bound active items leave when the list runs out.
-// 8x8 patches: the register budget for three waves per SIMD (the kernels
-// need 170 VGPRs, two waves, without it; no spills at 167) is 8% faster at
-// ten thousand active patches; larger patches keep their own allocation.
+// step_waves: the waves per SIMD that the registers must allow.  __WAVES__
+template <int TX, int TY, int NT>
+constexpr int step_waves()
+{
+    return Geo<TX, TY>::NPOS <= NT && TX < 32 ? 4 : 1;
+}
+
 template <int MX, int MY, int TX, int TY, int NT, int NPP, bool FREG, bool DEF>
-__global__ void __launch_bounds__(NT * NPP, (MX == 8 ? 3 : 1)) k_all(const BatchArgs* pa)
+__global__ void __launch_bounds__(NT * NPP, (step_waves<TX, TY, NT>())) k_all(const BatchArgs* pa)
 {
     using TL = Tiling<MX, MY, TX, TY>;
     constexpr int NB = NT * NPP;  // threads of the workgroup
