@@ -242,9 +242,10 @@ struct gf_pool {
     double* h_cfl = nullptr;    // pinned
     // batched path
     double* hmax2 = nullptr;               // [2][capacity]
-    unsigned long long* cflbits = nullptr; // [capacity] per scenario
+    unsigned long long* cflbits = nullptr; // [gf::QUEUES][capacity] per scenario
     int* list_wet = nullptr;
     int* list_dry = nullptr;
+    gf::RegionSrc* regions = nullptr;      // [capacity][gf::REGIONS] halo sources of the described slots
     int* counters = nullptr;               // gf::NCOUNTERS
     long long* stats = nullptr;            // [4] see gf_pool_stats
     gf::BatchArgs* d_args = nullptr;       // device copy read by the persistent kernel
@@ -458,8 +459,9 @@ const char* gf_last_error(void) { return g_err.c_str(); }
 long long gf_pool_bytes(int mx, int my, int mbc, int capacity)
 {
     const long long np2 = (long long)(mx + 2 * mbc) * (my + 2 * mbc);
-    const long long per = (2 * 3 * np2 + np2) * 8 + (long long)sizeof(PatchDesc) + 8 /*cfl*/ + 16 /*hmax*/ +
-                          8 /*cflbits*/ + 8 /*lists*/ + 8 /*legacy hmax*/ + 4 /*dry age*/ + sizeof(ScenCtrl);
+    const long long per = (2 * 3 * np2 + np2) * 8 + (long long)sizeof(PatchDesc) +
+                          (long long)(gf::REGIONS * sizeof(gf::RegionSrc)) + 8 /*cfl*/ + 16 /*hmax*/ +
+                          8 * gf::QUEUES /*cflbits*/ + 8 /*lists*/ + 8 /*legacy hmax*/ + 4 /*dry age*/ + sizeof(ScenCtrl);
     const long long staging = (long long)kChunk * 4 * np2 * 8;
     return per * capacity + staging;
 }
@@ -634,9 +636,10 @@ try {
               hipHostMalloc(&p->h_stage, chunk * 4 * p->np2 * sizeof(double), hipHostMallocDefault) == hipSuccess &&
               hipHostMalloc(&p->h_cfl, (size_t)capacity * sizeof(double), hipHostMallocDefault) == hipSuccess &&
               hipMalloc(&p->hmax2, (size_t)2 * capacity * sizeof(double)) == hipSuccess &&
-              hipMalloc(&p->cflbits, (size_t)capacity * sizeof(unsigned long long)) == hipSuccess &&
+              hipMalloc(&p->cflbits, (size_t)gf::QUEUES * capacity * sizeof(unsigned long long)) == hipSuccess &&
               hipMalloc(&p->list_wet, (size_t)capacity * sizeof(int)) == hipSuccess &&
               hipMalloc(&p->list_dry, (size_t)capacity * sizeof(int)) == hipSuccess &&
+              hipMalloc(&p->regions, (size_t)capacity * gf::REGIONS * sizeof(gf::RegionSrc)) == hipSuccess &&
               hipMalloc(&p->counters, gf::NCOUNTERS * sizeof(int)) == hipSuccess &&
               hipMalloc(&p->stats, 4 * sizeof(long long)) == hipSuccess &&
               hipMalloc(&p->d_args, sizeof(gf::BatchArgs)) == hipSuccess &&
@@ -656,7 +659,7 @@ try {
              hipMemsetAsync(p->hmax, 0, (size_t)capacity * sizeof(double), g.stream) == hipSuccess &&
              hipMemsetAsync(p->ctrl, 0, (size_t)capacity * sizeof(ScenCtrl), g.stream) == hipSuccess &&
              hipMemsetAsync(p->hmax2, 0, (size_t)2 * capacity * sizeof(double), g.stream) == hipSuccess &&
-             hipMemsetAsync(p->cflbits, 0, (size_t)capacity * sizeof(unsigned long long), g.stream) == hipSuccess &&
+             hipMemsetAsync(p->cflbits, 0, (size_t)gf::QUEUES * capacity * sizeof(unsigned long long), g.stream) == hipSuccess &&
              hipMemsetAsync(p->counters, 0, gf::NCOUNTERS * sizeof(int), g.stream) == hipSuccess &&
              hipMemsetAsync(p->stats, 0, 4 * sizeof(long long), g.stream) == hipSuccess &&
              hipMemsetAsync(p->tile_cfl, 0, (size_t)capacity * sizeof(unsigned long long), g.stream) == hipSuccess &&
@@ -708,6 +711,7 @@ try {
     hipFree(p->cflbits);
     hipFree(p->list_wet);
     hipFree(p->list_dry);
+    hipFree(p->regions);
     hipFree(p->counters);
     hipFree(p->stats);
     hipFree(p->d_args);
@@ -756,6 +760,7 @@ try {
     p->h_ctrl.assign(p->capacity, ScenCtrl{});
     free_hydrographs(p);
     HIPCHK(hipMemcpyAsync(p->desc, p->h_desc.data(), sizeof(PatchDesc) * p->capacity, hipMemcpyHostToDevice, g.stream));
+    HIPCHK(gf::launch_regions(p->mx, p->my, p->desc, p->regions, 0, n, g.stream));
     HIPCHK(hipMemsetAsync(p->ctrl, 0, sizeof(ScenCtrl) * p->capacity, g.stream));
     if (int r = reset_dry_age(p, 0, p->capacity)) return r;
     HIPCHK(hipStreamSynchronize(g.stream));
@@ -791,6 +796,7 @@ try {
     }
     if (first + n > p->n) p->n = first + n;
     HIPCHK(hipMemcpyAsync(p->desc + first, p->h_desc.data() + first, sizeof(PatchDesc) * n, hipMemcpyHostToDevice, g.stream));
+    HIPCHK(gf::launch_regions(p->mx, p->my, p->desc, p->regions, first, n, g.stream));
     if (int r = reset_dry_age(p, first, n)) return r;
     HIPCHK(hipStreamSynchronize(g.stream));
     return GF_OK;
@@ -1222,7 +1228,7 @@ try {
     HIPCHK(hipStreamSynchronize(g.stream));
     free_hydrographs(p);
     if (int r = rebuild_inflow(p)) return r;
-    HIPCHK(hipMemsetAsync(p->cflbits, 0, sizeof(unsigned long long) * p->capacity, g.stream));
+    HIPCHK(hipMemsetAsync(p->cflbits, 0, sizeof(unsigned long long) * gf::QUEUES * p->capacity, g.stream));
     if (int r = reset_dry_age(p, 0, p->capacity)) return r;
     HIPCHK(hipStreamSynchronize(g.stream));
     p->graph_dirty = true;
@@ -1311,6 +1317,7 @@ static gf::BatchArgs host_batch_args(gf_pool* p)
     a.nscen = p->nscen;  // the scenario ids in use so far; removed ones are inactive
     a.list_wet = p->list_wet;
     a.list_dry = p->list_dry;
+    a.regions = p->regions;
     a.counters = p->counters;
     a.stats = p->stats;
     a.P = g.P;
@@ -1990,7 +1997,7 @@ try {
     }
     // undo the candidates' side effects on the attempt's counters and maxima
     HIPCHK(hipMemsetAsync(p->counters, 0, gf::NCOUNTERS * sizeof(int), g.stream));
-    HIPCHK(hipMemsetAsync(p->cflbits, 0, (size_t)p->capacity * sizeof(unsigned long long), g.stream));
+    HIPCHK(hipMemsetAsync(p->cflbits, 0, (size_t)gf::QUEUES * p->capacity * sizeof(unsigned long long), g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
     p->variant = saved;
     p->wet_grid = 0;

@@ -154,21 +154,21 @@ __device__ __forceinline__ double wall_hstar(const Recip& r, double u, double sg
 // momentum of wave 2, wave 3 (3): the other two components of wave 2 are exact
 // zeros (geoclaw_riemann_utils.f:289-299: fw(1,2) = beta(2)*r(2,2) = 0,
 // fw(3,2) = 0).  A face with both sides dry gives zeros, as the reference
-// leaves them.  With RC, rc holds the right-hand cell's quantities when it is wet.
-template <bool FAST, bool RC>
+// leaves them.  cL, cR: the two cells' velocities, sqrt(g h) and reciprocal
+// depth, used where the cell is wet.
+template <bool FAST>
 __device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, double bL,
                                           double hR, double huR, double hvR, double bR,
-                                          const Params& P, double s[3], double w[7], const CellVel& rc = CellVel{})
+                                          const CellVel& cL, const CellVel& cR,
+                                          const Params& P, double s[3], double w[7])
 {
     const double g = P.grav, drytol = P.dry_tolerance, halfg = P.halfg;
     const bool wetL = hL > drytol, wetR = hR > drytol;
     const bool still = hL <= drytol && hR <= drytol;
     // Both sides as if wet; the lanes of a wave that have a dry side are put
     // right below, in code that the other waves skip.
-    Recip rL = recip<FAST>(hL), rR = RC ? Recip{hR, rc.y} : recip<FAST>(hR);
-    double uL = quot<FAST>(huL, rL), vL = quot<FAST>(hvL, rL), sgL = root<FAST>(g * hL);
-    double uR = RC ? rc.u : quot<FAST>(huR, rR), vR = RC ? rc.v : quot<FAST>(hvR, rR);
-    double sgR = RC ? rc.sg : root<FAST>(g * hR);
+    Recip rL{hL, cL.y}, rR{hR, cR.y};
+    double uL = cL.u, vL = cL.v, sgL = cL.sg, uR = cR.u, vR = cR.v, sgR = cR.sg;
     double phiL = halfg * (hL * hL) + quot<FAST>(huL * huL, rL);
     double phiR = halfg * (hR * hR) + quot<FAST>(huR * huR, rR);
     const bool front = !(wetL && wetR);
@@ -223,9 +223,10 @@ __device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, dou
         s2m = s1m;
     }
 
-    // (the sign of a zero speed matters to the limiter: Flang's MIN and MAX)
-    const double sE1 = fminf64(fminf64(sL, sRoe1), s2m);
-    const double sE2 = fmaxf64(fmaxf64(sR, sRoe2), s1m);
+    // (the sign of a zero speed matters to the limiter; in the fast range these
+    // are sums, whose zeros are all +0)
+    const double sE1 = vmin<FAST>(vmin<FAST>(sL, sRoe1), s2m);
+    const double sE2 = vmax<FAST>(vmax<FAST>(sR, sRoe2), s1m);
     const double lam0 = sE1, lam2 = sE2;
     const double lam1 = 0.5 * (lam0 + lam2);
     // r(:,1) = (1, lam0, lam0^2), r(:,2) = (0, 0, 1), r(:,3) = (1, lam2, lam2^2)
@@ -360,27 +361,23 @@ __device__ __forceinline__ bool quotients_tiny(const double (&a)[N])
 // amdq of the face on the cell's right/top and the imp = 2 split of apdq of
 // the face on its left/bottom share the same Jacobian).
 struct Rpt2Cell {
-    bool active;
-    double u, s0, s2;
-    double dn[3], up[3];  // the speeds of the waves that go down / up, 0 for the others
+    bool active, lo, hi;  // lo / hi: the surface reaches the neighbour below / above
+    double u, s0, s1, s2;
 };
 
+template <bool FAST>
 __device__ __forceinline__ Rpt2Cell rpt2_setup(double h, double u, double v, double sg, double b,
                                                double topo1, double topo3, double tol)
 {
     Rpt2Cell c;
     const double eta = h + b;
-    c.active = !(h <= tol) && !(eta < fminf64(topo1, topo3));
+    c.active = !(h <= tol) && !(eta < vmin<FAST>(topo1, topo3));
+    c.lo = eta >= topo1;
+    c.hi = eta >= topo3;
     c.u = u;
     c.s0 = v - sg;
+    c.s1 = v;
     c.s2 = v + sg;
-    const double sv[3] = {c.s0, v, c.s2};
-    const bool lo = eta >= topo1, hi = eta >= topo3;
-#pragma unroll
-    for (int mw = 0; mw < 3; mw++) {
-        c.dn[mw] = (sv[mw] < 0.0 && lo) ? sv[mw] : 0.0;
-        c.up[mw] = (sv[mw] > 0.0 && hi) ? sv[mw] : 0.0;
-    }
     return c;
 }
 
@@ -418,15 +415,20 @@ __device__ __forceinline__ void cell_transverse(const Rpt2Cell& c, const double 
     }
     const double b1[3] = {be[0], -c.u * am_next[0] + am_next[1], be[1]};
     const double b2[3] = {be[2], -c.u * ap_own[0] + ap_own[1], be[3]};
+    // the waves that go down are those of negative speed, where the surface
+    // reaches the bed below, and the others count with speed 0; likewise up
+    const double dn[3] = {vmin<FAST>(c.s0, 0.0), vmin<FAST>(c.s1, 0.0), vmin<FAST>(c.s2, 0.0)};
+    const double up[3] = {vmax<FAST>(c.s0, 0.0), vmax<FAST>(c.s1, 0.0), vmax<FAST>(c.s2, 0.0)};
+    const double hlo = c.lo ? hd : 0.0, hhi = c.hi ? hd : 0.0;
     double d1[3], d2[3];
-    rpt2_side(c.dn, b1, c, d1);
-    rpt2_side(c.dn, b2, c, d2);
+    rpt2_side(dn, b1, c, d1);
+    rpt2_side(dn, b2, c, d2);
 #pragma unroll
-    for (int k = 0; k < 3; k++) G1[k] = -(hd * d1[k]) - hd * d2[k];
-    rpt2_side(c.up, b1, c, d1);
-    rpt2_side(c.up, b2, c, d2);
+    for (int k = 0; k < 3; k++) G1[k] = -(hlo * d1[k]) - hlo * d2[k];
+    rpt2_side(up, b1, c, d1);
+    rpt2_side(up, b2, c, d2);
 #pragma unroll
-    for (int k = 0; k < 3; k++) G2[k] = -(hd * d1[k]) - hd * d2[k];
+    for (int k = 0; k < 3; k++) G2[k] = -(hhi * d1[k]) - hhi * d2[k];
 }
 
 // Manning friction of fc2d_geoclaw_src2 (geoclaw_src2_fort.f90:41-71) for one

@@ -57,6 +57,30 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
+// One step of a wave reduction on the register shuffles of the vector unit
+// (lanes without a source keep their own value): a shift within rows of 16,
+// or a row's last lane to the next row or rows.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double max_from(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = (int)b, hi = (int)(b >> 32);
+    const unsigned l = (unsigned)__builtin_amdgcn_update_dpp(lo, lo, CTRL, ROWS, 0xf, false);
+    const unsigned h = (unsigned)__builtin_amdgcn_update_dpp(hi, hi, CTRL, ROWS, 0xf, false);
+    return max_nan(v, __longlong_as_double((long long)((unsigned long long)h << 32 | l)));
+}
+
+// Maximum over the wave, valid in its last lane.
+__device__ __forceinline__ double wave_max_last(double v)
+{
+    v = max_from<0x111, 0xf>(v);  // row_shr:1
+    v = max_from<0x112, 0xf>(v);
+    v = max_from<0x114, 0xf>(v);
+    v = max_from<0x118, 0xf>(v);
+    v = max_from<0x142, 0xa>(v);  // row_bcast:15
+    return max_from<0x143, 0xc>(v);  // row_bcast:31
+}
+
 // Dot product of two 3-vectors given in direction-local order (h, n, t),
 // summed in the reference's physical component order (h, hu, hv):
 // x-direction (h, n, t) = (h, hu, hv); y-direction (h, n, t) = (h, hv, hu).
@@ -67,17 +91,35 @@ __device__ __forceinline__ double pdot(const double* a, const double* b)
     return a[0] * b[0] + a[2] * b[2] + a[1] * b[1];
 }
 
+// A face's own waves (at) and, wave by wave, the neighbour's that the limiter
+// compares with: the face before (-step) when the wave moves forwards, else the
+// face after.
+template <int NPOS>
+__device__ __forceinline__ void load_waves(const double* at, int step, const double s[3], double w[7], double wn[7])
+{
+#pragma unroll
+    for (int k = 0; k < 7; k++) w[k] = at[k * NPOS];
+    const double* n0 = at + (s[0] > 0.0 ? -step : step);
+    const double* n1 = at + (s[1] > 0.0 ? -step : step);
+    const double* n2 = at + (s[2] > 0.0 ? -step : step);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        wn[k] = n0[k * NPOS];
+        wn[4 + k] = n2[(4 + k) * NPOS];
+    }
+    wn[3] = n1[3 * NPOS];
+}
+
 // Limiter, second-order correction and fluctuation split of one face
 // (geoclaw_flux2fw_fort.f:143-224 with geoclaw_limiter_fort.f:34-58 and
-// philim.f).  w: own compressed unlimited waves; wl / wr: those of the faces
-// before / after along the sweep.  Outputs in direction-local order: faddm,
+// philim.f).  w: own compressed unlimited waves; wn: for each wave that of the
+// face it comes from (load_waves).  Outputs in direction-local order: faddm,
 // faddp (flux increments) and amdq*, apdq* (fluctuations handed to rpt2).
 // DEF: the default method (order 2, transverse 2, MC limiter on all three
 // families) fixed at compile time; otherwise the method is read from P.
 template <int DIR, bool DEF, bool FAST>
 __device__ __forceinline__ void face_second_order(const double w[7], const double s[3],
-                                                  const double wl[7], const double wr[7],
-                                                  double dtdx, const Params& P,
+                                                  const double wn[7], double dtdx, const Params& P,
                                                   double faddm[3], double faddp[3],
                                                   double amq[3], double apq[3])
 {
@@ -94,14 +136,11 @@ __device__ __forceinline__ void face_second_order(const double w[7], const doubl
         }
         return;
     }
-    // limiter on the three wave families with the unlimited neighbour on the
-    // side the wave comes from (wave 2 has its normal momentum only): the
-    // ratios b / a of the dot products, then the factor of each family (1
+    // limiter on the three wave families (wave 2 has its normal momentum only):
+    // the ratios b / a of the dot products, then the factor of each family (1
     // where the wave vanishes or its family is not limited)
     const double a[3] = {pdot<DIR>(w, w), w[3] * w[3], pdot<DIR>(w + 4, w + 4)};
-    const double b[3] = {s[0] > 0.0 ? pdot<DIR>(wl, w) : pdot<DIR>(w, wr),
-                         s[1] > 0.0 ? wl[3] * w[3] : w[3] * wr[3],
-                         s[2] > 0.0 ? pdot<DIR>(wl + 4, w + 4) : pdot<DIR>(w + 4, wr + 4)};
+    const double b[3] = {pdot<DIR>(wn, w), wn[3] * w[3], pdot<DIR>(wn + 4, w + 4)};
     double r[3];
 #pragma unroll
     for (int mw = 0; mw < 3; mw++) r[mw] = quot<FAST>(b[mw], a[mw]);
@@ -132,10 +171,7 @@ __device__ __forceinline__ void face_second_order(const double w[7], const doubl
     }
 }
 
-// Maximum over a group of NT threads (the workgroup, or one of the groups
-// of a workgroup that steps several patches; ltid is the thread's index in
-// its group, NT a multiple of 64) with one barrier of the whole workgroup;
-// the result is valid in the group's thread 0.
+// Maximum over a workgroup of NT threads; the result is valid in thread 0.
 template <int NT>
 __device__ __forceinline__ double block_max(double v, double* red, int ltid)
 {
@@ -150,21 +186,24 @@ __device__ __forceinline__ double block_max(double v, double* red, int ltid)
     return r;
 }
 
-// Group maxima of two values with one barrier (results valid in every
-// thread of the group).  red holds 2 * NT / 64 doubles per group; the caller
-// guarantees that no thread still reads red from an earlier use (a barrier
-// separates them).
+// Maxima of two values over the group of NT threads that steps a tile (ltid:
+// the thread's index in its group), valid in the group's thread 0, the only
+// one that waits for them: the others go on to their next item after the one
+// barrier.  red holds 2 * NT / 64 doubles per group; the caller guarantees
+// that no thread still reads red from an earlier use (a barrier separates
+// them).
 template <int NT>
-__device__ __forceinline__ void block_max2(double& a, double& b, double* red, int ltid)
+__device__ __forceinline__ void group_max2(double& a, double& b, double* red, int ltid)
 {
     constexpr int NWAVE = NT / 64;
-    a = wave_max(a);
-    b = wave_max(b);
-    if ((ltid & 63) == 0) {
+    a = wave_max_last(a);
+    b = wave_max_last(b);
+    if ((ltid & 63) == 63) {
         red[ltid >> 6] = a;
         red[NWAVE + (ltid >> 6)] = b;
     }
     __syncthreads();
+    if (ltid != 0) return;
     a = red[0];
     b = red[NWAVE];
 #pragma unroll
@@ -208,23 +247,39 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
     // are read back from there by the face itself, so that they do not stay
     // in registers while the other slots solve their Riemann problems.
     double Sr[SLOTS][3];
-    // each position's own cell (the right-hand cell of its x- and y-face and the
-    // cell of both transverse splits): hu/h, hv/h and sqrt(g*h) once, for a wet
-    // cell, instead of in each of those four places.  Kept for the large tiles
-    // of up to 768 threads only: there one workgroup per CU is set by LDS and
-    // the extra registers are free (up to 168 at three waves per SIMD), while
-    // the other variants' occupancy is set by registers.
-    constexpr bool OWN = TX >= 32 && TY >= 32 && NT <= 768;
-    CellVel C[SLOTS];
+    // Each cell's velocities, sqrt(g h) and reciprocal depth, once: a position
+    // keeps its own cell's (the right-hand cell of its two faces and the cell of
+    // both transverse splits) and hands them to the face on its right and the
+    // one above, whose left-hand cell it is.  (Values of dry cells are garbage
+    // that no one uses.)  LC, at a position: the cell on its left, in the x-face
+    // increments' place, which is free until the limiter, or in the waves'.
+    constexpr bool LF = !FREG && 4 * NPOS <= 6 * G::NF;
+    double* const LC = LF ? F : E;
+    const auto put_cell = [&](double* at, const CellVel& c) {
+        at[0] = c.u;
+        at[NPOS] = c.v;
+        at[2 * NPOS] = c.sg;
+        at[3 * NPOS] = c.y;
+    };
+    const auto get_cell = [&](const double* at) { return CellVel{at[0], at[NPOS], at[2 * NPOS], at[3 * NPOS]}; };
+    const auto cell_of = [&](int k) { return cell_velocity<FAST>(T[k], T[NP2 + k], T[2 * NP2 + k], g); };
+    // the cells left of column 0 and below row 0 belong to no position: lanes of
+    // the last wave, which has the fewest positions, form them
+    const int edge = tid - (NT - 64);
+    static_assert(G::PY <= 64 && PX <= 64, "one wave forms an edge's cells");
+    CellVel C[SLOTS], CL[SLOTS];
 #pragma unroll
-    for (int s = 0; s < SLOTS; s++) {
-        C[s] = CellVel{0.0, 0.0, 0.0, 0.0};
-        if (OWN) {
-            const int k = G::ti(pi[s], pj[s]);
-            const double h = in[s] ? T[k] : 0.0;
-            if (h > drytol) C[s] = cell_velocity<FAST>(h, T[NP2 + k], T[2 * NP2 + k], g);
+    for (int s = 0; s < SLOTS; s++)
+        if (in[s]) {
+            C[s] = cell_of(G::ti(pi[s], pj[s]));
+            if (pi[s] < PX - 1) put_cell(LC + tid + s * NT + 1, C[s]);
         }
-    }
+    if (edge >= 0 && edge < G::PY) put_cell(LC + edge * PX, cell_of(G::ti(-1, edge)));
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < SLOTS; s++)
+        if (in[s]) CL[s] = get_cell(LC + tid + s * NT);
+    if (!LF) __syncthreads();
     double AP[SLOTS][3], AM[SLOTS][3], GA[SLOTS][3], GB[SLOTS][3];
     double FX[FREG ? SLOTS : 1][6];  // FREG: the position's x-face increments (faddm, faddp)
 
@@ -236,8 +291,8 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         double wc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (in[s] && j <= TY + 1) {
             const int kL = G::ti(i - 1, j), kR = G::ti(i, j);
-            rpn2_face<FAST, OWN>(T[kL], T[NP2 + kL], T[2 * NP2 + kL], T[3 * NP2 + kL],
-                                 T[kR], T[NP2 + kR], T[2 * NP2 + kR], T[3 * NP2 + kR], P, sw, wc, C[s]);
+            rpn2_face<FAST>(T[kL], T[NP2 + kL], T[2 * NP2 + kL], T[3 * NP2 + kL],
+                            T[kR], T[NP2 + kR], T[2 * NP2 + kR], T[3 * NP2 + kR], CL[s], C[s], P, sw, wc);
 #pragma unroll
             for (int mw = 0; mw < 3; mw++) smax = vmax<FAST>(smax, fabs(sw[mw]));
         }
@@ -259,15 +314,10 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         const int i = pi[s], j = pj[s];
         const int p = tid + s * NT;
         if (in[s] && i >= 1 && i <= TX + 1 && j <= TY + 1) {
-            double wl[7], wc[7], wr[7];
-#pragma unroll
-            for (int k = 0; k < 7; k++) {
-                wl[k] = E[k * NPOS + p - 1];
-                wc[k] = E[k * NPOS + p];
-                wr[k] = E[k * NPOS + p + 1];
-            }
+            double wc[7], wn[7];
+            load_waves<NPOS>(E + p, 1, Sr[s], wc, wn);
             double fxm[3], fxp[3];
-            face_second_order<0, DEF, FAST>(wc, Sr[s], wl, wr, dtdx, P, fxm, fxp, AM[s], AP[s]);
+            face_second_order<0, DEF, FAST>(wc, Sr[s], wn, dtdx, P, fxm, fxp, AM[s], AP[s]);
             if constexpr (FREG) {
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
@@ -308,21 +358,23 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         for (int k = 0; k < 3; k++) { GA[s][k] = 0.0; GB[s][k] = 0.0; }
         if (transverse && in[s] && i >= 1 && i <= TX && j <= TY + 1) {
             const int kc = G::ti(i, j);
-            const CellVel V = OWN ? C[s] : cell_velocity<FAST>(T[kc], T[NP2 + kc], T[2 * NP2 + kc], g);
-            const Rpt2Cell R = rpt2_setup(T[kc], V.u, V.v, V.sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i, j - 1)],
+            const Rpt2Cell R = rpt2_setup<FAST>(T[kc], C[s].u, C[s].v, C[s].sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i, j - 1)],
                                           T[3 * NP2 + G::ti(i, j + 1)], drytol);
             const double amn[3] = {E[p + 1], E[NPOS + p + 1], E[2 * NPOS + p + 1]};
             cell_transverse<FAST>(R, amn, AP[s], hdx, GA[s], GB[s]);  // GA = G1 (below), GB = G2 (above)
         }
     }
     __syncthreads();
+    // (with the increments, the cell below each position for the y-faces)
 #pragma unroll
     for (int s = 0; s < SLOTS; s++)
         if (in[s]) {
             const int p = tid + s * NT;
 #pragma unroll
             for (int k = 0; k < 3; k++) E[k * NPOS + p] = GB[s][k];
+            if (pj[s] < G::PY - 1) put_cell(E + 3 * NPOS + p + PX, C[s]);
         }
+    if (edge >= 0 && edge < PX) put_cell(E + 3 * NPOS + edge, cell_of(G::ti(edge, -1)));
     __syncthreads();
     // GT(i, J) = GX2(i, J-1) + GX1(i, J): the x-sweep part of gm and gp at y-face (i, J)
     double GT[SLOTS][3];
@@ -337,6 +389,7 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
 #pragma unroll
             for (int k = 0; k < 3; k++) GT[s][k] = 0.0;
         }
+        if (in[s]) CL[s] = get_cell(E + 3 * NPOS + p);
     }
     __syncthreads();
 
@@ -349,9 +402,10 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         if (in[s] && i <= TX + 1) {
             const int kL = G::ti(i, j - 1), kR = G::ti(i, j);
             // direction-local order for y: (h, hv, hu)
-            rpn2_face<FAST, OWN>(T[kL], T[2 * NP2 + kL], T[NP2 + kL], T[3 * NP2 + kL],
-                                 T[kR], T[2 * NP2 + kR], T[NP2 + kR], T[3 * NP2 + kR], P, sw, wc,
-                                 CellVel{C[s].v, C[s].u, C[s].sg, C[s].y});
+            rpn2_face<FAST>(T[kL], T[2 * NP2 + kL], T[NP2 + kL], T[3 * NP2 + kL],
+                            T[kR], T[2 * NP2 + kR], T[NP2 + kR], T[3 * NP2 + kR],
+                            CellVel{CL[s].v, CL[s].u, CL[s].sg, CL[s].y}, CellVel{C[s].v, C[s].u, C[s].sg, C[s].y},
+                            P, sw, wc);
 #pragma unroll
             for (int mw = 0; mw < 3; mw++) smax = vmax<FAST>(smax, fabs(sw[mw]));
         }
@@ -373,14 +427,9 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
 #pragma unroll
         for (int k = 0; k < 3; k++) { GMr[s][k] = 0.0; GPr[s][k] = 0.0; AM[s][k] = 0.0; AP[s][k] = 0.0; }
         if (in[s] && i <= TX + 1 && j >= 1 && j <= TY + 1) {
-            double wl[7], wc[7], wr[7], fm[3], fp[3];
-#pragma unroll
-            for (int k = 0; k < 7; k++) {
-                wl[k] = E[k * NPOS + p - PX];
-                wc[k] = E[k * NPOS + p];
-                wr[k] = E[k * NPOS + p + PX];
-            }
-            face_second_order<1, DEF, FAST>(wc, Sr[s], wl, wr, dtdy, P, fm, fp, AM[s], AP[s]);
+            double wc[7], wn[7], fm[3], fp[3];
+            load_waves<NPOS>(E + p, PX, Sr[s], wc, wn);
+            face_second_order<1, DEF, FAST>(wc, Sr[s], wn, dtdy, P, fm, fp, AM[s], AP[s]);
             // gm = GT + faddm in physical order (h, hu, hv) = local (0, 2, 1)
             GMr[s][0] = GT[s][0] + fm[0];
             GMr[s][1] = GT[s][1] + fm[2];
@@ -410,8 +459,7 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         for (int k = 0; k < 3; k++) { GA[s][k] = 0.0; GB[s][k] = 0.0; }
         if (transverse && in[s] && i <= TX + 1 && j >= 1 && j <= TY) {
             const int kc = G::ti(i, j);
-            const CellVel V = OWN ? C[s] : cell_velocity<FAST>(T[kc], T[NP2 + kc], T[2 * NP2 + kc], g);
-            const Rpt2Cell R = rpt2_setup(T[kc], V.v, V.u, V.sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i - 1, j)],
+            const Rpt2Cell R = rpt2_setup<FAST>(T[kc], C[s].v, C[s].u, C[s].sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i - 1, j)],
                                           T[3 * NP2 + G::ti(i + 1, j)], drytol);
             const double amn[3] = {E[p + PX], E[NPOS + p + PX], E[2 * NPOS + p + PX]};
             cell_transverse<FAST>(R, amn, AP[s], hdy, GA[s], GB[s]);  // GA = left (side 1), GB = right (side 2)
@@ -494,7 +542,7 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
     // non-finite new state makes the CFL number NaN, which the cap keeps)
     cfl = fmaxf64(cfl, dtdy * smax);
     double v = bad ? quiet_nan() : cfl, hmx = hm;
-    block_max2<NT>(v, hmx, red, tid);
+    group_max2<NT>(v, hmx, red, tid);
     if (tid == 0) {
         cfl_res = v;
         hmax_res = hmx;
@@ -547,24 +595,22 @@ __device__ __forceinline__ Params uniform(const Params& p)
 // increments is the one that reads them back) instead of in LDS -- the "LDS
 // split" of a step variant.
 //
-// Hook: called by thread NT-1 (of group 0) right after the tile is in LDS:
-// that thread has no position in the last slot, so its wave has slack in
-// the phases that follow.
+// Hook: called by the last wave (of group 0) right after the tile is in LDS:
+// it has the fewest positions, so it has slack in the phases that follow.
 struct NoHook {
-    __device__ void operator()() const {}
+    __device__ void operator()(int) const {}
 };
 
 template <int MX, int MY, int TX, int TY, int NT, bool PULL, bool DEF, bool FREG = false, typename Hook = NoHook>
-__device__ __forceinline__ void step_patch(double* T, double* E, double* F, double* red, const PatchDesc* dptr, int patch,
+__device__ __forceinline__ void step_patch(double* T, double* E, double* F, double* red, const RegionSrc* regions, int patch,
                            int ox, int oy, const gdouble* q_src, gdouble* q_dst, const gdouble* aux,
-                           double dt, const Params& P, double& cfl_res, double& hmax_res,
+                           double dt, double dtdx, double dtdy, const Params& P, double& cfl_res, double& hmax_res,
                            int ltid, bool valid, const Hook& hook = Hook())
 {
     using G = Geo<TX, TY>;   // tile geometry (LDS)
     using GP = Geo<MX, MY>;  // patch geometry (HBM)
-    constexpr int NXP = G::NXP, NP2 = G::NP2, PX = G::PX, NPOS = G::NPOS;
+    constexpr int NXP = G::NXP, NP2 = G::NP2;
     constexpr int PNP2 = GP::NP2;
-    constexpr int SLOTS = (NPOS + NT - 1) / NT;
     // Opaque copy of the thread index: inside the persistent loop this stops
     // the compiler from hoisting every index computation of the body out of
     // the loop, which would keep them live in registers across iterations.
@@ -574,48 +620,38 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     gdouble* dst = q_dst + (size_t)patch * 3 * PNP2;
     const gdouble* auxp = aux + (size_t)patch * PNP2;
     const double drytol = P.dry_tolerance;
-    const double dtdx = uniform(dt / dptr->dx);
-    const double dtdy = uniform(dt / dptr->dy);
 
     // ---- tile load (+ halo gather) + b4step2 (geoclaw_b4step2_fort.f90:153-156) ----
     // Addresses of every cell this thread loads first, then all loads, then
     // the LDS stores: one memory round trip per tile instead of one per cell
     // group.
     constexpr int LS = (NP2 + NT - 1) / NT;
-    const gdouble* lbase[LS];
-    int lk[LS], lpc[LS];
-    bool lok[LS], lnu[LS], lnv[LS];
+    const gdouble* at[LS];
+    int lpc[LS], neg[LS];
+    bool lok[LS];
 #pragma unroll
     for (int r = 0; r < LS; r++) {
         const int c = tid + r * NT;
         lok[r] = valid && c < NP2;
         const int cc = lok[r] ? c : 0;
         const int fi = ox + cc % NXP - 1, fj = oy + cc / NXP - 1;  // patch Fortran indices
-        const int pc = GP::ti(fi, fj);
-        const gdouble* base = src;
-        int k = pc;
-        bool nu = false, nv = false;
+        lpc[r] = GP::ti(fi, fj);
+        neg[r] = 0;
+        at[r] = src + lpc[r];
         if (PULL) {
-            const bool interior = (fi >= 1 && fi <= MX && fj >= 1 && fj <= MY);
-            int sp = patch, si = fi, sj = fj;
-            if (!interior && ghost_source<MX, MY>(dptr->nbr, patch, fi, fj, sp, si, sj, nu, nv)) {
-                base = q_src + (size_t)sp * 3 * PNP2;
-                k = GP::ti(si, sj);
-            }
+            const int region = (fi < 1 ? 0 : (fi > MX ? 2 : 1)) + (fj < 1 ? 0 : (fj > MY ? 6 : 3));
+            const RegionSrc g = regions[region];
+            at[r] = q_src + (g.off + (fi * g.kx + fj * (g.ky_neg >> 2)));
+            neg[r] = g.ky_neg;
         }
-        lbase[r] = base;
-        lk[r] = k;
-        lpc[r] = pc;
-        lnu[r] = nu;
-        lnv[r] = nv;
     }
     double lh[LS], lhu[LS], lhv[LS], lb[LS];
 #pragma unroll
     for (int r = 0; r < LS; r++) {
         if (lok[r]) {
-            lh[r] = lbase[r][lk[r]];
-            lhu[r] = lbase[r][PNP2 + lk[r]];
-            lhv[r] = lbase[r][2 * PNP2 + lk[r]];
+            lh[r] = at[r][0];
+            lhu[r] = at[r][PNP2];
+            lhv[r] = at[r][2 * PNP2];
             lb[r] = auxp[lpc[r]];
         }
     }
@@ -627,7 +663,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     for (int r = 0; r < LS; r++) {
         if (lok[r]) {
             const int c = tid + r * NT;
-            double h = lh[r], hu = lnu[r] ? -lhu[r] : lhu[r], hv = lnv[r] ? -lhv[r] : lhv[r];
+            double h = lh[r], hu = (neg[r] & 1) ? -lhu[r] : lhu[r], hv = (neg[r] & 2) ? -lhv[r] : lhv[r];
             if (h < drytol) {
                 h = fmaxf64(h, 0.0);
                 hu = 0.0;
@@ -647,9 +683,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
         }
     }
     const int flags = __syncthreads_or(wet);
-    static_assert(NT - 1 + NT * (SLOTS - 1) >= G::NPOS || SLOTS == 1,
-                  "the hook thread must have no position in the last slot");
-    if (threadIdx.x == NT - 1) hook();
+    if (threadIdx.x / 64 == NT / 64 - 1) hook(threadIdx.x % 64);
 
     if (!(flags & 1)) {
         // Every face of the tile is dry on both sides: all fluctuations, waves
@@ -673,10 +707,11 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
         }
         // a non-finite cell (a NaN depth is neither wet nor dry) makes the
         // tile's CFL number NaN, which stops the scenario
+        double cfl = bad ? quiet_nan() : 0.0;
         if (bad) hm = quiet_nan();
-        hm = block_max<NT>(hm, red, tid);
+        group_max2<NT>(cfl, hm, red, tid);
         if (tid == 0) {
-            cfl_res = hm != hm ? quiet_nan() : 0.0;
+            cfl_res = cfl;
             hmax_res = hm;
         }
         return;
@@ -707,15 +742,19 @@ struct Tiling {
 // positive pattern), then counts itself in; the tile that completes the
 // count takes the patch's totals and clears the slots for the next use.
 // Returns true in thread 0 of that last tile, with the totals in cfl / hm.
+// Only atomics touch the slots, and a tile counts itself in once its maxima
+// have returned, which is when they are done for every workgroup: a device
+// fence here, which writes a whole L2 back, took half the time of launches
+// with many tiles (9,216 tiles of 16x16 cells: 650 us, 330 us without).
 __device__ __forceinline__ bool tile_fold(unsigned long long* tcfl, unsigned long long* th, int* tcnt,
                                           int patch, int ntiles, double& cfl, double& hm)
 {
-    if (cfl != 0.0) atomicMax(tcfl + patch, (unsigned long long)__double_as_longlong(cfl));
-    if (hm != 0.0) atomicMax(th + patch, (unsigned long long)__double_as_longlong(hm));
-    __threadfence();
+    unsigned long long old = 0;
+    if (cfl != 0.0) old |= atomicMax(tcfl + patch, (unsigned long long)__double_as_longlong(cfl));
+    if (hm != 0.0) old |= atomicMax(th + patch, (unsigned long long)__double_as_longlong(hm));
+    asm volatile("" : : "v"(old) : "memory");  // wait for both
     const int done = atomicAdd(tcnt + patch, 1);
     if (done != ntiles - 1) return false;
-    __threadfence();
     cfl = __longlong_as_double((long long)atomicExch(tcfl + patch, 0ull));
     hm = __longlong_as_double((long long)atomicExch(th + patch, 0ull));
     atomicExch(tcnt + patch, 0);
@@ -740,8 +779,10 @@ __global__ void __launch_bounds__(NT) k_step(StepArgs a)
     const gdouble* src = (const gdouble*)(a.cur ? a.q1 : a.q0);
     gdouble* dst = (gdouble*)(a.q1 ? (a.cur ? a.q0 : a.q1) : a.q0);
     double cfl = 0.0, hm = 0.0;
-    step_patch<MX, MY, TX, TY, NT, false, DEF, FREG>(T, E, F, red, a.desc + patch, patch, ox, oy, src, dst,
-                                                     (const gdouble*)a.aux, a.dt, a.P, cfl, hm, threadIdx.x, true);
+    const PatchDesc* d = a.desc + patch;
+    step_patch<MX, MY, TX, TY, NT, false, DEF, FREG>(T, E, F, red, nullptr, patch, ox, oy, src, dst, (const gdouble*)a.aux,
+                                                     a.dt, uniform(a.dt / d->dx), uniform(a.dt / d->dy), a.P, cfl, hm,
+                                                     threadIdx.x, true);
     if (threadIdx.x == 0) {
         bool last = true;
         if (TL::NTILES > 1) last = tile_fold(a.tile_cfl, a.tile_h, a.tile_cnt, patch, TL::NTILES, cfl, hm);
@@ -753,36 +794,39 @@ __global__ void __launch_bounds__(NT) k_step(StepArgs a)
     }
 }
 
-// What an active item needs before its tile can be loaded: the patch, its
-// descriptor and its scenario's buffer, dt and Manning n.  Reading them is a
+// What an active item needs before its tile can be loaded: the patch, where
+// its halo lies, its scenario's buffer, dt and Manning n.  Reading them is a
 // chain of dependent memory accesses (list -> descriptor -> control record),
 // so the item before fetches them for its successor (ItemPrefetch) and the
 // item starts with them in LDS.
 struct ItemHead {
-    PatchDesc d;
-    int patch, cur;
-    double dt, manning;
+    RegionSrc region[REGIONS];
+    double dt, dtdx, dtdy, manning;
+    int patch, scen, cur, pad;
 };
 
-__device__ __forceinline__ void load_head(const BatchArgs& a, int patch, ItemHead* h)
+// By one wave.
+__device__ __forceinline__ void fill_head(const BatchArgs& a, int patch, ItemHead* h, int lane)
 {
-    // the descriptor as 8-byte words, in registers (a struct copy would go
-    // through the private stack)
-    static_assert(sizeof(PatchDesc) % 8 == 0 && offsetof(PatchDesc, scen) % 8 == 0, "PatchDesc layout");
-    constexpr int W = sizeof(PatchDesc) / 8;
-    const long long* s = reinterpret_cast<const long long*>(a.desc + patch);
-    long long w[W];
-#pragma unroll
-    for (int k = 0; k < W; k++) w[k] = s[k];
-    long long* d = reinterpret_cast<long long*>(&h->d);
-#pragma unroll
-    for (int k = 0; k < W; k++) d[k] = w[k];
-    const int scen = (int)(unsigned)(w[offsetof(PatchDesc, scen) / 8] & 0xffffffffll);
-    const ScenCtrl& c = a.ctrl[scen];
-    h->patch = patch;
-    h->cur = c.cur;
-    h->dt = c.dt;
-    h->manning = c.manning_n;
+    const PatchDesc* d = a.desc + patch;
+    const int scen = d->scen;
+    const ScenCtrl* c = a.ctrl + scen;
+    const double dt = c->dt;
+    // (as 8-byte words, one per lane)
+    constexpr int W = sizeof(h->region) / 8;
+    static_assert(W <= 64, "one word per lane");
+    if (lane < W)
+        reinterpret_cast<long long*>(h->region)[lane] =
+            reinterpret_cast<const long long*>(a.regions + (size_t)patch * REGIONS)[lane];
+    if (lane == 0) {
+        h->dt = dt;
+        h->dtdx = dt / d->dx;
+        h->dtdy = dt / d->dy;
+        h->manning = c->manning_n;
+        h->patch = patch;
+        h->scen = scen;
+        h->cur = c->cur;
+    }
 }
 
 // The item after the workgroup's first ones: the next of its queue (items x,
@@ -795,23 +839,25 @@ __device__ __forceinline__ int next_item(int* counters, int limit)
     return grid + x + nq * atomicAdd(&counters[CURSOR_LINE * (1 + x)], 1);
 }
 
-// Run by one thread of the current active item: takes the next item from
-// the queue, publishes it, and when it is active fills its ItemHeads (one
-// per patch of the item: entries next*NPP .. of the active tile list).
+// Run by one wave of the current active item: takes the next item from the
+// queue, publishes it, and when it is active fills its ItemHeads (one per
+// patch of the item: entries next*NPP .. of the active tile list).
 template <int NTILES, int NPP>
 struct ItemPrefetch {
     const BatchArgs* pa;
     int* next_slot;
     ItemHead* next_head;
     int nwet, limit;
-    __device__ void operator()() const
+    __device__ void operator()(int lane) const
     {
-        const int next = next_item(pa->counters, limit);
-        *next_slot = next;
+        int next = 0;
+        if (lane == 0) next = next_item(pa->counters, limit);
+        next = uniform(next);
+        if (lane == 0) *next_slot = next;
 #pragma unroll
         for (int g = 0; g < NPP; g++) {
             const int e = next * NPP + g;
-            if (e < nwet) load_head(*pa, pa->list_wet[e / NTILES], next_head + g);
+            if (e < nwet) fill_head(*pa, uniform(pa->list_wet[e / NTILES]), next_head + g, lane);
         }
     }
 };
@@ -830,7 +876,7 @@ struct ItemPrefetch {
 // idx*NPP .. idx*NPP+NPP-1 of the active list, one per group of NT threads.
 template <int MX, int MY, int TX, int TY, int NT, int NPP, bool FREG, bool DEF>
 __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const ItemHead* head, ItemHead* next_head,
-                                         int* next_slot, int nwet, int limit)
+                                         int* next_slot, int nwet, int limit, const Params& params)
 {
     using G = Geo<TX, TY>;
     using TL = Tiling<MX, MY, TX, TY>;
@@ -850,20 +896,20 @@ __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const Ite
     const int patch = uniform(hd->patch);
     int ox, oy;
     TL::origin(uniform(entry % TL::NTILES), ox, oy);
-    const int scen = uniform(hd->d.scen);
+    const int scen = uniform(hd->scen);
     const int cur = uniform(hd->cur);
-    const double dt = uniform(hd->dt);
     const gdouble* src = (const gdouble*)(cur ? a.q1 : a.q0);
     gdouble* dst = (gdouble*)(cur ? a.q0 : a.q1);
-    Params P = uniform(a.P);
+    Params P = uniform(params);
     P.manning_n = uniform(hd->manning);
     if (ltid == 0 && valid) a.dry_age[patch] = 0;
     double cfl = 0.0, hm = 0.0;
     const ItemPrefetch<TL::NTILES, NPP> pf{pa, next_slot, next_head, nwet, limit};
     step_patch<MX, MY, TX, TY, NT, true, DEF, FREG>(T + grp * 4 * G::NP2, E + grp * 7 * G::NPOS,
                                                     F + (FREG ? 0 : grp * 6 * G::NF), red + grp * 2 * (NT / 64),
-                                                    &hd->d, patch, ox, oy, src, dst, (const gdouble*)a.aux, dt, P, cfl, hm, ltid,
-                                                    valid, pf);
+                                                    hd->region, patch, ox, oy, src, dst, (const gdouble*)a.aux,
+                                                    uniform(hd->dt), uniform(hd->dtdx), uniform(hd->dtdy), P, cfl, hm,
+                                                    ltid, valid, pf);
     if (ltid == 0 && valid) {
         bool last = true;
         if (TL::NTILES > 1) last = tile_fold(a.tile_cfl, a.tile_h, a.tile_cnt, patch, TL::NTILES, cfl, hm);
@@ -874,14 +920,15 @@ __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const Ite
             // doubles, but -0.0 (which the CFL maximum can return for a patch
             // with no waves) sorts above them all: zeros are left out (the
             // scenario's maximum starts at +0.0).  NaN still propagates.
-            // Most patches do not raise it: a look first leaves the one address
-            // that all of a scenario's patches share mostly unwritten.
-            const unsigned long long bits = (unsigned long long)__double_as_longlong(cfl);
-            if (cfl != 0.0 && bits > __hip_atomic_load(a.cflbits + scen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                atomicMax(a.cflbits + scen, bits);
+            // Each queue has a maximum of its own (the workgroups of one XCD),
+            // and nothing waits for the atomic.
+            if (cfl != 0.0)
+                atomicMax(a.cflbits + (size_t)(blockIdx.x % QUEUES) * a.capacity + scen,
+                          (unsigned long long)__double_as_longlong(cfl));
         }
     }
-    __syncthreads();
+    // No barrier: the next item's tile goes to LDS after every thread has read
+    // this one (group_max2's barrier), and its heads are the other pair.
 }
 
 // Dry patches per work item of the unified kernel: about eight cells per
@@ -997,7 +1044,11 @@ __device__ __forceinline__ void dry_item(const BatchArgs* pa, int k, int next, i
 // (wet_item), then the dry patches in items of dry_per_item (dry_item), from
 // the item queues.  The streaming dry items fill the tail that the
 // compute-bound active items leave when the list runs out.
-// step_waves: the waves per SIMD that the registers must allow.  __WAVES__
+// step_waves: the waves per SIMD that the registers must allow.  The kernels
+// whose threads own one position each need 136-143 VGPRs when left to the
+// scheduler and 117-126 without a spill when held to four waves (8x8, 16,384
+// patches: 170-213 us, against 171-220 us before; three waves 171-220 us); 32x32
+// tiles are alone on a CU by their LDS, and the two-position kernels spill.
 template <int TX, int TY, int NT>
 constexpr int step_waves()
 {
@@ -1012,16 +1063,20 @@ __global__ void __launch_bounds__(NT * NPP, (step_waves<TX, TY, NT>())) k_all(co
     constexpr int DPI = dry_per_item<MX, MY, NB>();
     __shared__ int item[2];
     __shared__ ItemHead head[2][NPP];
+    __shared__ Params params;
     __shared__ int unsteady[DPI];  // per dry patch of an item: a cell at dry_tolerance
     const int nwet = pa->counters[CNT_WET] * TL::NTILES;  // active tiles
     const int witems = (nwet + NPP - 1) / NPP;             // active items
     const int limit = witems + (pa->counters[CNT_DRY] + DPI - 1) / DPI;
     if ((int)blockIdx.x >= limit) return;
-    if (threadIdx.x == 0) {
-        item[0] = (int)blockIdx.x;
+    if (threadIdx.x < 64) {
         for (int g = 0; g < NPP; g++)
             if ((int)blockIdx.x * NPP + g < nwet)
-                load_head(*pa, pa->list_wet[((int)blockIdx.x * NPP + g) / TL::NTILES], &head[0][g]);
+                fill_head(*pa, pa->list_wet[((int)blockIdx.x * NPP + g) / TL::NTILES], &head[0][g], threadIdx.x);
+    }
+    if (threadIdx.x == NB - 1) {
+        item[0] = (int)blockIdx.x;
+        params = pa->P;
     }
     if (threadIdx.x < DPI) unsteady[threadIdx.x] = 0;
     __syncthreads();
@@ -1032,13 +1087,40 @@ __global__ void __launch_bounds__(NT * NPP, (step_waves<TX, TY, NT>())) k_all(co
             // active items come first in the cursor's order, so an active
             // item's successor's heads are always prefetched by an active item
             wet_item<MX, MY, TX, TY, NT, NPP, FREG, DEF>(pa, idx, head[it & 1], head[(it + 1) & 1],
-                                                         &item[(it + 1) & 1], nwet, limit);
+                                                         &item[(it + 1) & 1], nwet, limit, params);
         } else {
             int next = 0;
             if (threadIdx.x == 0) next = next_item(pa->counters, limit);
             dry_item<MX, MY, NB>(pa, idx - witems, next, &item[(it + 1) & 1], unsteady);
         }
     }
+}
+
+// The region tables of slots [first, first + n), whenever they are described.
+template <int MX, int MY>
+__device__ __forceinline__ RegionSrc region_source(const int* nbr, int patch, int region)
+{
+    using GP = Geo<MX, MY>;
+    const int rx = region % 3, ry = region / 3;
+    // two cells of the region one apart in both directions
+    const int fi0 = rx == 0 ? 0 : (rx == 2 ? MX + 1 : 1), fj0 = ry == 0 ? 0 : (ry == 2 ? MY + 1 : 1);
+    const int di = rx == 0 ? -1 : 1, dj = ry == 0 ? -1 : 1;
+    int sp = patch, si = fi0, sj = fj0, sp1, si1 = fi0 + di, sj1 = fj0 + dj;
+    bool nu = false, nv = false, nu1, nv1;
+    if (region != 4 && ghost_source<MX, MY>(nbr, patch, fi0, fj0, sp, si, sj, nu, nv))
+        ghost_source<MX, MY>(nbr, patch, fi0 + di, fj0 + dj, sp1, si1, sj1, nu1, nv1);
+    const int kx = (si1 - si) * di, ky = (sj1 - sj) * dj * GP::NXP;
+    return RegionSrc{(long long)sp * 3 * GP::NP2 + GP::ti(si, sj) - kx * fi0 - ky * fj0, kx,
+                     ky * 4 + (nu ? 1 : 0) + (nv ? 2 : 0)};
+}
+
+template <int MX, int MY>
+__global__ void __launch_bounds__(256) k_regions(const PatchDesc* desc, RegionSrc* regions, int first, int n)
+{
+    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (e >= n * REGIONS) return;
+    const int patch = first + e / REGIONS;
+    regions[(size_t)first * REGIONS + e] = region_source<MX, MY>(desc[patch].nbr, patch, e % REGIONS);
 }
 
 // ---------------------------------------------------------------------------
@@ -1447,8 +1529,12 @@ __global__ void __launch_bounds__(64) k_batch_control(const BatchArgs* pa)
     if (s >= a.nscen) return;
     ScenCtrl* c = a.ctrl + s;
     if (!c->active) return;
-    const double m = __longlong_as_double((long long)a.cflbits[s]);
-    a.cflbits[s] = 0ull;
+    double m = 0.0;
+#pragma unroll
+    for (int q = 0; q < QUEUES; q++)
+        m = max_nan(m, __longlong_as_double((long long)a.cflbits[(size_t)q * a.capacity + s]));
+#pragma unroll
+    for (int q = 0; q < QUEUES; q++) a.cflbits[(size_t)q * a.capacity + s] = 0ull;
     control_step(c, m);
 }
 
@@ -2237,6 +2323,16 @@ hipError_t launch_batch_control(const BatchArgs* da, int scenarios, hipStream_t 
     case 64064: CALL(64, 64); break;               \
     default: return hipErrorInvalidValue;          \
     }
+
+hipError_t launch_regions(int mx, int my, const PatchDesc* desc, RegionSrc* regions, int first, int n, hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    const int grid = (int)(((long long)n * REGIONS + 255) / 256);
+#define GF_RG(M, N) k_regions<M, N><<<grid, 256, 0, st>>>(desc, regions, first, n)
+    GF_SIZES(GF_RG)
+#undef GF_RG
+    return hipGetLastError();
+}
 
 hipError_t launch_average2coarse(int mx, int my, const RegridArgs& a, hipStream_t st)
 {
