@@ -221,10 +221,10 @@ using gint = __attribute__((address_space(1))) int;
 // The step of one tile in LDS (T: h, hu, hv, b after b4step2, at least one
 // cell wet), by a group of NT threads; arguments as in step_patch.  FAST: every
 // cell and parameter lies in the range of gf_exact.h.
-template <int MX, int MY, int TX, int TY, int NT, bool DEF, bool FREG, bool FAST>
+template <int MX, int MY, int TX, int TY, int NT, bool DEF, bool FREG, bool FAST, typename Ahead>
 __device__ __forceinline__ void step_tile(const double* T, double* E, double* F, double* red, int ox, int oy,
                                           gdouble* dst, double dtdx, double dtdy, double dt, const Params& P,
-                                          double& cfl_res, double& hmax_res, int tid, bool valid)
+                                          double& cfl_res, double& hmax_res, int tid, bool valid, const Ahead& ahead)
 {
     using G = Geo<TX, TY>;   // tile geometry (LDS)
     using GP = Geo<MX, MY>;  // patch geometry (HBM)
@@ -449,6 +449,8 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         }
     __syncthreads();
 
+    ahead();
+
     // ================= y-transverse (cell-centred rpt2) =================
     const double hdy = 0.5 * dtdy;
 #pragma unroll
@@ -559,6 +561,13 @@ __device__ __forceinline__ double uniform(double v)
     const unsigned lo = (unsigned)uniform((int)b), hi = (unsigned)uniform((int)(b >> 32));
     return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
 }
+template <typename T>
+__device__ __forceinline__ T* uniform(T* p)
+{
+    const unsigned long long b = (unsigned long long)p;
+    const unsigned lo = (unsigned)uniform((int)b), hi = (unsigned)uniform((int)(b >> 32));
+    return (T*)((unsigned long long)hi << 32 | lo);
+}
 __device__ __forceinline__ Params uniform(const Params& p)
 {
     constexpr int W = sizeof(Params) / sizeof(int);
@@ -601,11 +610,59 @@ struct NoHook {
     __device__ void operator()(int) const {}
 };
 
-template <int MX, int MY, int TX, int TY, int NT, bool PULL, bool DEF, bool FREG = false, typename Hook = NoHook>
+// What a thread loads of a tile: up to LS cells of it and its halo.
+template <int LS>
+struct TileCells {
+    double h[LS], hu[LS], hv[LS], b[LS];
+};
+
+// Region of the patch (or its halo) that cell (fi, fj) lies in.
+template <int MX, int MY>
+__device__ __forceinline__ int region_of(int fi, int fj)
+{
+    return (fi < 1 ? 0 : (fi > MX ? 2 : 1)) + (fj < 1 ? 0 : (fj > MY ? 6 : 3));
+}
+
+// Issues the loads of a thread's cells of the tile at (ox, oy) of a patch and
+// its halo (PULL: by the slot's regions in q_src; otherwise from the patch's
+// own ghost cells): every address first, then every load, one memory round
+// trip per tile.
+template <int MX, int MY, int TX, int TY, int NT, bool PULL, int LS>
+__device__ __forceinline__ void load_tile(const RegionSrc* regions, int patch, int ox, int oy, const gdouble* q_src,
+                                          const gdouble* aux, int tid, TileCells<LS>& cells)
+{
+    using G = Geo<TX, TY>;
+    using GP = Geo<MX, MY>;
+    const gdouble* src = q_src + (size_t)patch * 3 * GP::NP2;
+    const gdouble* auxp = aux + (size_t)patch * GP::NP2;
+    const gdouble* at[LS];
+    int own[LS];
+#pragma unroll
+    for (int r = 0; r < LS; r++) {
+        const int c = tid + r * NT < G::NP2 ? tid + r * NT : 0;
+        const int fi = ox + c % G::NXP - 1, fj = oy + c / G::NXP - 1;  // patch Fortran indices
+        own[r] = GP::ti(fi, fj);
+        at[r] = src + own[r];
+        if (PULL) {
+            const RegionSrc g = regions[region_of<MX, MY>(fi, fj)];
+            at[r] = q_src + (g.off + (fi * g.kx + fj * (g.ky_neg >> 2)));
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < LS; r++)
+        if (tid + r * NT < G::NP2) {
+            cells.h[r] = at[r][0];
+            cells.hu[r] = at[r][GP::NP2];
+            cells.hv[r] = at[r][2 * GP::NP2];
+            cells.b[r] = auxp[own[r]];
+        }
+}
+
+template <int MX, int MY, int TX, int TY, int NT, bool PULL, bool DEF, bool FREG, int LS, typename Hook, typename Ahead>
 __device__ __forceinline__ void step_patch(double* T, double* E, double* F, double* red, const RegionSrc* regions, int patch,
                            int ox, int oy, const gdouble* q_src, gdouble* q_dst, const gdouble* aux,
                            double dt, double dtdx, double dtdy, const Params& P, double& cfl_res, double& hmax_res,
-                           int ltid, bool valid, const Hook& hook = Hook())
+                           int ltid, bool valid, TileCells<LS>& cells, bool loaded, const Hook& hook, const Ahead& ahead)
 {
     using G = Geo<TX, TY>;   // tile geometry (LDS)
     using GP = Geo<MX, MY>;  // patch geometry (HBM)
@@ -616,54 +673,26 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     // the loop, which would keep them live in registers across iterations.
     int tid = ltid;
     asm volatile("" : "+v"(tid));
-    const gdouble* src = q_src + (size_t)patch * 3 * PNP2;
     gdouble* dst = q_dst + (size_t)patch * 3 * PNP2;
-    const gdouble* auxp = aux + (size_t)patch * PNP2;
     const double drytol = P.dry_tolerance;
 
     // ---- tile load (+ halo gather) + b4step2 (geoclaw_b4step2_fort.f90:153-156) ----
-    // Addresses of every cell this thread loads first, then all loads, then
-    // the LDS stores: one memory round trip per tile instead of one per cell
-    // group.
-    constexpr int LS = (NP2 + NT - 1) / NT;
-    const gdouble* at[LS];
-    int lpc[LS], neg[LS];
-    bool lok[LS];
-#pragma unroll
-    for (int r = 0; r < LS; r++) {
-        const int c = tid + r * NT;
-        lok[r] = valid && c < NP2;
-        const int cc = lok[r] ? c : 0;
-        const int fi = ox + cc % NXP - 1, fj = oy + cc / NXP - 1;  // patch Fortran indices
-        lpc[r] = GP::ti(fi, fj);
-        neg[r] = 0;
-        at[r] = src + lpc[r];
-        if (PULL) {
-            const int region = (fi < 1 ? 0 : (fi > MX ? 2 : 1)) + (fj < 1 ? 0 : (fj > MY ? 6 : 3));
-            const RegionSrc g = regions[region];
-            at[r] = q_src + (g.off + (fi * g.kx + fj * (g.ky_neg >> 2)));
-            neg[r] = g.ky_neg;
-        }
-    }
-    double lh[LS], lhu[LS], lhv[LS], lb[LS];
-#pragma unroll
-    for (int r = 0; r < LS; r++) {
-        if (lok[r]) {
-            lh[r] = at[r][0];
-            lhu[r] = at[r][PNP2];
-            lhv[r] = at[r][2 * PNP2];
-            lb[r] = auxp[lpc[r]];
-        }
-    }
+    static_assert(LS == (NP2 + NT - 1) / NT, "cells per thread");
+    if (!loaded && valid) load_tile<MX, MY, TX, TY, NT, PULL>(regions, patch, ox, oy, q_src, aux, tid, cells);
     // bit 0: a wet cell; bit 1: a cell, a parameter or a step size outside the
     // range of the fast quotients (gf_exact.h)
     int wet = 0;
     if (!(P.fast && dtdx >= 0x1p-100 && dtdx <= 0x1p100 && dtdy >= 0x1p-100 && dtdy <= 0x1p100)) wet = 2;
 #pragma unroll
     for (int r = 0; r < LS; r++) {
-        if (lok[r]) {
-            const int c = tid + r * NT;
-            double h = lh[r], hu = (neg[r] & 1) ? -lhu[r] : lhu[r], hv = (neg[r] & 2) ? -lhv[r] : lhv[r];
+        const int c = tid + r * NT;
+        if (valid && c < NP2) {
+            double h = cells.h[r], hu = cells.hu[r], hv = cells.hv[r];
+            if (PULL) {
+                const int neg = regions[region_of<MX, MY>(ox + c % NXP - 1, oy + c / NXP - 1)].ky_neg;
+                hu = (neg & 1) ? -hu : hu;
+                hv = (neg & 2) ? -hv : hv;
+            }
             if (h < drytol) {
                 h = fmaxf64(h, 0.0);
                 hu = 0.0;
@@ -672,10 +701,9 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
             T[c] = h;
             T[NP2 + c] = hu;
             T[2 * NP2 + c] = hv;
-            T[3 * NP2 + c] = lb[r];
-            wet |= (h > drytol) | (step_cell_in_range(h, hu, hv, lb[r]) ? 0 : 2);
-        } else if (!valid && tid + r * NT < NP2) {
-            const int c = tid + r * NT;  // a group without a patch: a dry zero tile
+            T[3 * NP2 + c] = cells.b[r];
+            wet |= (h > drytol) | (step_cell_in_range(h, hu, hv, cells.b[r]) ? 0 : 2);
+        } else if (!valid && c < NP2) {  // a group without a patch: a dry zero tile
             T[c] = 0.0;
             T[NP2 + c] = 0.0;
             T[2 * NP2 + c] = 0.0;
@@ -718,9 +746,9 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
     }
 
     if (flags & 2)
-        step_tile<MX, MY, TX, TY, NT, DEF, FREG, false>(T, E, F, red, ox, oy, dst, dtdx, dtdy, dt, P, cfl_res, hmax_res, tid, valid);
+        step_tile<MX, MY, TX, TY, NT, DEF, FREG, false>(T, E, F, red, ox, oy, dst, dtdx, dtdy, dt, P, cfl_res, hmax_res, tid, valid, ahead);
     else
-        step_tile<MX, MY, TX, TY, NT, DEF, FREG, true>(T, E, F, red, ox, oy, dst, dtdx, dtdy, dt, P, cfl_res, hmax_res, tid, valid);
+        step_tile<MX, MY, TX, TY, NT, DEF, FREG, true>(T, E, F, red, ox, oy, dst, dtdx, dtdy, dt, P, cfl_res, hmax_res, tid, valid, ahead);
 }
 
 // Tile decomposition of an MX x MY patch into TX x TY tiles.
@@ -780,9 +808,10 @@ __global__ void __launch_bounds__(NT) k_step(StepArgs a)
     gdouble* dst = (gdouble*)(a.q1 ? (a.cur ? a.q0 : a.q1) : a.q0);
     double cfl = 0.0, hm = 0.0;
     const PatchDesc* d = a.desc + patch;
+    TileCells<(G::NP2 + NT - 1) / NT> cells;
     step_patch<MX, MY, TX, TY, NT, false, DEF, FREG>(T, E, F, red, nullptr, patch, ox, oy, src, dst, (const gdouble*)a.aux,
                                                      a.dt, uniform(a.dt / d->dx), uniform(a.dt / d->dy), a.P, cfl, hm,
-                                                     threadIdx.x, true);
+                                                     threadIdx.x, true, cells, false, NoHook(), [] {});
     if (threadIdx.x == 0) {
         bool last = true;
         if (TL::NTILES > 1) last = tile_fold(a.tile_cfl, a.tile_h, a.tile_cnt, patch, TL::NTILES, cfl, hm);
@@ -874,9 +903,20 @@ struct ItemPrefetch {
 //
 // NPP patches per workgroup (untiled variants): the item is entries
 // idx*NPP .. idx*NPP+NPP-1 of the active list, one per group of NT threads.
-template <int MX, int MY, int TX, int TY, int NT, int NPP, bool FREG, bool DEF>
+//
+// tile_ahead: the kernel loads the next item's tile into registers while this
+// one takes its last steps (cells, loaded).  One 32x32 tile fills a CU's LDS,
+// so nothing else hides the 6,000 cycles of its loads (of 55,000); the smaller
+// tiles share their CU with others and need the registers.
+template <int TX, int TY, int NT>
+constexpr bool tile_ahead()
+{
+    return TX >= 32 && TY >= 32 && NT <= 768;
+}
+
+template <int MX, int MY, int TX, int TY, int NT, int NPP, bool FREG, bool DEF, int LS>
 __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const ItemHead* head, ItemHead* next_head,
-                                         int* next_slot, int nwet, int limit, const Params& params)
+                                         int* next_slot, int nwet, int limit, TileCells<LS>& cells, bool& loaded)
 {
     using G = Geo<TX, TY>;
     using TL = Tiling<MX, MY, TX, TY>;
@@ -898,24 +938,44 @@ __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const Ite
     TL::origin(uniform(entry % TL::NTILES), ox, oy);
     const int scen = uniform(hd->scen);
     const int cur = uniform(hd->cur);
-    const gdouble* src = (const gdouble*)(cur ? a.q1 : a.q0);
-    gdouble* dst = (gdouble*)(cur ? a.q0 : a.q1);
-    Params P = uniform(params);
+    double* const q0 = uniform(a.q0);
+    double* const q1 = uniform(a.q1);
+    const gdouble* aux = (const gdouble*)uniform(a.aux);
+    const gdouble* src = (const gdouble*)(cur ? q1 : q0);
+    gdouble* dst = (gdouble*)(cur ? q0 : q1);
+    Params P = uniform(a.P);
     P.manning_n = uniform(hd->manning);
-    if (ltid == 0 && valid) a.dry_age[patch] = 0;
+    if (ltid == 0 && valid) ((gint*)a.dry_age)[patch] = 0;
     double cfl = 0.0, hm = 0.0;
     const ItemPrefetch<TL::NTILES, NPP> pf{pa, next_slot, next_head, nwet, limit};
+    constexpr bool AHEAD = tile_ahead<TX, TY, NT>();
+    TileCells<LS> fresh;
+    const bool have = AHEAD && loaded;
+    loaded = false;
+    const auto ahead = [&] {
+        if constexpr (AHEAD) {
+            const int next = uniform(*next_slot);
+            if (next >= nwet) return;
+            int nx, ny;
+            TL::origin(next % TL::NTILES, nx, ny);
+            int t = ltid;
+            asm volatile("" : "+v"(t));
+            load_tile<MX, MY, TX, TY, NT, true>(next_head->region, uniform(next_head->patch), nx, ny,
+                                                (const gdouble*)(uniform(next_head->cur) ? q1 : q0), aux, t, cells);
+            loaded = true;
+        }
+    };
     step_patch<MX, MY, TX, TY, NT, true, DEF, FREG>(T + grp * 4 * G::NP2, E + grp * 7 * G::NPOS,
                                                     F + (FREG ? 0 : grp * 6 * G::NF), red + grp * 2 * (NT / 64),
-                                                    hd->region, patch, ox, oy, src, dst, (const gdouble*)a.aux,
+                                                    hd->region, patch, ox, oy, src, dst, aux,
                                                     uniform(hd->dt), uniform(hd->dtdx), uniform(hd->dtdy), P, cfl, hm,
-                                                    ltid, valid, pf);
+                                                    ltid, valid, AHEAD ? cells : fresh, have, pf, ahead);
     if (ltid == 0 && valid) {
         bool last = true;
         if (TL::NTILES > 1) last = tile_fold(a.tile_cfl, a.tile_h, a.tile_cnt, patch, TL::NTILES, cfl, hm);
         if (last) {
             if (cfl > 1000.0) cfl = 0.0;  // MAXCFL_CAP per patch (fc2d_cpucuda.cpp:392)
-            a.hmax[(size_t)(cur ^ 1) * a.capacity + patch] = hm;
+            ((gdouble*)a.hmax)[(size_t)(cur ^ 1) * a.capacity + patch] = hm;
             // The unsigned order of bit patterns is the order of non-negative
             // doubles, but -0.0 (which the CFL maximum can return for a patch
             // with no waves) sorts above them all: zeros are left out (the
@@ -1063,21 +1123,27 @@ __global__ void __launch_bounds__(NT * NPP, (step_waves<TX, TY, NT>())) k_all(co
     constexpr int DPI = dry_per_item<MX, MY, NB>();
     __shared__ int item[2];
     __shared__ ItemHead head[2][NPP];
-    __shared__ Params params;
+    // the arguments, read once: an item's reads of them from memory were a round
+    // trip at its start
+    __shared__ BatchArgs args;
     __shared__ int unsteady[DPI];  // per dry patch of an item: a cell at dry_tolerance
     const int nwet = pa->counters[CNT_WET] * TL::NTILES;  // active tiles
     const int witems = (nwet + NPP - 1) / NPP;             // active items
     const int limit = witems + (pa->counters[CNT_DRY] + DPI - 1) / DPI;
+    TileCells<(Geo<TX, TY>::NP2 + NT - 1) / NT> cells;  // of the item, when loaded ahead
+    bool loaded = false;
     if ((int)blockIdx.x >= limit) return;
     if (threadIdx.x < 64) {
         for (int g = 0; g < NPP; g++)
             if ((int)blockIdx.x * NPP + g < nwet)
                 fill_head(*pa, pa->list_wet[((int)blockIdx.x * NPP + g) / TL::NTILES], &head[0][g], threadIdx.x);
     }
-    if (threadIdx.x == NB - 1) {
-        item[0] = (int)blockIdx.x;
-        params = pa->P;
-    }
+    if (threadIdx.x == NB - 1) item[0] = (int)blockIdx.x;
+    constexpr int AW = sizeof(BatchArgs) / 8;
+    static_assert(AW <= 64 && sizeof(BatchArgs) % 8 == 0, "one word per lane of the last wave");
+    if ((int)threadIdx.x - (NB - 64) >= 0 && (int)threadIdx.x - (NB - 64) < AW)
+        reinterpret_cast<long long*>(&args)[threadIdx.x - (NB - 64)] =
+            reinterpret_cast<const long long*>(pa)[threadIdx.x - (NB - 64)];
     if (threadIdx.x < DPI) unsteady[threadIdx.x] = 0;
     __syncthreads();
     for (int it = 0;; it++) {
@@ -1086,12 +1152,12 @@ __global__ void __launch_bounds__(NT * NPP, (step_waves<TX, TY, NT>())) k_all(co
         if (idx < witems) {
             // active items come first in the cursor's order, so an active
             // item's successor's heads are always prefetched by an active item
-            wet_item<MX, MY, TX, TY, NT, NPP, FREG, DEF>(pa, idx, head[it & 1], head[(it + 1) & 1],
-                                                         &item[(it + 1) & 1], nwet, limit, params);
+            wet_item<MX, MY, TX, TY, NT, NPP, FREG, DEF>(&args, idx, head[it & 1], head[(it + 1) & 1],
+                                                         &item[(it + 1) & 1], nwet, limit, cells, loaded);
         } else {
             int next = 0;
-            if (threadIdx.x == 0) next = next_item(pa->counters, limit);
-            dry_item<MX, MY, NB>(pa, idx - witems, next, &item[(it + 1) & 1], unsteady);
+            if (threadIdx.x == 0) next = next_item(args.counters, limit);
+            dry_item<MX, MY, NB>(&args, idx - witems, next, &item[(it + 1) & 1], unsteady);
         }
     }
 }
