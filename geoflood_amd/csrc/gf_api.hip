@@ -253,8 +253,8 @@ struct gf_pool {
     unsigned long long* tile_h = nullptr;
     int* tile_cnt = nullptr;
     int* dry_age = nullptr;                // [capacity] steady dry patches (gf::DRY_STEADY)
-    int variant = 0;                       // step variant (tile shape, threads); see gf_pool_autotune
-    int wet_grid = 0;                      // workgroups of the persistent step kernel (0: not computed)
+    int variant = -1;                      // step variant chosen by the caller or the autotuner (-1: default_variant)
+    int graph_variant = -1;                // variant of the captured graph
     int* inflow_list = nullptr;            // [capacity] patches with a hydrograph side
     int* inflow_n = nullptr;               // [1] entries of inflow_list
     bool has_inflow = false;               // inflow_list is not empty (the graph launches k_inflow)
@@ -1013,6 +1013,12 @@ try {
     return GF_OK;
 } GF_CATCH_STATUS
 
+// The step variant of a launch over n patches.
+static int step_variant(const gf_pool* p, int n, bool whole = false)
+{
+    return p->variant >= 0 ? p->variant : gf::default_variant(p->mx, p->my, n, g.num_cu, whole);
+}
+
 static int pool_step_impl(gf_pool* p, int first, int n, int src, int dst, double dt, double* cfl,
                           double* maxcfl, bool plain)
 {
@@ -1020,17 +1026,18 @@ static int pool_step_impl(gf_pool* p, int first, int n, int src, int dst, double
     if (first < 0 || n < 0 || first + n > p->n) return fail(GF_EINVAL, "patches [%d,%d) outside [0,%d)", first, first + n, p->n);
     if ((src != 0 && src != 1) || (dst != 0 && dst != 1)) return fail(GF_EINVAL, "buffers must be 0 or 1");
     if (!(dt > 0.0)) return fail(GF_EINVAL, "dt must be > 0");
+    const int variant = step_variant(p, plain ? 1 : n, src == dst);
     if (src == dst) {
         // A tiled variant steps a patch with several workgroups, each reading
         // its halo from the neighbouring tiles' cells, which the others
         // overwrite in place: only one workgroup per patch may step in place.
         gf::StepVariant v;
-        if (!gf::get_variant(p->mx, p->my, p->variant, &v)) return fail(GF_ESTATE, "no step variant %d", p->variant);
+        if (!gf::get_variant(p->mx, p->my, variant, &v)) return fail(GF_ESTATE, "no step variant %d", variant);
         if (v.tx != p->mx || v.ty != p->my)
             return fail(GF_EUNSUPPORTED,
                         "an in-place step (src == dst) needs a step variant with one tile per patch; variant %d "
                         "splits %dx%d patches into %dx%d tiles (step into the other buffer instead)",
-                        p->variant, p->mx, p->my, v.tx, v.ty);
+                        variant, p->mx, p->my, v.tx, v.ty);
     }
     double* q0 = (src == dst) ? p->q[src] : p->q[0];
     double* q1 = (src == dst) ? nullptr : p->q[1];
@@ -1042,12 +1049,12 @@ static int pool_step_impl(gf_pool* p, int first, int n, int src, int dst, double
     if (plain) {
         for (int k = 0; k < n; k++) {
             HIPCHK(hipEventRecord(g.ev_step[2 * k], g.stream));
-            HIPCHK(gf::launch_step(p->mx, p->my, p->variant, step_args(p, first + k, 1, q0, q1, nullptr, dt, cur), g.stream));
+            HIPCHK(gf::launch_step(p->mx, p->my, variant, step_args(p, first + k, 1, q0, q1, nullptr, dt, cur), g.stream));
             HIPCHK(hipEventRecord(g.ev_step[2 * k + 1], g.stream));
         }
     } else if (n > 0) {
         HIPCHK(hipEventRecord(g.ev_step[0], g.stream));
-        HIPCHK(gf::launch_step(p->mx, p->my, p->variant, step_args(p, first, n, q0, q1, nullptr, dt, cur), g.stream));
+        HIPCHK(gf::launch_step(p->mx, p->my, variant, step_args(p, first, n, q0, q1, nullptr, dt, cur), g.stream));
         HIPCHK(hipEventRecord(g.ev_step[1], g.stream));
     }
     if (n > 0) HIPCHK(hipMemcpyAsync(p->h_cfl, p->cfl + first, sizeof(double) * n, hipMemcpyDeviceToHost, g.stream));
@@ -1353,10 +1360,9 @@ static int sync_batch_args(gf_pool* p)
 
 // Workgroups of the persistent step kernel: every CU filled to the
 // variant's occupancy.
-static int wet_grid(gf_pool* p)
+static int wet_grid(const gf_pool* p, int variant)
 {
-    if (p->wet_grid == 0) p->wet_grid = g.num_cu * gf::wet_occupancy(p->mx, p->my, p->variant);
-    return p->wet_grid;
+    return g.num_cu * gf::wet_occupancy(p->mx, p->my, variant);
 }
 
 // The multi-level ghost update of a resident AMR pool, which leaves what
@@ -1408,7 +1414,7 @@ static int enqueue_ghost_update(gf_pool* p, int buf, double t, bool classify)
 // persistent kernel over the active tiles and then the dry patches ->
 // controller, all on one stream.  With k >= 0, timing events bracket the
 // step kernel.
-static int enqueue_attempt(gf_pool* p, int k)
+static int enqueue_attempt(gf_pool* p, int k, int variant, int grid)
 {
     if (p->amr) {
         if (int r = enqueue_ghost_update(p, -1, 0.0, true)) return r;
@@ -1419,7 +1425,7 @@ static int enqueue_attempt(gf_pool* p, int k)
         HIPCHK(gf::launch_classify(p->d_args, p->capacity, g.stream));
     }
     if (k >= 0) HIPCHK(hipEventRecord(g.ev_step[2 * k], g.stream));
-    HIPCHK(gf::launch_all(p->mx, p->my, p->variant, gf::default_method(g.P), p->d_args, wet_grid(p), g.stream));
+    HIPCHK(gf::launch_all(p->mx, p->my, variant, gf::default_method(g.P), p->d_args, grid, g.stream));
     if (k >= 0) HIPCHK(hipEventRecord(g.ev_step[2 * k + 1], g.stream));
     HIPCHK(gf::launch_batch_control(p->d_args, p->capacity, g.stream));
     return GF_OK;
@@ -1443,14 +1449,15 @@ static int any_active_flag(gf_pool* p, int* any_active)
 static int run_attempts(gf_pool* p, int substeps, int use_graph)
 {
     if (int r = sync_batch_args(p)) return r;
+    const int variant = step_variant(p, p->n), grid = wet_grid(p, variant);
     if (use_graph) {
-        if (p->graph_dirty) {
+        if (p->graph_dirty || p->graph_variant != variant) {
             if (p->graph_exec) HIPCHK(hipGraphExecDestroy(p->graph_exec));
             if (p->graph) HIPCHK(hipGraphDestroy(p->graph));
             p->graph_exec = nullptr;
             p->graph = nullptr;
             HIPCHK(hipStreamBeginCapture(g.stream, hipStreamCaptureModeThreadLocal));
-            int r = enqueue_attempt(p, -1);
+            int r = enqueue_attempt(p, -1, variant, grid);
             hipGraph_t graph = nullptr;
             hipError_t e = hipStreamEndCapture(g.stream, &graph);
             if (r != GF_OK) return r;
@@ -1458,6 +1465,7 @@ static int run_attempts(gf_pool* p, int substeps, int use_graph)
             p->graph = graph;
             HIPCHK(hipGraphInstantiate(&p->graph_exec, p->graph, nullptr, nullptr, 0));
             p->graph_dirty = false;
+            p->graph_variant = variant;
         }
         HIPCHK(hipEventRecord(g.ev_begin, g.stream));
         for (int k = 0; k < substeps; k++) HIPCHK(hipGraphLaunch(p->graph_exec, g.stream));
@@ -1472,7 +1480,7 @@ static int run_attempts(gf_pool* p, int substeps, int use_graph)
         if (int r = ensure_step_events(std::max(1, substeps))) return r;
         HIPCHK(hipEventRecord(g.ev_begin, g.stream));
         for (int k = 0; k < substeps; k++)
-            if (int r = enqueue_attempt(p, k)) return r;
+            if (int r = enqueue_attempt(p, k, variant, grid)) return r;
         HIPCHK(hipEventRecord(g.ev_end, g.stream));
         HIPCHK(hipStreamSynchronize(g.stream));
         float ms = 0.f;
@@ -1589,7 +1597,7 @@ try {
                                          inflow_grid(), g.stream));
             for (int k = hc[s].first_patch; k < hc[s].first_patch + hc[s].npatch; k++, e++) {
                 HIPCHK(hipEventRecord(g.ev_step[2 * e], g.stream));
-                HIPCHK(gf::launch_step(p->mx, p->my, p->variant,
+                HIPCHK(gf::launch_step(p->mx, p->my, step_variant(p, 1),
                                        step_args(p, k, 1, p->q[0], p->q[1], nullptr, hc[s].dt, hc[s].cur), g.stream));
                 HIPCHK(hipEventRecord(g.ev_step[2 * e + 1], g.stream));
             }
@@ -1683,7 +1691,7 @@ try {
             std::memcpy(sa, aux[k], maux * np2 * sizeof(double));
         }, 1))
         return r;
-    HIPCHK(gf::launch_step(mx, my, p->variant, step_args(p, 0, n, p->q[0], p->q[1], nullptr, dt, 0), g.stream));
+    HIPCHK(gf::launch_step(mx, my, step_variant(p, n), step_args(p, 0, n, p->q[0], p->q[1], nullptr, dt, 0), g.stream));
     HIPCHK(gf::launch_max(p->cfl, n, g.d_max, g.stream));
     HIPCHK(hipMemcpyAsync(g.h_max, g.d_max, sizeof(double), hipMemcpyDeviceToHost, g.stream));
     if (int r = staged_download(p, 0, n, 1, [&](int k, const double* sq) {
@@ -1771,7 +1779,7 @@ try {
     a.tile_cfl = tcfl;
     a.tile_h = tcfl + n;
     a.tile_cnt = reinterpret_cast<int*>(tcfl + 2 * (size_t)n);
-    HIPCHK(gf::launch_step(mx, my, 0, a, g.stream));
+    HIPCHK(gf::launch_step(mx, my, gf::default_variant(mx, my, n, g.num_cu, false), a, g.stream));
     HIPCHK(gf::launch_max(base + L.cfl, n, base + L.dmax, g.stream));
     HIPCHK(gf::launch_unpack(st, q1, 0, n, (int)np2, g.stream));
     for (int k = 0; k < n; k++)
@@ -1915,7 +1923,7 @@ int gf_pool_variants(gf_pool* p, int* current, int* count, int* desc)
 try {
     if (!p) return fail(GF_EINVAL, "pool is NULL");
     const int n = gf::num_variants(p->mx, p->my);
-    if (current) *current = p->variant;
+    if (current) *current = step_variant(p, p->n);
     if (count) *count = n;
     if (desc)
         for (int k = 0; k < n; k++) {
@@ -1935,11 +1943,7 @@ try {
     if (!p) return fail(GF_EINVAL, "pool is NULL");
     if (variant < 0 || variant >= gf::num_variants(p->mx, p->my))
         return fail(GF_EINVAL, "variant %d outside [0,%d)", variant, gf::num_variants(p->mx, p->my));
-    if (variant != p->variant) {
-        p->variant = variant;
-        p->wet_grid = 0;
-        p->graph_dirty = true;
-    }
+    p->variant = variant;
     return GF_OK;
 } GF_CATCH_STATUS
 
@@ -1971,17 +1975,15 @@ try {
         return fail(GF_ESTATE, "no active or dry patch to time: every scenario is inactive or steady");
     }
     if (int r = ensure_pair_events(g.ev_tune, 1)) return r;
-    const int saved = p->variant;
     double best_ms = 0.0;
-    int best_v = saved;
+    int best_v = 0;
     for (int v = 0; v < nv; v++) {
-        p->variant = v;
-        p->wet_grid = 0;
+        const int grid = wet_grid(p, v);
         double tot = 0.0;
         for (int r = 0; r <= reps; r++) {  // the first run warms up
             HIPCHK(hipMemsetAsync(p->counters + gf::CURSOR_LINE, 0, gf::CURSOR_LINE * gf::QUEUES * sizeof(int), g.stream));
             HIPCHK(hipEventRecord(g.ev_tune[0], g.stream));
-            HIPCHK(gf::launch_all(p->mx, p->my, v, gf::default_method(g.P), p->d_args, wet_grid(p), g.stream));
+            HIPCHK(gf::launch_all(p->mx, p->my, v, gf::default_method(g.P), p->d_args, grid, g.stream));
             HIPCHK(hipEventRecord(g.ev_tune[1], g.stream));
             HIPCHK(hipEventSynchronize(g.ev_tune[1]));
             float t = 0.f;
@@ -1999,8 +2001,6 @@ try {
     HIPCHK(hipMemsetAsync(p->counters, 0, gf::NCOUNTERS * sizeof(int), g.stream));
     HIPCHK(hipMemsetAsync(p->cflbits, 0, (size_t)gf::QUEUES * p->capacity * sizeof(unsigned long long), g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
-    p->variant = saved;
-    p->wet_grid = 0;
     if (best) *best = best_v;
     return gf_pool_set_variant(p, best_v);
 } GF_CATCH_STATUS

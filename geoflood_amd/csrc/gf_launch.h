@@ -218,6 +218,8 @@ struct StepVariant {
 };
 int num_variants(int mx, int my);
 bool get_variant(int mx, int my, int k, StepVariant* out);
+// The variant for a launch over `patches` patches when the caller chose none.
+int default_variant(int mx, int my, int patches, int num_cu, bool whole);
 // Resident workgroups per CU of the persistent step kernel of a variant.
 int wet_occupancy(int mx, int my, int variant);
 

@@ -2234,9 +2234,9 @@ bool default_method(const Params& P)
 
 // Step variants per patch shape: X(MX, TX, TY, NT, NPP, FREG) = tiles of
 // TX x TY cells, NT threads per tile, NPP patches per workgroup (one-tile
-// variants), x-face increments in registers (FREG 1) or LDS (0).  The first
-// variant of a shape is its default; the autotuner picks among them by
-// timing.  Every variant gives the same results bit for bit.
+// variants), x-face increments in registers (FREG 1) or LDS (0).  The default
+// is default_variant's; the autotuner picks among all by timing.  Every
+// variant gives the same results bit for bit.
 #define GF_VARIANTS(X)       \
     X(8, 8, 8, 128, 1, 0)       \
     X(8, 8, 8, 128, 1, 1)       \
@@ -2279,6 +2279,34 @@ bool get_variant(int mx, int my, int k, StepVariant* out)
             return true;
         }
     return false;
+}
+
+// Times below: one launch of the batched kernel, every cell wet, 256 CUs.
+//  * 32x32 and 64x64 patches: 16x16 tiles while there are at most two a CU
+//    (the chip is not full: a smaller tile's chain of phases is shorter).
+//    64 patches of 32x32: 18.4 against 27.7 us; 128: 25.5 against 28.2; 192:
+//    45 against 28.9.  16 patches of 64x64: 20.4 against 28.8 us; 32: 26.8
+//    against 30.2; 64: 48 against 32.4.  Else 32x32 tiles of 768 threads
+//    (2,304 patches of 32x32: 217 us; 16x16 tiles 323, 640 threads 262).
+//  * 16x16 patches: 384 threads, one position each, until there are six a
+//    CU; then 192 and two, three workgroups a CU more (4,096 patches: 122
+//    against 147 us; 256: 19.5 against 17.2; 1,600: 68.6 against 70.1, and
+//    27.8 against 25.1 where two thirds of them are dry).
+//  * 8x8 patches: the increments in registers (10,000 patches: 101 against
+//    103.5 us).
+// The population on the device is not known here: the patches described bound
+// it.  whole: one tile per patch, for a step in place.
+int default_variant(int mx, int my, int patches, int num_cu, bool whole)
+{
+    const long long small_tiles = (long long)patches * (mx / 16) * (my / 16);
+    int tx = 32, nt = 768, freg = 0;
+    if (mx == 8) tx = 8, nt = 128, freg = 1;
+    else if (mx == 16) tx = 16, nt = patches > 6 * num_cu ? 192 : 384, freg = 1;
+    else if (!whole && small_tiles <= 2 * num_cu) tx = 16, nt = 384, freg = mx == 32;
+    StepVariant v;
+    for (int k = 0; get_variant(mx, my, k, &v); k++)
+        if (v.tx == tx && v.nt == nt && v.npp == 1 && v.freg == freg) return k;
+    return 0;
 }
 
 static bool same_variant(const StepVariant& v, int mx, int tx, int ty, int nt, int npp, int freg)

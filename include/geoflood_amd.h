@@ -365,7 +365,10 @@ int gf_pool_tag_coarsen(gf_pool *pool, int buf, double t, const gf_refine *crit,
  * variant k.  A tile smaller than the patch splits each patch into tiles with
  * their own 2-cell halo; several patches per workgroup step side by side,
  * one per group of threads.  The results do not depend on the variant.
- * *current is the variant in use.  Any pointer may be NULL.  The reference
+ * *current is the variant in use: the one set or tuned, else the default for
+ * the patches described (fewer patches than fill the GPU take smaller tiles;
+ * a step in place takes one tile per patch where the shape has such a
+ * variant).  Any pointer may be NULL.  The reference
  * fixes one shape (cudaclaw_flux2.cu:68-120: one block of 128 threads per
  * patch). */
 int gf_pool_variants(gf_pool *pool, int *current, int *count, int *desc);
