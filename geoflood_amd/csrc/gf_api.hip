@@ -283,12 +283,12 @@ struct gf_pool {
     std::vector<int> h_links, h_link_level; // the links as given, [n][coarse, fine, side, igrid], and their coarse levels
     std::vector<int> h_inflow;             // the slots of inflow_list
     std::vector<int> slot_item;            // [capacity] scratch of rebuild_ghost_items, -1 between calls
-    // one device block: the numbers of items per level and of links, [5][link_cap]
-    // coarse, fine, side, igrid, scenario in item order, then the items by level
+    // one device block: the numbers of items per pass and of links, [5][link_cap]
+    // coarse, fine, side, igrid, scenario in item order, then the items by pass
     int* d_amr = nullptr;
     int link_cap = 0, nlinks = 0;
-    int level_items[kMaxLevels + 1] = {};  // first item of each level in the block (a multiple of 64 apart)
-    unsigned ghost_levels = 0;             // bit l: level l has items
+    int pass_items[kMaxLevels + 1] = {};  // first item of each pass in the block (a multiple of 64 apart)
+    unsigned ghost_passes = 0;             // bit k: pass k has items
 };
 
 static void default_params()
@@ -482,15 +482,74 @@ static void free_hydrographs(gf_pool* p)
     }
 }
 
+// One patch of the resident ghost update: the coarse patch of `links` links,
+// or one with a hydrograph side, or both.
+struct GhostEntry {
+    int patch, level, links, inflow, pass;
+};
+
+// The passes of the resident ghost update.  ForestClaw's order goes level by
+// level, coarse to fine; but of the ghost cells that a coarser level's links
+// write into a patch, the patch's own item reads only
+//  * for a face link, those beside the cells at its half's end: the side
+//    perpendicular to it there (and its own side); for a corner link the two
+//    sides that meet there.  No corner ghost cells.
+//  * for a hydrograph side, the ring beside it, which only the ghost cells at
+//    its two ends depend on (no link reads those).
+// So an item waits for a coarser one only if its patch takes a side that its
+// links read from it, and the items of every level that wait for none go
+// together.  In a forest balanced across corners no link waits: patches two
+// levels apart would touch at the corner between the two sides.  A hydrograph
+// patch that a coarser one writes to has its hydrograph side filled again
+// after that (an entry of its own), for the ends.
+static void ghost_passes(const gf_pool* p, std::vector<GhostEntry>& e, const std::vector<int>& item_of)
+{
+    const int nl = (int)p->h_link_level.size();
+    const int* link = p->h_links.data();
+    int top = 0;
+    bool level_order = false;  // levels given anew since the links were: keep the levels' own order
+    for (GhostEntry& x : e) {
+        x.pass = x.level;
+        top = std::max(top, x.level);
+    }
+    for (int k = 0; k < nl; k++)
+        level_order |= p->h_level[link[4 * k]] != p->h_link_level[k] || p->h_level[link[4 * k + 1]] != p->h_link_level[k] + 1;
+    if (level_order) return;
+    std::vector<unsigned char> takes(p->capacity, 0);  // face sides that a coarser patch's link writes; 16: a corner
+    std::vector<unsigned char> after(p->capacity, 0);  // the pass after those links'
+    std::vector<unsigned char> reads(e.size(), 0);     // face sides that the item's links read
+    for (int k = 0; k < nl; k++) {
+        const int side = link[4 * k + 2], igrid = link[4 * k + 3];
+        takes[link[4 * k + 1]] |= side < 4 ? 1 << (side ^ 1) : 16;
+        reads[item_of[k]] |= side < 2   ? (1 << side) | (4 << igrid)
+                             : side < 4 ? (1 << side) | (1 << igrid)
+                                        : (1 << ((side - 4) & 1)) | (4 << ((side - 4) >> 1));
+    }
+    for (int l = 0; l <= top; l++) {
+        for (size_t i = 0; i < e.size(); i++) {
+            if (e[i].level != l) continue;
+            e[i].pass = (takes[e[i].patch] & reads[i]) ? after[e[i].patch] : 0;
+        }
+        for (int k = 0; k < nl; k++) {
+            if (p->h_link_level[k] != l) continue;
+            unsigned char& a = after[link[4 * k + 1]];
+            a = std::max<int>(a, e[item_of[k]].pass + 1);
+        }
+    }
+    for (size_t i = 0, n = e.size(); i < n; i++)
+        if (e[i].inflow && after[e[i].patch] > e[i].pass) {
+            if (e[i].links) e.push_back({e[i].patch, e[i].level, 0, 1, after[e[i].patch]});
+            else e[i].pass = after[e[i].patch];
+        }
+}
+
 // Rebuild the device items of the resident ghost update from the pool's links
-// and hydrograph patches: one item per patch, level by level, each with its
+// and hydrograph patches: one item per patch, pass by pass, each with its
 // links in one run.
 static int rebuild_ghost_items(gf_pool* p)
 {
     const int nl = (int)p->h_link_level.size();
-    struct Entry {
-        int patch, level, links, inflow;
-    };
+    using Entry = GhostEntry;
     std::vector<Entry> e;
     p->slot_item.resize(p->capacity, -1);
     std::vector<int> item_of(nl);
@@ -498,7 +557,7 @@ static int rebuild_ghost_items(gf_pool* p)
         int& i = p->slot_item[p->h_links[4 * k]];
         if (i < 0) {
             i = (int)e.size();
-            e.push_back({p->h_links[4 * k], p->h_link_level[k], 0, 0});
+            e.push_back({p->h_links[4 * k], p->h_link_level[k], 0, 0, 0});
         }
         e[i].links++;
         item_of[k] = i;
@@ -507,20 +566,21 @@ static int rebuild_ghost_items(gf_pool* p)
     for (int s : p->h_inflow) {
         const int i = p->slot_item[s];
         if (i >= 0 && e[i].level == p->h_level[s]) e[i].inflow = 1;
-        else e.push_back({s, p->h_level[s], 0, 1});
+        else e.push_back({s, p->h_level[s], 0, 1, 0});
     }
     for (size_t i = 0; i < linked; i++) p->slot_item[e[i].patch] = -1;
-    // the place of each level's items in the block is part of the captured
-    // graph: it is kept while every level's items fit
+    ghost_passes(p, e, item_of);
+    // the place of each pass's items in the block is part of the captured
+    // graph: it is kept while every pass's items fit
     int count[kMaxLevels] = {};
-    for (const Entry& x : e) count[x.level]++;
+    for (const Entry& x : e) count[x.pass]++;
     bool fits = p->d_amr != nullptr && nl <= p->link_cap;
-    for (int l = 0; l < kMaxLevels; l++) fits = fits && count[l] <= p->level_items[l + 1] - p->level_items[l];
+    for (int l = 0; l < kMaxLevels; l++) fits = fits && count[l] <= p->pass_items[l + 1] - p->pass_items[l];
     if (!fits) {
         const int lc = nl > p->link_cap ? std::max(nl, 2 * p->link_cap) : p->link_cap;
         int first[kMaxLevels + 1] = {};
         for (int l = 0; l < kMaxLevels; l++) {
-            const int had = p->level_items[l + 1] - p->level_items[l];
+            const int had = p->pass_items[l + 1] - p->pass_items[l];
             first[l + 1] = first[l] + (count[l] > had ? (2 * count[l] + 63) / 64 * 64 : had);
         }
         int* d = nullptr;
@@ -529,16 +589,16 @@ static int rebuild_ghost_items(gf_pool* p)
         HIPCHK(hipFree(p->d_amr));
         p->d_amr = d;
         p->link_cap = lc;
-        std::copy(first, first + kMaxLevels + 1, p->level_items);
+        std::copy(first, first + kMaxLevels + 1, p->pass_items);
         p->graph_dirty = true;  // the graph holds the block's addresses
     }
-    std::vector<int> h(kAmrHead + 5 * (size_t)p->link_cap + sizeof(gf::GhostItem) / sizeof(int) * (size_t)p->level_items[kMaxLevels], 0);
-    unsigned levels = 0;
+    std::vector<int> h(kAmrHead + 5 * (size_t)p->link_cap + sizeof(gf::GhostItem) / sizeof(int) * (size_t)p->pass_items[kMaxLevels], 0);
+    unsigned passes = 0;
     int next[kMaxLevels];
     for (int l = 0; l < kMaxLevels; l++) {
         h[l] = count[l];
-        if (count[l]) levels |= 1u << l;
-        next[l] = p->level_items[l];
+        if (count[l]) passes |= 1u << l;
+        next[l] = p->pass_items[l];
     }
     h[kMaxLevels] = nl;
     int* links = h.data() + kAmrHead;
@@ -546,7 +606,7 @@ static int rebuild_ghost_items(gf_pool* p)
     std::vector<int> cursor(e.size());
     int off = 0;
     for (size_t i = 0; i < e.size(); i++) {
-        items[next[e[i].level]++] = {e[i].patch, p->h_desc[e[i].patch].scen, off, off + e[i].links, e[i].inflow};
+        items[next[e[i].pass]++] = {e[i].patch, p->h_desc[e[i].patch].scen, off, off + e[i].links, e[i].inflow};
         cursor[i] = off;
         off += e[i].links;
     }
@@ -555,9 +615,9 @@ static int rebuild_ghost_items(gf_pool* p)
         for (int m = 0; m < 4; m++) links[(size_t)m * p->link_cap + at] = p->h_links[4 * k + m];
         links[4 * (size_t)p->link_cap + at] = p->h_desc[p->h_links[4 * k]].scen;
     }
-    if (levels != p->ghost_levels || nl != p->nlinks) {
-        if (levels != p->ghost_levels || (nl > 0) != (p->nlinks > 0)) p->graph_dirty = true;
-        p->ghost_levels = levels;
+    if (passes != p->ghost_passes || nl != p->nlinks) {
+        if (passes != p->ghost_passes || (nl > 0) != (p->nlinks > 0)) p->graph_dirty = true;
+        p->ghost_passes = passes;
         p->nlinks = nl;
     }
     HIPCHK(hipMemcpyAsync(p->d_amr, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice, g.stream));
@@ -1369,7 +1429,8 @@ static int wet_grid(const gf_pool* p, int variant)
 // ForestClaw's order leaves (fclaw2d_ghost_update with time_interp off): the
 // coarse ghost cells that finer neighbours cover, averaged from them; then for
 // each level from coarse to fine its hydrograph sides, and the next finer
-// level's ghost cells interpolated from it (k_ghost_begin, k_ghost_level).
+// level's ghost cells interpolated from it (k_ghost_begin, k_ghost_level; the
+// levels share a launch where nothing waits, ghost_passes).
 // classify: the attempt's classification shares the first launch (buf < 0;
 // p->d_args is up to date).  Same-level copies and
 // walls need no pass: every reader takes them from the neighbours
@@ -1401,8 +1462,8 @@ static int enqueue_ghost_update(gf_pool* p, int buf, double t, bool classify)
     HIPCHK(gf::launch_ghost_begin(p->mx, p->my, a, buf < 0 ? p->d_args : nullptr, classify ? p->capacity : 0,
                                   p->nlinks > 0 ? kLinkBlocks : 0, buf < 0 && p->has_inflow ? kHydroBlocks : 0, g.stream));
     for (int l = 0; l < kMaxLevels; l++) {
-        if (!(p->ghost_levels >> l & 1u)) continue;
-        a.items = items + p->level_items[l];
+        if (!(p->ghost_passes >> l & 1u)) continue;
+        a.items = items + p->pass_items[l];
         a.count = p->d_amr + l;
         HIPCHK(gf::launch_ghost_level(p->mx, p->my, a, kGhostGrid, g.stream));
     }

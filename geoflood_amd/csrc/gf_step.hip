@@ -1331,6 +1331,9 @@ struct Ring {
     }
 };
 
+// Sides that bc2 fills.
+__device__ __forceinline__ bool is_bc(int code) { return code == NB_WALL || code == NB_EXTRAP || code == NB_INFLOW; }
+
 // Ghost ring of one hydrograph patch (base: the q buffer) by a workgroup of
 // 256 threads.  It is a chain of dependent steps rather than work (a few
 // hundred cells): the last wave looks the discharge up (or takes it from
@@ -1408,7 +1411,7 @@ __device__ void inflow_patch(double* L, double* hu_sh, double* base, double* aux
     const double hu0 = *hu_sh;
     for (int side = 0; side < 4; side++) {
         const int code = dp->nbr[side];
-        if (code != NB_WALL && code != NB_EXTRAP && code != NB_INFLOW) continue;
+        if (!is_bc(code)) continue;
         bc2_side<MX, MY>(L, side, code, dp, c, hu0, P);
         __syncthreads();
     }
@@ -1416,6 +1419,12 @@ __device__ void inflow_patch(double* L, double* hu_sh, double* base, double* aux
         int fi, fj;
         R::cell(e, fi, fj);
         if (fi >= 1 && fi <= MX && fj >= 1 && fj <= MY) continue;
+        // stored cells that no side pass wrote are left alone: a coarser
+        // patch's item may be writing them
+        const int xs = fi < 1 ? 0 : fi > MX ? 1 : -1, ys = fj < 1 ? 2 : fj > MY ? 3 : -1;
+        const bool pass = (xs >= 0 && is_bc(dp->nbr[xs])) || (ys >= 0 && is_bc(dp->nbr[ys]));
+        const int region = xs < 0 ? ys : ys < 0 ? xs : 4 + xs + 2 * (ys - 2);
+        if (!pass && dp->nbr[region] == NB_STORED) continue;
         const int k = G::ti(fi, fj);
         q[k] = L[k];
         q[NP2 + k] = L[NP2 + k];
@@ -2025,14 +2034,14 @@ __global__ void __launch_bounds__(64) k_interpolate_ghost(RegridArgs a)
 //  * k_ghost_begin: the coarse ghost cells under finer neighbours, averaged
 //    from their interiors, of every level; the discharge of every scenario's
 //    hydrograph at its time; and the attempt's classification.
-//  * k_ghost_level, once per level: one workgroup per patch that has finer
-//    neighbours or a hydrograph side fills its hydrograph sides, then the ghost
-//    cells of those neighbours.  All that these read of ghost cells is the
-//    patch's own, so only the levels follow each other (a patch's ghost cells
-//    towards a coarser one are written by the coarser level's launch).
-// On four levels of 16x16 patches (0.9k leaves) the five launches take 50 us;
-// averaging, hydrographs, interpolation and classification as nine launches of
-// their own took 63 us and three more launch gaps.
+//  * k_ghost_level: one workgroup per patch that has finer neighbours or a
+//    hydrograph side fills its hydrograph sides, then the ghost cells of those
+//    neighbours.  All that these read of ghost cells is the patch's own, and
+//    where that is none that a coarser patch writes, the levels share one
+//    launch (the passes are the host's, which knows the links).
+// On four levels of 16x16 patches (1,970 leaves) the three launches take
+// 26 us; a launch per level took 50, and averaging, hydrographs,
+// interpolation and classification on their own nine launches and 63.
 __device__ __forceinline__ double* link_buffer(const GhostLevelArgs& a, int scen)
 {
     if (a.buf >= 0) return a.buf ? a.q1 : a.q0;
