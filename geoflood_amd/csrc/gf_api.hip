@@ -1043,6 +1043,7 @@ static gf::InflowArgs inflow_args(gf_pool* p, int first, int last, int buf, doub
 {
     gf::InflowArgs a{};
     a.desc = p->desc;
+    a.regions = p->regions;
     a.ctrl = p->ctrl;
     a.q0 = p->q[0];
     a.q1 = p->q[1];
@@ -1442,7 +1443,7 @@ static int enqueue_ghost_update(gf_pool* p, int buf, double t, bool classify)
     gf::GhostLevelArgs a{};
     const int* links = p->d_amr + kAmrHead;
     const gf::GhostItem* items = reinterpret_cast<const gf::GhostItem*>(links + 5 * (size_t)p->link_cap);
-    a.links.desc = p->desc;
+    a.links.regions = p->regions;
     a.links.aux = p->aux;
     a.links.cs = links;
     a.links.fs = links + p->link_cap;
@@ -1465,7 +1466,8 @@ static int enqueue_ghost_update(gf_pool* p, int buf, double t, bool classify)
         if (!(p->ghost_passes >> l & 1u)) continue;
         a.items = items + p->pass_items[l];
         a.count = p->d_amr + l;
-        HIPCHK(gf::launch_ghost_level(p->mx, p->my, a, kGhostGrid, g.stream));
+        a.room = p->pass_items[l + 1] - p->pass_items[l];
+        HIPCHK(gf::launch_ghost_level(p->mx, p->my, a, std::min(kGhostGrid, a.room), g.stream));
     }
     return GF_OK;
 }
@@ -2257,7 +2259,7 @@ static int regrid_impl(gf_pool* p, int buf, int n, const int* cs, const int* fs,
     int *dcs = nullptr, *dfs = nullptr;
     if (int r = regrid_lists(p, n, cs, fs, &dcs, &dfs)) return r;
     gf::RegridArgs a{};
-    a.desc = p->desc;
+    a.regions = p->regions;
     a.q = p->q[buf];
     a.aux = p->aux;
     a.cs = dcs;
@@ -2342,7 +2344,7 @@ static int cf_ghost_impl(gf_pool* p, int buf, int n, const int* cs, const int* f
         HIPCHK(hipMemcpyAsync(d + k * stride, src, sizeof(int) * n, hipMemcpyHostToDevice, g.stream));
     }
     gf::RegridArgs a{};
-    a.desc = p->desc;
+    a.regions = p->regions;
     a.q = p->q[buf];
     a.aux = p->aux;
     a.cs = (const int*)d;

@@ -49,11 +49,24 @@ struct GaugeArgs {
     double dry_tolerance;
 };
 
+// Where the cells of one of the nine regions of a patch and its halo (left /
+// inside / right by below / inside / above) lie in a q buffer: cell (fi, fj) at
+// off + kx fi + ky fj, with hu / hv negated or not.  ghost_source's rule is
+// linear in each region, and is evaluated once per region when a slot is
+// described: per cell of every tile load, its branches were a sixth of a 32x32
+// tile's time (9,000 of 57,000 cycles).
+constexpr int REGIONS = 9;
+struct RegionSrc {
+    long long off;
+    int kx;
+    int ky_neg;  // ky * 4 + (hu negated) + 2 (hv negated)
+};
+
 // Regrid between levels on resident patches (refinement ratio 2): family f
 // has the coarse patch in slot cs[f] and its children in slots fs[4f + g],
 // g = igrid = 0..3 (x fastest), all in buffer q.
 struct RegridArgs {
-    const PatchDesc* desc;
+    const RegionSrc* regions;  // of every slot
     double* q;
     const double* aux;
     const int* cs;
@@ -83,6 +96,7 @@ struct TimeInterpArgs {
 // and time and skips inactive scenarios; otherwise buffer buf at time t.
 struct InflowArgs {
     const PatchDesc* desc;
+    const RegionSrc* regions;  // of every slot
     const ScenCtrl* ctrl;
     double* q0;
     double* q1;
@@ -116,22 +130,10 @@ struct GhostLevelArgs {
     double* aux;
     const GhostItem* items;
     const int* count;      // links (k_ghost_begin) or items (k_ghost_level)
+    int room;              // places for items, from `items` on
     int buf;
     double t;
     Params P;
-};
-
-// Where the cells of one of the nine regions of a patch and its halo (left /
-// inside / right by below / inside / above) lie in a q buffer: cell (fi, fj) at
-// off + kx fi + ky fj, with hu / hv negated or not.  ghost_source's rule is
-// linear in each region, and is evaluated once per region when a slot is
-// described: per cell of every tile load, its branches were a sixth of a 32x32
-// tile's time (9,000 of 57,000 cycles).
-constexpr int REGIONS = 9;
-struct RegionSrc {
-    long long off;
-    int kx;
-    int ky_neg;  // ky * 4 + (hu negated) + 2 (hv negated)
 };
 
 // Dry-list entries carry the patch's current buffer: patch | cur << 30.
