@@ -240,6 +240,7 @@ struct gf_pool {
     double* h_stage = nullptr;  // pinned host staging
     size_t stage_doubles = 0;   // size of each staging buffer
     double* h_cfl = nullptr;    // pinned
+    ScenCtrl* h_rec = nullptr;  // pinned: a scenario's record (gf_pool_advance)
     // batched path
     double* hmax2 = nullptr;               // [2][capacity]
     unsigned long long* cflbits = nullptr; // [gf::QUEUES][capacity] per scenario
@@ -695,6 +696,7 @@ try {
               hipMalloc(&p->d_stage, chunk * 4 * p->np2 * sizeof(double)) == hipSuccess &&
               hipHostMalloc(&p->h_stage, chunk * 4 * p->np2 * sizeof(double), hipHostMallocDefault) == hipSuccess &&
               hipHostMalloc(&p->h_cfl, (size_t)capacity * sizeof(double), hipHostMallocDefault) == hipSuccess &&
+              hipHostMalloc(&p->h_rec, sizeof(ScenCtrl), hipHostMallocDefault) == hipSuccess &&
               hipMalloc(&p->hmax2, (size_t)2 * capacity * sizeof(double)) == hipSuccess &&
               hipMalloc(&p->cflbits, (size_t)gf::QUEUES * capacity * sizeof(unsigned long long)) == hipSuccess &&
               hipMalloc(&p->list_wet, (size_t)capacity * sizeof(int)) == hipSuccess &&
@@ -786,6 +788,7 @@ try {
     for (double* m : p->hyd_mem) hipFree(m);
     if (p->h_stage) hipHostFree(p->h_stage);
     if (p->h_cfl) hipHostFree(p->h_cfl);
+    if (p->h_rec) hipHostFree(p->h_rec);
     delete p;
     return GF_OK;
 } GF_CATCH_STATUS
@@ -1508,8 +1511,9 @@ static int any_active_flag(gf_pool* p, int* any_active)
 
 // `substeps` attempts of every active scenario (graph replays or stream
 // launches), then a stream synchronisation; the device time between the
-// first and the last attempt goes to g.last_total_ms.
-static int run_attempts(gf_pool* p, int substeps, int use_graph)
+// first and the last attempt goes to g.last_total_ms.  record >= 0: that
+// scenario's record is in p->h_rec afterwards.
+static int run_attempts(gf_pool* p, int substeps, int use_graph, int record = -1)
 {
     if (int r = sync_batch_args(p)) return r;
     const int variant = step_variant(p, p->n), grid = wet_grid(p, variant);
@@ -1533,6 +1537,7 @@ static int run_attempts(gf_pool* p, int substeps, int use_graph)
         HIPCHK(hipEventRecord(g.ev_begin, g.stream));
         for (int k = 0; k < substeps; k++) HIPCHK(hipGraphLaunch(p->graph_exec, g.stream));
         HIPCHK(hipEventRecord(g.ev_end, g.stream));
+        if (record >= 0) HIPCHK(gf::launch_read_record(p->ctrl + record, p->h_rec, g.stream));
         HIPCHK(hipStreamSynchronize(g.stream));
         float ms = 0.f;
         HIPCHK(hipEventElapsedTime(&ms, g.ev_begin, g.ev_end));
@@ -1545,6 +1550,7 @@ static int run_attempts(gf_pool* p, int substeps, int use_graph)
         for (int k = 0; k < substeps; k++)
             if (int r = enqueue_attempt(p, k, variant, grid)) return r;
         HIPCHK(hipEventRecord(g.ev_end, g.stream));
+        if (record >= 0) HIPCHK(gf::launch_read_record(p->ctrl + record, p->h_rec, g.stream));
         HIPCHK(hipStreamSynchronize(g.stream));
         float ms = 0.f;
         HIPCHK(hipEventElapsedTime(&ms, g.ev_begin, g.ev_end));
@@ -1575,17 +1581,21 @@ try {
     if (s < 0 || s >= p->capacity || p->h_ctrl[s].npatch == 0) return fail(GF_EINVAL, "scenario %d unknown", s);
     if (target_steps <= 0) return fail(GF_EINVAL, "target_steps must be > 0");
     if (!p->inflow_error.empty()) return fail(GF_EINVAL, "%s", p->inflow_error.c_str());
-    // the stop condition, as gf_pool_set_scenario_stop sets it (t_end off)
+    // the stop condition, as gf_pool_set_scenario_stop sets it (t_end off).
+    // The records go through pinned memory that kernels write, the last one in
+    // the same wait as the attempts: three pageable copies and their waits
+    // took a quarter of the 360 us of a call of four attempts.
     ScenCtrl& c = p->h_ctrl[s];
-    HIPCHK(hipMemcpyAsync(&c, p->ctrl + s, sizeof(ScenCtrl), hipMemcpyDeviceToHost, g.stream));
+    HIPCHK(gf::launch_read_record(p->ctrl + s, p->h_rec, g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
+    c = *p->h_rec;
     if (max_attempts > 0 && target_steps - c.nsteps > max_attempts)
         return fail(GF_ESTATE, "scenario %d: %d steps short of %d exceed max_attempts %d", s, target_steps - c.nsteps,
                     target_steps, max_attempts);
     c.target_steps = target_steps;
     c.t_end = 0.0;
     c.active = (c.status == gf::SCEN_OK && c.nsteps < target_steps) ? 1 : 0;
-    HIPCHK(hipMemcpyAsync(p->ctrl + s, &c, sizeof(ScenCtrl), hipMemcpyHostToDevice, g.stream));
+    HIPCHK(gf::launch_set_target(p->ctrl + s, target_steps, c.active, g.stream));
     // one attempt per missing step, then single attempts for the retakes
     double total_ms = 0.0;
     int attempts = 0;
@@ -1595,11 +1605,10 @@ try {
         if (max_attempts > 0 && attempts + k > max_attempts)
             return fail(GF_ESTATE, "scenario %d: %d steps short of %d after %d attempts", s, target_steps - now.nsteps,
                         target_steps, attempts);
-        if (int r = run_attempts(p, k, use_graph)) return r;
+        if (int r = run_attempts(p, k, use_graph, s)) return r;
         total_ms += g.last_total_ms;
         attempts += k;
-        HIPCHK(hipMemcpyAsync(&now, p->ctrl + s, sizeof(ScenCtrl), hipMemcpyDeviceToHost, g.stream));
-        HIPCHK(hipStreamSynchronize(g.stream));
+        now = *p->h_rec;
     }
     g.last_total_ms = total_ms;
     p->h_ctrl[s] = now;

@@ -257,6 +257,9 @@ hipError_t launch_frame_pack(int mx, int my, double* q, const double* aux, int f
                              hipStream_t st);
 hipError_t launch_gauges(int mx, int my, const GaugeArgs& a, hipStream_t st);
 hipError_t launch_hmax(int mx, int my, const double* q, double* hmax, int first, int n, hipStream_t st);
+// A scenario's record to pinned host memory; its stop condition.
+hipError_t launch_read_record(const ScenCtrl* c, ScenCtrl* host, hipStream_t st);
+hipError_t launch_set_target(ScenCtrl* c, int target_steps, int active, hipStream_t st);
 hipError_t launch_step(int mx, int my, int variant, const StepArgs& a, hipStream_t st);
 hipError_t launch_ghost(int mx, int my, const GhostArgs& a, hipStream_t st);
 hipError_t launch_control(ScenCtrl* ctrl, int nscen, const double* cfl, hipStream_t st);

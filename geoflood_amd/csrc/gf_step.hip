@@ -892,7 +892,7 @@ struct ItemPrefetch {
 };
 
 // Persistent step kernel over the device work list of active patches:
-// each workgroup takes the next (patch, tile) entry from an atomic counter,
+// each workgroup takes (patch, tile) entries (its own index, then its queue's),
 // pulls the tile's halo from the patch and its neighbours, steps it, and
 // folds the patch's capped CFL number into the scenario's maximum
 // (atomicMax on the bit pattern of a CFL > 0).  One entry of the persistent
@@ -1610,6 +1610,23 @@ __global__ void __launch_bounds__(64) k_batch_control(const BatchArgs* pa)
 #pragma unroll
     for (int q = 0; q < QUEUES; q++) a.cflbits[(size_t)q * a.capacity + s] = 0ull;
     control_step(c, m);
+}
+
+// A scenario's record to pinned host memory (one wave): a copy of its own
+// costs more than this launch, and needs its own wait.
+__global__ void __launch_bounds__(64) k_read_record(const ScenCtrl* c, ScenCtrl* host)
+{
+    constexpr int W = sizeof(ScenCtrl) / 8;
+    static_assert(W <= 64 && sizeof(ScenCtrl) % 8 == 0, "one word a lane");
+    if (threadIdx.x < W) ((long long*)host)[threadIdx.x] = ((const long long*)c)[threadIdx.x];
+}
+
+// A scenario's stop condition: target_steps accepted steps, no end time.
+__global__ void k_set_target(ScenCtrl* c, int target_steps, int active)
+{
+    c->target_steps = target_steps;
+    c->t_end = 0.0;
+    c->active = active;
 }
 
 // Maximum interior depth of patches [first, first+n) of a q buffer.
@@ -2372,6 +2389,18 @@ hipError_t launch_step(int mx, int my, int variant, const StepArgs& a, hipStream
     GF_VARIANTS(GF_STEP)
 #undef GF_STEP
     return hipErrorInvalidValue;
+}
+
+hipError_t launch_read_record(const ScenCtrl* c, ScenCtrl* host, hipStream_t st)
+{
+    k_read_record<<<1, 64, 0, st>>>(c, host);
+    return hipGetLastError();
+}
+
+hipError_t launch_set_target(ScenCtrl* c, int target_steps, int active, hipStream_t st)
+{
+    k_set_target<<<1, 1, 0, st>>>(c, target_steps, active);
+    return hipGetLastError();
 }
 
 hipError_t launch_ghost(int mx, int my, const GhostArgs& a, hipStream_t st)
