@@ -460,9 +460,8 @@ const char* gf_last_error(void) { return g_err.c_str(); }
 long long gf_pool_bytes(int mx, int my, int mbc, int capacity)
 {
     const long long np2 = (long long)(mx + 2 * mbc) * (my + 2 * mbc);
-    const long long per = (2 * 3 * np2 + np2) * 8 + (long long)sizeof(PatchDesc) +
-                          (long long)(gf::REGIONS * sizeof(gf::RegionSrc)) + 8 /*cfl*/ + 16 /*hmax*/ +
-                          8 * gf::QUEUES /*cflbits*/ + 8 /*lists*/ + 8 /*legacy hmax*/ + 4 /*dry age*/ + sizeof(ScenCtrl);
+    const long long per = (2 * 3 * np2 + np2) * 8 + (long long)sizeof(PatchDesc) + 8 /*cfl*/ + 16 /*hmax*/ +
+                          8 /*cflbits*/ + 8 /*lists*/ + 8 /*legacy hmax*/ + 4 /*dry age*/ + sizeof(ScenCtrl);
     const long long staging = (long long)kChunk * 4 * np2 * 8;
     return per * capacity + staging;
 }

@@ -135,7 +135,9 @@ int gf_get_params(gf_params *params);
 const char *gf_last_error(void);
 
 /* Number of bytes of HBM a pool of `capacity` patches of mx x my occupies
- * (both q buffers, aux, descriptors, per-patch scratch). */
+ * (both q buffers, aux, descriptors, per-patch scratch).  The step's work
+ * tables (halo sources, tile folds, queue maxima: 224 bytes a patch) are not
+ * in it. */
 long long gf_pool_bytes(int mx, int my, int mbc, int capacity);
 
 /* ---- drop-in batch step (reference architecture) ------------------------ */
