@@ -25,6 +25,7 @@
 #include <vector>
 
 #include "../../include/geoflood_amd.h"
+#include "gf_exact.h"
 #include "gf_launch.h"
 #include "gf_output.h"
 

@@ -82,40 +82,32 @@ GF_DEVICE double rsq_seed(double b) { return __builtin_amdgcn_rsq(b); }
 GF_DEVICE int exponent_of(double a) { return __builtin_amdgcn_frexp_exp(a); }  // 0 for 0, NaN and Inf
 #endif
 
+namespace fast {
+
 // A denominator with its refined reciprocal.
 struct Recip {
     double b, y;
 };
 
-template <bool FAST>
 GF_DEVICE Recip recip(double b)
 {
-    if (!FAST) return Recip{b, 0.0};
     double y = rcp_seed(b);
     y = ::fma(y, ::fma(-b, y, 1.0), y);
     y = ::fma(y, ::fma(-b, y, 1.0), y);
     return Recip{b, y};
 }
 
-template <bool FAST>
 GF_DEVICE double quot(double a, const Recip& d)
 {
-    if (!FAST) return a / d.b;
     const double q = a * d.y;
     return ::fma(::fma(-d.b, q, a), d.y, q);
 }
 
-template <bool FAST>
-GF_DEVICE double quot(double a, double b)
-{
-    return quot<FAST>(a, recip<FAST>(b));
-}
+GF_DEVICE double quot(double a, double b) { return quot(a, recip(b)); }
 
-// sqrt(x); FAST: x = 0 or 2^-700 <= x <= 2^700.
-template <bool FAST>
+// sqrt(x), x = 0 or 2^-700 <= x <= 2^700.
 GF_DEVICE double root(double x)
 {
-    if (!FAST) return ::sqrt(x);
     const double y = rsq_seed(::fmax(x, 0x1p-700));
     double s = x * y, h = 0.5 * y;
     const double r = ::fma(-h, s, 0.5);
@@ -125,18 +117,12 @@ GF_DEVICE double root(double x)
     return ::fma(::fma(-s, s, x), h, s);
 }
 
-// Maximum and minimum as LLVM Flang evaluates MAX and MIN.  FAST: the
-// operands are numbers and the sign of a zero result does not matter, and one
-// instruction does it instead of a compare and two selects.
-template <bool FAST>
-GF_DEVICE double vmax(double a, double b)
-{
-    return FAST ? ::fmax(a, b) : (a > b ? a : b);
-}
-template <bool FAST>
-GF_DEVICE double vmin(double a, double b)
-{
-    return FAST ? ::fmin(a, b) : (a < b ? a : b);
-}
+// Maximum and minimum of two numbers where the sign of a zero result does not
+// matter: one instruction instead of a compare and two selects.  (A NaN operand
+// is lost here; LLVM Flang's MAX and MIN, fmaxf64 and fminf64, return the
+// second operand then.)
+GF_DEVICE double vmax(double a, double b) { return ::fmax(a, b); }
+GF_DEVICE double vmin(double a, double b) { return ::fmin(a, b); }
 
+}  // namespace fast
 }  // namespace gf

@@ -6,22 +6,17 @@
 // momentum) with respect to the face being solved, which is how rpn2/rpt2
 // index them through mu/nv (rpn2_geoclaw.f:101-107, rpt2_geoclaw.f:46-54).
 //
+// These are the general operations: they hold for every value, and a tile with
+// a cell, a parameter or a step size outside the range of gf_exact.h (a NaN or
+// an infinity among them) is stepped with them.  Tiles inside it take the
+// cheaper forms of gf_physics_fast.h, which give the same results there.
+//
 // Fortran intrinsics keep LLVM Flang's semantics: MAX(a,b) = a > b ? a : b,
 // MIN(a,b) = a < b ? a : b, SIGN(1,x) = copysign(1,x).
-//
-// FAST selects the quotients, roots, maxima and minima of gf_exact.h for
-// tiles whose cells lie in its range; the results are the same.  Either way
-// terms that are exact zeros for finite values (Cramer's rule of the sparse
-// eigenvector matrix, the second wave's two zero components) are left out,
-// which changes no more than the sign of a zero.  On the 4096^2 dam break a
-// launch of the 32x32 step kernel (about 2,360 active patches) fell from
-// 1.275e8 to 1.019e8 VALU instructions and from 346 to 284 us (with the other
-// steps of the kernel since: 8.8e7 on 2,244 active patches, 253 us).
 #pragma once
 
 #include <hip/hip_runtime.h>
 
-#include "gf_exact.h"
 #include "gf_pow.h"
 
 namespace gf {
@@ -49,167 +44,181 @@ struct Params {
 __device__ __forceinline__ double fmaxf64(double a, double b) { return a > b ? a : b; }
 __device__ __forceinline__ double fminf64(double a, double b) { return a < b ? a : b; }
 
-// Quotients of one cell's depth: for a wet cell hu/h, hv/h, sqrt(g h) and the
-// reciprocal they share, formed once for the faces and splits that use them.
-struct CellVel {
-    double u, v, sg, y;
-};
-
-template <bool FAST>
-__device__ __forceinline__ CellVel cell_velocity(double h, double hu, double hv, double g)
+// riemanntype (geoclaw_riemann_utils.f:566-677) with maxiter = 1; returns
+// hm and the middle-state speeds s1m, s2m (rare1/rare2 are unused by callers).
+// sgL, sgR are sqrt(g*hL), sqrt(g*hR), which the caller has already formed:
+// every sqrt(g*h) of hL, hR, h_min or h_max below is one of them, bit for bit.
+__device__ __forceinline__ void riemanntype(double hL, double hR, double uL, double uR,
+                                            double sgL, double sgR, double drytol, double g, double halfg, double inv16g,
+                                            double& hm, double& s1m, double& s2m)
 {
-    const Recip d = recip<FAST>(h);
-    return CellVel{quot<FAST>(hu, d), quot<FAST>(hv, d), root<FAST>(g * h), d.y};
-}
-
-// Speeds s1m, s2m of riemanntype's middle state (geoclaw_riemann_utils.f:
-// 566-677, maxiter = 1) for two depths above drytol.  rL, rR: the depths with
-// their reciprocals; sgL, sgR = sqrt(g*hL), sqrt(g*hR): every sqrt(g*h) of hL,
-// hR, h_min or h_max is one of them, bit for bit.
-template <bool FAST>
-__device__ __forceinline__ void middle_speeds(const Recip& rL, const Recip& rR, double uL, double uR, double sgL,
-                                              double sgR, const Params& P, double& s1m, double& s2m)
-{
-    const double hL = rL.b, hR = rR.b, g = P.grav, halfg = P.halfg;
-    const bool left = !(hR > hL);  // the left depth is the larger, or they are equal
-    const double h_min = left ? hR : hL;
-    const double h_max = left ? hL : hR;
-    const double dh = h_max - h_min;
+    const double h_min = fminf64(hR, hL);
+    const double h_max = fmaxf64(hR, hL);
+    const double sg_min = hR < hL ? sgR : sgL;  // sqrt(g * h_min)
+    const double sg_max = hR > hL ? sgR : sgL;  // sqrt(g * h_max)
     const double delu = uR - uL;
-    const double F_min = delu + 2.0 * ((left ? sgR : sgL) - (left ? sgL : sgR));
-    const double F_max = delu + dh * root<FAST>(quot<FAST>(halfg * (h_max + h_min), h_max * h_min));
-    // two rarefactions and the shock-rarefaction pair are formed by every lane,
-    // the two-shock case by the lanes that have it: a branch costs a wave more
-    // than the few instructions of the first two
-    const bool rare = F_min > 0.0, shocks = !rare && F_max <= 0.0;
-    // F0 = delu + 2(sqrt(g h0) - sqrt(g h_max)) + (h0 - h_min) sqrt(g/2 (1/h0 + 1/h_min))
-    // at h0 = h_min: the last product is (+0) times a finite positive
-    // whenever g/h_min cannot overflow, so F0 is F_min + 0.0 exactly
-    const double F0 = FAST || (h_min >= 1e-150 && g <= 1e150)
-                          ? F_min
-                          : F_min + 0.0 * sqrt(halfg * (1 / h_min + 1 / h_min));
-    const double tr = vmax<FAST>(0.0, -delu + 2.0 * (sgL + sgR));
-    double hm = rare ? P.inv16g * (tr * tr) : h_min - quot<FAST>(F0, quot<FAST>(F_max - F0, dh));
-    double u1m = 0.0, u2m = 0.0;
-    if (shocks) {
-        // one Newton step on sqrt(h) from h0 = h_max.  The side at h0 has a zero
-        // (h0 - h) factor: only the other side's terms remain, and 1/h0 is that
-        // side's own 1/h
-        const double i_max = quot<FAST>(1.0, left ? rL : rR);
-        const double i_min = quot<FAST>(1.0, left ? rR : rL);
-        const double gs = root<FAST>(halfg * (i_max + i_max));
-        const double go = root<FAST>(halfg * (i_max + i_min));
-        const double F0s = delu + dh * go;
-        const double T = quot<FAST>(g * dh, 4.0 * (h_max * h_max) * go);
-        const double dfdh = left ? (gs + go) - T : (go - T) + gs;
-        const double rh = root<FAST>(h_max);
-        const double slope = 2.0 * rh * dfdh;
-        const double t = rh - quot<FAST>(F0s, slope);
-        hm = t * t;
-        const double im = quot<FAST>(1.0, hm);
-        u1m = uL - (hm - hL) * root<FAST>(halfg * (im + (left ? i_max : i_min)));
-        u2m = uR + (hm - hR) * root<FAST>(halfg * (im + (left ? i_min : i_max)));
+    if (h_min <= drytol) {
+        hm = 0.0;
+        s1m = uR + uL - 2.0 * sgR + 2.0 * sgL;
+        s2m = s1m;
+        return;
     }
-    const double sghm = root<FAST>(g * hm);
+    const double F_min = delu + 2.0 * (sg_min - sg_max);
+    const double F_max = delu + (h_max - h_min) * (sqrt(halfg * (h_max + h_min) / (h_max * h_min)));
+    // The three branches leave hm (and, for two shocks, u1m, u2m); sqrt(g*hm)
+    // and the speeds are formed once after them, so that a wave whose lanes
+    // take different branches pays for the shared part only once.
+    double u1m = 0.0, u2m = 0.0;
+    int kind;  // 0: two rarefactions, 1: two shocks, 2: one shock, one rarefaction
+    if (F_min > 0.0) {
+        const double t = fmaxf64(0.0, -delu + 2.0 * (sgL + sgR));
+        hm = inv16g * (t * t);
+        kind = 0;
+    } else if (F_max <= 0.0) {  // one Newton step on sqrt(h)
+        double h0 = h_max;
+        const double gL = sqrt(halfg * (1 / h0 + 1 / hL));
+        const double gR = sqrt(halfg * (1 / h0 + 1 / hR));
+        const double F0 = delu + (h0 - hL) * gL + (h0 - hR) * gR;
+        const double dfdh = gL - g * (h0 - hL) / (4.0 * (h0 * h0) * gL) + gR -
+                            g * (h0 - hR) / (4.0 * (h0 * h0) * gR);
+        const double slope = 2.0 * sqrt(h0) * dfdh;
+        const double t = sqrt(h0) - F0 / slope;
+        h0 = t * t;
+        hm = h0;
+        u1m = uL - (hm - hL) * sqrt(halfg * (1 / hm + 1 / hL));
+        u2m = uR + (hm - hR) * sqrt(halfg * (1 / hm + 1 / hR));
+        kind = 1;
+    } else {
+        // F0 = delu + 2(sqrt(g h0) - sqrt(g h_max)) + (h0 - h_min) sqrt(g/2 (1/h0 + 1/h_min))
+        // at h0 = h_min: the last product is (+0) times a finite positive
+        // whenever g/h_min cannot overflow, so F0 is F_min + 0.0 exactly
+        double h0 = h_min;
+        const double F0 = (h_min >= 1e-150 && g <= 1e150)
+                              ? F_min + 0.0
+                              : delu + 2.0 * (sg_min - sg_max) + (h0 - h_min) * sqrt(halfg * (1 / h0 + 1 / h_min));
+        const double slope = (F_max - F0) / (h_max - h_min);
+        h0 = h0 - F0 / slope;
+        hm = h0;
+        kind = 2;
+    }
+    const double sghm = sqrt(g * hm);
     // two rarefactions:      s1m = (uL + 2 sqrt(g hL)) - 3 sghm, s2m = (uR - 2 sqrt(g hR)) + 3 sghm
     // shock-rarefaction:     hL > hR: a = uL + 2 sqrt(g hL), s1m = a - 3 sghm, s2m = a - sghm
     //                        else:    a = uR - 2 sqrt(g hR), s2m = a + 3 sghm, s1m = a + sghm
     // two shocks:            s1m = u1m - sghm, s2m = u2m + sghm
     const double A = uL + 2.0 * sgL, B = uR - 2.0 * sgR, s3 = 3.0 * sghm;
-    const bool fromL = hL > hR;
-    s1m = shocks ? u1m - sghm : (rare || fromL) ? A - s3 : B + sghm;
-    s2m = shocks ? u2m + sghm : (rare || !fromL) ? B + s3 : A - sghm;
+    if (kind == 1) {
+        s1m = u1m - sghm;
+        s2m = u2m + sghm;
+    } else if (kind == 0 || hL > hR) {
+        s1m = A - s3;
+        s2m = kind == 0 ? B + s3 : A - sghm;
+    } else {
+        s1m = B + sghm;
+        s2m = B + s3;
+    }
 }
 
-// hm of riemanntype(h, h, u, -u), h > drytol, the wall test of rpn2
-// (rpn2_geoclaw.f:185-242), whose speeds the caller does not use.  With
-// hL = hR = h every (h_max - h_min) factor is an exact +0: F_min = F_max =
-// delu, a positive F takes the two-rarefaction branch and any other the
-// two-shock branch with gL = gR and dfdh = gL + gL.
-template <bool FAST>
-__device__ __forceinline__ double wall_hstar(const Recip& r, double u, double sg, const Params& P)
+// hm of riemanntype(h, h, u, -u), the wall test of rpn2 (rpn2_geoclaw.f:
+// 185-242), whose speeds the caller does not use.  With hL = hR = h every
+// (h_max - h_min) factor is an exact +0: F_min = F_max = delu + 0.0, a
+// positive F takes the two-rarefaction branch and any other the two-shock
+// branch with gL = gR and dfdh = gL + gL.  Outside the range where those
+// zeros are exact (g/h overflowing) the general routine is used.
+__device__ __forceinline__ double wall_hstar(double h, double u, double sg, double drytol, double g, double halfg, double inv16g)
 {
-    const double delu = -u - u;
-    if (delu > 0.0) {
-        const double t = vmax<FAST>(0.0, -delu + 2.0 * (sg + sg));
-        return P.inv16g * (t * t);
+    if (!(h >= 1e-150 && g <= 1e150) || h <= drytol) {
+        double hm, s1m, s2m;
+        riemanntype(h, h, u, -u, sg, sg, drytol, g, halfg, inv16g, hm, s1m, s2m);
+        return hm;
     }
-    // (where g/h overflows the zero factor is not exact, and the reference's
-    // F_max can be NaN, which takes its third branch to a NaN depth)
-    if (!FAST && !(r.b >= 1e-150 && P.grav <= 1e150) &&
-        !(delu + 0.0 * sqrt(P.halfg * (r.b + r.b) / (r.b * r.b)) <= 0.0))
-        return __longlong_as_double(0x7ff8000000000000ll);
-    const double ih = quot<FAST>(1.0, r);
-    const double gL = root<FAST>(P.halfg * (ih + ih));
-    const double rh = root<FAST>(r.b);
-    const double slope = 2.0 * rh * (gL + gL);
-    const double t = rh - quot<FAST>(delu, slope);
+    const double delu = -u - u;
+    const double F = delu + 0.0;
+    if (F > 0.0) {
+        const double t = fmaxf64(0.0, -delu + 2.0 * (sg + sg));
+        return inv16g * (t * t);
+    }
+    const double gL = sqrt(halfg * (1 / h + 1 / h));
+    const double F0 = (delu + 0.0) + 0.0;
+    const double dfdh = gL + gL;
+    const double slope = 2.0 * sqrt(h) * dfdh;
+    const double t = sqrt(h) - F0 / slope;
     return t * t;
 }
 
 // One face of rpn2 (rpn2_geoclaw.f:84-330) followed by riemann_aug_JCP
 // (geoclaw_riemann_utils.f:2-311, maxiter = 1, no rarefaction corrector).
-// Inputs are the left/right states in direction-local order (h, normal
-// momentum, transverse momentum) and the left/right bathymetry.  Outputs: the
-// speeds s[3] and the f-waves in compressed form, wave 1 (3), the normal
-// momentum of wave 2, wave 3 (3): the other two components of wave 2 are exact
-// zeros (geoclaw_riemann_utils.f:289-299: fw(1,2) = beta(2)*r(2,2) = 0,
-// fw(3,2) = 0).  A face with both sides dry gives zeros, as the reference
-// leaves them.  cL, cR: the two cells' velocities, sqrt(g h) and reciprocal
-// depth, used where the cell is wet.
-template <bool FAST>
-__device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, double bL,
+// Inputs are the left/right states in direction-local order and the left/right
+// bathymetry.  Outputs: speeds s[3] and f-waves w[mw][k] with k in
+// direction-local order.  Returns false when both sides are dry (the
+// reference leaves s and the f-waves at zero).
+__device__ __forceinline__ bool rpn2_face(double hL, double huL, double hvL, double bL,
                                           double hR, double huR, double hvR, double bR,
-                                          const CellVel& cL, const CellVel& cR,
-                                          const Params& P, double s[3], double w[7])
+                                          const Params& P,
+                                          double s[3], double w[3][3])
 {
     const double g = P.grav, drytol = P.dry_tolerance, halfg = P.halfg;
-    const bool wetL = hL > drytol, wetR = hR > drytol;
-    const bool still = hL <= drytol && hR <= drytol;
-    // Both sides as if wet; the lanes of a wave that have a dry side are put
-    // right below, in code that the other waves skip.
-    Recip rL{hL, cL.y}, rR{hR, cR.y};
-    double uL = cL.u, vL = cL.v, sgL = cL.sg, uR = cR.u, vR = cR.v, sgR = cR.sg;
-    double phiL = halfg * (hL * hL) + quot<FAST>(huL * huL, rL);
-    double phiR = halfg * (hR * hR) + quot<FAST>(huR * huR, rR);
-    const bool front = !(wetL && wetR);
-    bool wallL = false, wallR = false;
-    if (front) {
-        if (!wetL) {
-            hL = 0.0; huL = 0.0; hvL = 0.0; uL = 0.0; vL = 0.0; phiL = 0.0; sgL = 0.0;
+    if (hL <= drytol && hR <= drytol) {
+#pragma unroll
+        for (int mw = 0; mw < 3; mw++) {
+            s[mw] = 0.0;
+            w[mw][0] = 0.0; w[mw][1] = 0.0; w[mw][2] = 0.0;
         }
-        if (!wetR) {
-            hR = 0.0; huR = 0.0; hvR = 0.0; uR = 0.0; vR = 0.0; phiR = 0.0; sgR = 0.0;
+        return false;
+    }
+    double uR, vR, phiR, uL, vL, phiL;
+    if (hR > drytol) {
+        uR = huR / hR;
+        vR = hvR / hR;
+        phiR = halfg * (hR * hR) + (huR * huR) / hR;
+    } else {
+        hR = 0.0; huR = 0.0; hvR = 0.0; uR = 0.0; vR = 0.0; phiR = 0.0;
+    }
+    if (hL > drytol) {
+        uL = huL / hL;
+        vL = hvL / hL;
+        phiL = halfg * (hL * hL) + (huL * huL) / hL;
+    } else {
+        hL = 0.0; huL = 0.0; hvL = 0.0; uL = 0.0; vL = 0.0; phiL = 0.0;
+    }
+
+    double wall0 = 1.0, wall1 = 1.0, wall2 = 1.0;
+    // the wall test of whichever side is dry: riemanntype(hL, hL, uL, -uL) or
+    // riemanntype(hR, hR, -uR, uR), one call for both kinds of lane
+    double hstar = 0.0;
+    if (hR <= drytol || hL <= drytol) {
+        const double hw = hR <= drytol ? hL : hR;
+        const double uw = hR <= drytol ? uL : -uR;
+        hstar = wall_hstar(hw, uw, sqrt(g * hw), drytol, g, halfg, P.inv16g);
+    }
+    if (hR <= drytol) {
+        const double hstartest = fmaxf64(hL, hstar);
+        if (hstartest + bL < bR) {
+            wall1 = 0.0; wall2 = 0.0;
+            hR = hL; huR = -huL; bR = bL; phiR = phiL; uR = -uL; vR = vL;
+        } else if (hL + bL < bR) {
+            bR = hL + bL;
         }
-        // the wall test of whichever side is dry: riemanntype(hL, hL, uL, -uL) or
-        // riemanntype(hR, hR, -uR, uR), one call for both kinds of lane; a dry
-        // side that the water cannot climb is a wall (the wet side mirrored)
-        const double hstar = wall_hstar<FAST>(wetL ? rL : rR, wetL ? uL : -uR, wetL ? sgL : sgR, P);
-        if (!wetR) {
-            const double hstartest = fmaxf64(hL, hstar);
-            if (hstartest + bL < bR) {
-                wallR = true;
-                hR = hL; huR = -huL; bR = bL; phiR = phiL; uR = -uL; vR = vL; sgR = sgL; rR = rL;
-            } else if (hL + bL < bR) {
-                bR = hL + bL;
-            }
-        } else {
-            const double hstartest = fmaxf64(hR, hstar);
-            if (hstartest + bR < bL) {
-                wallL = true;
-                hL = hR; huL = -huR; bL = bR; phiL = phiR; uL = -uR; vL = vR; sgL = sgR; rL = rR;
-            } else if (hR + bR < bL) {
-                bL = hR + bR;
-            }
+    } else if (hL <= drytol) {
+        const double hstartest = fmaxf64(hR, hstar);
+        if (hstartest + bR < bL) {
+            wall0 = 0.0; wall1 = 0.0;
+            hL = hR; huL = -huR; bL = bR; phiL = phiR; uL = -uR; vL = vR;
+        } else if (hR + bR < bL) {
+            bL = hR + bR;
         }
     }
 
-    const double sL = uL - sgL;
-    const double sR = uR + sgR;
-    const double uhat = quot<FAST>(sgL * uL + sgR * uR, sgR + sgL);
-    const double chat = root<FAST>(halfg * (hR + hL));
+    const double sghL = sqrt(g * hL);
+    const double sghR = sqrt(g * hR);
+    const double sL = uL - sghL;
+    const double sR = uR + sghR;
+    const double uhat = (sghL * uL + sghR * uR) / (sghR + sghL);
+    const double chat = sqrt(halfg * (hR + hL));
     const double sRoe1 = uhat - chat;
     const double sRoe2 = uhat + chat;
+    double sE1 = fminf64(sL, sRoe1);
+    double sE2 = fmaxf64(sR, sRoe2);
 
     // ---- riemann_aug_JCP ----
     const double delh = hR - hL;
@@ -217,224 +226,215 @@ __device__ __forceinline__ void rpn2_face(double hL, double huL, double hvL, dou
     const double delphi = phiR - phiL;
     const double delb = bR - bL;
 
-    double s1m, s2m;
-    middle_speeds<FAST>(rL, rR, uL, uR, sgL, sgR, P, s1m, s2m);
-    if (front && fminf64(hR, hL) <= drytol) {
-        s1m = uR + uL - 2.0 * sgR + 2.0 * sgL;
-        s2m = s1m;
-    }
+    double hm, s1m, s2m;
+    riemanntype(hL, hR, uL, uR, sghL, sghR, drytol, g, halfg, P.inv16g, hm, s1m, s2m);
 
-    // (the sign of a zero speed matters to the limiter; in the fast range these
-    // are sums, whose zeros are all +0)
-    const double sE1 = vmin<FAST>(vmin<FAST>(sL, sRoe1), s2m);
-    const double sE2 = vmax<FAST>(vmax<FAST>(sR, sRoe2), s1m);
-    const double lam0 = sE1, lam2 = sE2;
+    const double lam0 = fminf64(sE1, s2m);
+    const double lam2 = fmaxf64(sE2, s1m);
+    sE1 = lam0;
+    sE2 = lam2;
+    const double hstarHLL = fmaxf64((huL - huR + sE2 * hR - sE1 * hL) / (sE2 - sE1), 0.0);
     const double lam1 = 0.5 * (lam0 + lam2);
+
     // r(:,1) = (1, lam0, lam0^2), r(:,2) = (0, 0, 1), r(:,3) = (1, lam2, lam2^2)
     const double r10 = lam0, r20 = lam0 * lam0;
     const double r12 = lam2, r22 = lam2 * lam2;
 
-    // a level bed has delb = 0, and with it deldelh = deldelphi = 0 whatever
-    // the bounds below (each lies on the other side of 0)
-    double deldelh = 0.0, deldelphi = 0.0;
-    if (!FAST || delb != 0.0) {
-        const double hstarHLL = vmax<FAST>(quot<FAST>(huL - huR + sE2 * hR - sE1 * hL, sE2 - sE1), 0.0);
-        const double crit = P.crit, crit2 = P.crit2;
-        const double hbar = vmax<FAST>(0.5 * (hL + hR), 0.0);
-        const double tu = uL + uR;
-        const double s1s2bar = 0.25 * (tu * tu) - g * hbar;
-        const double s1s2tilde = vmax<FAST>(0.0, uL * uR) - g * hbar;
-        const bool sonic = (fabs(s1s2bar) <= crit) | (s1s2bar * s1s2tilde <= P.critsq) |
-                           (s1s2bar * sE1 * sE2 <= P.critsq) | (vmin<FAST>(fabs(sE1), fabs(sE2)) < crit2) |
-                           ((sE1 < crit2) & (s1m > -crit2)) | ((sE2 > -crit2) & (s2m < crit2)) |
-                           ((uL + sgL) * (uR + sgR) < 0.0) | ((uL - sgL) * (uR - sgR) < 0.0);
-        const Recip rb = recip<FAST>(s1s2bar);
-        const double gb = delb * g * hbar, gn = -delb * g * hbar;
-        deldelh = sonic ? -delb : quot<FAST>(gb, rb);
-        // the bounds' two quotients are formed once for every lane (the three
-        // cases use them in different combinations)
-        const double hs = hstarHLL * (sE2 - sE1);
-        const double q2 = quot<FAST>(hs, sE2);
-        const double q1 = quot<FAST>(hs, sE1);
-        const bool sub = sE1 < -crit && sE2 > crit, right = !sub && sE1 >= crit, left = !sub && !right && sE2 <= -crit;
-        const double upper = sub ? q2 : right ? q1 : hR, lower = sub ? q1 : right ? -hL : q2;
-        const double bounded = vmax<FAST>(vmin<FAST>(deldelh, upper), lower);
-        deldelh = (sub || right || left) ? bounded : deldelh;
-        deldelphi = sonic ? -g * hbar * delb : quot<FAST>(gn * s1s2tilde, rb);
-        deldelphi = vmin<FAST>(deldelphi, g * vmax<FAST>(-hL * delb, -hR * delb));
-        deldelphi = vmax<FAST>(deldelphi, g * vmin<FAST>(-hL * delb, -hR * delb));
+    const double criticaltol = P.crit;
+    const double criticaltol_2 = P.crit2;
+
+    const double hbar = fmaxf64(0.5 * (hL + hR), 0.0);
+    const double tu = uL + uR;
+    const double s1s2bar = 0.25 * (tu * tu) - g * hbar;
+    const double s1s2tilde = fmaxf64(0.0, uL * uR) - g * hbar;
+
+    bool sonic;
+    if (fabs(s1s2bar) <= criticaltol) sonic = true;
+    else if (s1s2bar * s1s2tilde <= P.critsq) sonic = true;
+    else if (s1s2bar * sE1 * sE2 <= P.critsq) sonic = true;
+    else if (fminf64(fabs(sE1), fabs(sE2)) < criticaltol_2) sonic = true;
+    else if (sE1 < criticaltol_2 && s1m > -criticaltol_2) sonic = true;
+    else if (sE2 > -criticaltol_2 && s2m < criticaltol_2) sonic = true;
+    else if ((uL + sghL) * (uR + sghR) < 0.0) sonic = true;
+    else if ((uL - sghL) * (uR - sghR) < 0.0) sonic = true;
+    else sonic = false;
+
+    double deldelh = sonic ? -delb : delb * g * hbar / s1s2bar;
+    // the bounds' two quotients are formed once for every lane (the three
+    // cases use them in different combinations)
+    const double q2 = hstarHLL * (sE2 - sE1) / sE2;
+    const double q1 = hstarHLL * (sE2 - sE1) / sE1;
+    if (sE1 < -criticaltol && sE2 > criticaltol) {
+        deldelh = fminf64(deldelh, q2);
+        deldelh = fmaxf64(deldelh, q1);
+    } else if (sE1 >= criticaltol) {
+        deldelh = fminf64(deldelh, q1);
+        deldelh = fmaxf64(deldelh, -hL);
+    } else if (sE2 <= -criticaltol) {
+        deldelh = fminf64(deldelh, hR);
+        deldelh = fmaxf64(deldelh, q2);
     }
+    double deldelphi = sonic ? -g * hbar * delb : -delb * g * hbar * s1s2tilde / s1s2bar;
+    deldelphi = fminf64(deldelphi, g * fmaxf64(-hL * delb, -hR * delb));
+    deldelphi = fmaxf64(deldelphi, g * fminf64(-hL * delb, -hR * delb));
 
     const double d0 = delh - deldelh;
     const double d1 = delhu;
     const double d2 = delphi - deldelphi;
 
-    // Cramer's rule as the reference writes it (geoclaw_riemann_utils.f:230-249)
-    // with r = [[1,0,1],[r10,0,r12],[r20,1,r22]], its zero terms left out
-    const Recip det = recip<FAST>(r10 - r12);
-    const double beta0 = quot<FAST>(d1 - d0 * r12, det);
-    const double beta1 = quot<FAST>(((d1 * r22 - r12 * d2) - d0 * (r10 * r22 - r12 * r20)) + (r10 * d2 - d1 * r20), det);
-    const double beta2 = quot<FAST>(d0 * r10 - d1, det);
+    // Cramer's rule exactly as the reference writes it (geoclaw_riemann_utils.f:230-249)
+    // with r = [[1,0,1],[r10,0,r12],[r20,1,r22]].
+    double det1 = 1.0 * (0.0 * r22 - r12 * 1.0);
+    double det2 = 0.0 * (r10 * r22 - r12 * r20);
+    double det3 = 1.0 * (r10 * 1.0 - 0.0 * r20);
+    const double determinant = det1 - det2 + det3;
+    double beta0, beta1, beta2;
+    det1 = d0 * (0.0 * r22 - r12 * 1.0);
+    det2 = 0.0 * (d1 * r22 - r12 * d2);
+    det3 = 1.0 * (d1 * 1.0 - 0.0 * d2);
+    beta0 = (det1 - det2 + det3) / determinant;
+    det1 = 1.0 * (d1 * r22 - r12 * d2);
+    det2 = d0 * (r10 * r22 - r12 * r20);
+    det3 = 1.0 * (r10 * d2 - d1 * r20);
+    beta1 = (det1 - det2 + det3) / determinant;
+    det1 = 1.0 * (0.0 * d2 - d1 * 1.0);
+    det2 = 0.0 * (r10 * d2 - d1 * r20);
+    det3 = d0 * (r10 * 1.0 - 0.0 * r20);
+    beta2 = (det1 - det2 + det3) / determinant;
 
     // f-waves (geoclaw_riemann_utils.f:289-306)
-    const double fw00 = beta0 * r10, fw20 = beta2 * r12;
-    double fw02 = fw00 * vL, fw22 = fw20 * vR;
-    const double rest = hR * uR * vR - hL * uL * vL - fw02 - fw22;
-    const bool below = huL + fw00 <= 0.0;
-    fw02 = below ? fw02 + rest : fw02;
-    fw22 = below ? fw22 : fw22 + rest;
+    double fw00 = beta0 * r10, fw01 = beta0 * r20, fw02 = beta0 * r10;
+    double fw10 = beta1 * 0.0, fw11 = beta1 * 1.0, fw12;
+    double fw20 = beta2 * r12, fw21 = beta2 * r22, fw22 = beta2 * r12;
+    fw02 = fw02 * vL;
+    fw22 = fw22 * vR;
+    fw12 = 0.0;
+    const double hustar_interface = huL + fw00;
+    if (hustar_interface <= 0.0)
+        fw02 = fw02 + (hR * uR * vR - hL * uL * vL - fw02 - fw22);
+    else
+        fw22 = fw22 + (hR * uR * vR - hL * uL * vL - fw02 - fw22);
 
-    s[0] = lam0; s[1] = lam1; s[2] = lam2;
-    w[0] = fw00; w[1] = beta0 * r20; w[2] = fw02;
-    w[3] = beta1;
-    w[4] = fw20; w[5] = beta2 * r22; w[6] = fw22;
-    if (front) {
-        // eliminate ghost fluxes for the wall problem (rpn2_geoclaw.f:303-309);
-        // no waves between dry cells (there the products are of garbage)
-        const double w0 = wallL ? 0.0 : 1.0, w1 = wallL || wallR ? 0.0 : 1.0, w2 = wallR ? 0.0 : 1.0;
-        const double f[3] = {w0, w1, w2};
-#pragma unroll
-        for (int k = 0; k < 3; k++) s[k] = still ? 0.0 : s[k] * f[k];
-#pragma unroll
-        for (int k = 0; k < 7; k++) w[k] = still ? 0.0 : w[k] * f[k / 3 < 1 ? 0 : (k == 3 ? 1 : 2)];
-    }
+    // eliminate ghost fluxes for the wall problem (rpn2_geoclaw.f:303-309)
+    s[0] = lam0 * wall0;
+    s[1] = lam1 * wall1;
+    s[2] = lam2 * wall2;
+    w[0][0] = fw00 * wall0; w[0][1] = fw01 * wall0; w[0][2] = fw02 * wall0;
+    w[1][0] = fw10 * wall1; w[1][1] = fw11 * wall1; w[1][2] = fw12 * wall1;
+    w[2][0] = fw20 * wall2; w[2][1] = fw21 * wall2; w[2][2] = fw22 * wall2;
+    return true;
 }
 
-// Fluctuations of one face (rpn2_geoclaw.f:359-376) from its compressed
-// waves, direction-local order: a wave goes to amdq when its speed is
-// negative, to apdq when it is positive and half to each at zero, i.e. times
-// 1, 1/2 or 0 to each (exact products).
-__device__ __forceinline__ void fluctuations(const double s[3], const double w[7], double amdq[3], double apdq[3])
+// Fluctuations of one face (rpn2_geoclaw.f:359-376), direction-local order.
+__device__ __forceinline__ void fluctuations(const double s[3], const double w[3][3],
+                                             double amdq[3], double apdq[3])
 {
-    double cm[3], cp[3];
+    amdq[0] = 0.0; amdq[1] = 0.0; amdq[2] = 0.0;
+    apdq[0] = 0.0; apdq[1] = 0.0; apdq[2] = 0.0;
 #pragma unroll
     for (int mw = 0; mw < 3; mw++) {
-        cm[mw] = s[mw] < 0.0 ? 1.0 : (s[mw] > 0.0 ? 0.0 : 0.5);
-        cp[mw] = 1.0 - cm[mw];
+        if (s[mw] < 0.0) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) amdq[k] = amdq[k] + w[mw][k];
+        } else if (s[mw] > 0.0) {
+#pragma unroll
+            for (int k = 0; k < 3; k++) apdq[k] = apdq[k] + w[mw][k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                amdq[k] = amdq[k] + 0.5 * w[mw][k];
+                apdq[k] = apdq[k] + 0.5 * w[mw][k];
+            }
+        }
     }
-    amdq[0] = cm[0] * w[0] + cm[2] * w[4];
-    amdq[1] = cm[0] * w[1] + cm[1] * w[3] + cm[2] * w[5];
-    amdq[2] = cm[0] * w[2] + cm[2] * w[6];
-    apdq[0] = cp[0] * w[0] + cp[2] * w[4];
-    apdq[1] = cp[0] * w[1] + cp[1] * w[3] + cp[2] * w[5];
-    apdq[2] = cp[0] * w[2] + cp[2] * w[6];
 }
 
-// The limiter function of philim (philim.f:65-126) at the ratio r = b / a,
-// a != 0; an out-of-range method falls through to minmod.
-template <bool FAST>
-__device__ __forceinline__ double philim(double r, int meth)
+// philim (philim.f:65-126); an out-of-range method falls through to minmod.
+__device__ __forceinline__ double philim(double a, double b, int meth)
 {
+    if (a == 0.0) return 0.0;
+    const double r = b / a;
     switch (meth) {
     case 2:
-        return vmax<FAST>(vmax<FAST>(0.0, vmin<FAST>(1.0, 2.0 * r)), vmin<FAST>(2.0, r));
+        return fmaxf64(fmaxf64(0.0, fminf64(1.0, 2.0 * r)), fminf64(2.0, r));
     case 3:
         return (r + fabs(r)) / (1.0 + fabs(r));
     case 4: {
         const double c = (1.0 + r) / 2.0;
-        return vmax<FAST>(0.0, vmin<FAST>(vmin<FAST>(c, 2.0), 2.0 * r));
+        return fmaxf64(0.0, fminf64(fminf64(c, 2.0), 2.0 * r));
     }
     case 5:
         return r;
     default:
-        return vmax<FAST>(0.0, vmin<FAST>(1.0, r));
+        return fmaxf64(0.0, fminf64(1.0, r));
     }
-}
-
-// Some non-zero value of the N is too small for quot<true> as a numerator or
-// denominator (gf_exact.h).
-template <int N>
-__device__ __forceinline__ bool quotients_tiny(const double (&a)[N])
-{
-    int e = 0;
-#pragma unroll
-    for (int k = 0; k < N; k++) {
-        const int x = exponent_of(a[k]);
-        e = x < e ? x : e;
-    }
-    return e < QUOT_MIN_EXP;
 }
 
 // Eigen-split of a transverse fluctuation for one cell (rpt2_geoclaw.f:61-187):
-// the cell's velocities (u normal, v transverse with respect to the normal
-// solve), its surface eta = h + b and the bathymetry of its two transverse
-// neighbours.  The split is applied to two fluctuations (the imp = 1 split of
-// amdq of the face on the cell's right/top and the imp = 2 split of apdq of
-// the face on its left/bottom share the same Jacobian).
+// the cell's state (h, un, vt in direction-local order with respect to the
+// normal solve), its surface eta = h + b and the bathymetry of its two
+// transverse neighbours.  Applies the split to two fluctuations at once (the
+// imp = 1 split of amdq of the face on the cell's right/top and the imp = 2
+// split of apdq of the face on its left/bottom share the same Jacobian).
 struct Rpt2Cell {
-    bool active, lo, hi;  // lo / hi: the surface reaches the neighbour below / above
-    double u, s0, s1, s2;
+    bool active;
+    double u, s0, s1, s2, eta, topo1, topo3;
 };
 
-template <bool FAST>
-__device__ __forceinline__ Rpt2Cell rpt2_setup(double h, double u, double v, double sg, double b,
-                                               double topo1, double topo3, double tol)
+__device__ __forceinline__ Rpt2Cell rpt2_setup(double h, double hun, double hvt, double b,
+                                               double topo1, double topo3, double g, double tol)
 {
     Rpt2Cell c;
+    c.active = false;
+    c.u = 0.0; c.s0 = 0.0; c.s1 = 0.0; c.s2 = 0.0; c.eta = 0.0; c.topo1 = topo1; c.topo3 = topo3;
+    if (h <= tol) return c;
+    const double u = hun / h;
+    const double v = hvt / h;
     const double eta = h + b;
-    c.active = !(h <= tol) && !(eta < vmin<FAST>(topo1, topo3));
-    c.lo = eta >= topo1;
-    c.hi = eta >= topo3;
+    if (eta < fminf64(topo1, topo3)) return c;
+    const double sgh = sqrt(g * h);
+    c.active = true;
     c.u = u;
-    c.s0 = v - sg;
+    c.s0 = v - sgh;
     c.s1 = v;
-    c.s2 = v + sg;
+    c.s2 = v + sgh;
+    c.eta = eta;
     return c;
 }
 
-// One side's sum over the waves of speed * beta * r with r(:,1) = (1, u, s0),
-// r(:,2) = (0, 1, 0), r(:,3) = (1, u, s2); sp is 0 for a wave that does not
-// go there.
-__device__ __forceinline__ void rpt2_side(const double sp[3], const double beta[3], const Rpt2Cell& c, double out[3])
+// bmasdq/bpasdq in direction-local order for one asdq.
+__device__ __forceinline__ void rpt2_apply(const Rpt2Cell& c, const double asdq[3],
+                                           double bm[3], double bp[3])
 {
-    const double t0 = sp[0] * beta[0], t1 = sp[1] * beta[1], t2 = sp[2] * beta[2];
-    out[0] = t0 + t2;
-    out[1] = t0 * c.u + t1 + t2 * c.u;
-    out[2] = t0 * c.s0 + t2 * c.s2;
-}
-
-// Transverse increments of one cell from the two normal fluctuations that its
-// state splits (geoclaw_flux2fw_fort.f:232-265): G1 (below/left) and G2
-// (above/right), direction-local order, hd = dt/dx / 2.
-template <bool FAST>
-__device__ __forceinline__ void cell_transverse(const Rpt2Cell& c, const double am_next[3], const double ap_own[3],
-                                                double hd, double G1[3], double G2[3])
-{
-#pragma unroll
-    for (int k = 0; k < 3; k++) { G1[k] = 0.0; G2[k] = 0.0; }
+    bm[0] = 0.0; bm[1] = 0.0; bm[2] = 0.0;
+    bp[0] = 0.0; bp[1] = 0.0; bp[2] = 0.0;
     if (!c.active) return;
-    const double den = c.s2 - c.s0;
-    const double n[4] = {c.s2 * am_next[0] - am_next[2], am_next[2] - c.s0 * am_next[0],
-                         c.s2 * ap_own[0] - ap_own[2], ap_own[2] - c.s0 * ap_own[0]};
-    double be[4];
-    const Recip r = recip<FAST>(den);
+    const double delf1 = asdq[0], delf2 = asdq[1], delf3 = asdq[2];
+    const double beta0 = (c.s2 * delf1 - delf3) / (c.s2 - c.s0);
+    const double beta1 = -c.u * delf1 + delf2;
+    const double beta2 = (delf3 - c.s0 * delf1) / (c.s2 - c.s0);
+    const double sv[3] = {c.s0, c.s1, c.s2};
+    const double bv[3] = {beta0, beta1, beta2};
+    // r(:,1) = (1, u, s0), r(:,2) = (0, 1, 0), r(:,3) = (1, u, s2)
+    const double r0[3] = {1.0, 0.0, 1.0};
+    const double r1[3] = {c.u, 1.0, c.u};
+    const double r2[3] = {c.s0, 0.0, c.s2};
 #pragma unroll
-    for (int k = 0; k < 4; k++) be[k] = quot<FAST>(n[k], r);
-    if (FAST && quotients_tiny(n)) {
-#pragma unroll
-        for (int k = 0; k < 4; k++) be[k] = n[k] / den;
+    for (int mw = 0; mw < 3; mw++) {
+        if ((sv[mw] < 0.0) && (c.eta >= c.topo1)) {
+            bm[0] = bm[0] + 1.0 * sv[mw] * bv[mw] * r0[mw];
+            bm[1] = bm[1] + 1.0 * sv[mw] * bv[mw] * r1[mw];
+            bm[2] = bm[2] + 1.0 * sv[mw] * bv[mw] * r2[mw];
+        } else if ((sv[mw] > 0.0) && (c.eta >= c.topo3)) {
+            bp[0] = bp[0] + 1.0 * sv[mw] * bv[mw] * r0[mw];
+            bp[1] = bp[1] + 1.0 * sv[mw] * bv[mw] * r1[mw];
+            bp[2] = bp[2] + 1.0 * sv[mw] * bv[mw] * r2[mw];
+        }
     }
-    const double b1[3] = {be[0], -c.u * am_next[0] + am_next[1], be[1]};
-    const double b2[3] = {be[2], -c.u * ap_own[0] + ap_own[1], be[3]};
-    // the waves that go down are those of negative speed, where the surface
-    // reaches the bed below, and the others count with speed 0; likewise up
-    const double dn[3] = {vmin<FAST>(c.s0, 0.0), vmin<FAST>(c.s1, 0.0), vmin<FAST>(c.s2, 0.0)};
-    const double up[3] = {vmax<FAST>(c.s0, 0.0), vmax<FAST>(c.s1, 0.0), vmax<FAST>(c.s2, 0.0)};
-    const double hlo = c.lo ? hd : 0.0, hhi = c.hi ? hd : 0.0;
-    double d1[3], d2[3];
-    rpt2_side(dn, b1, c, d1);
-    rpt2_side(dn, b2, c, d2);
-#pragma unroll
-    for (int k = 0; k < 3; k++) G1[k] = -(hlo * d1[k]) - hlo * d2[k];
-    rpt2_side(up, b1, c, d1);
-    rpt2_side(up, b2, c, d2);
-#pragma unroll
-    for (int k = 0; k < 3; k++) G2[k] = -(hhi * d1[k]) - hhi * d2[k];
 }
 
 // Manning friction of fc2d_geoclaw_src2 (geoclaw_src2_fort.f90:41-71) for one
 // interior cell; manning_break(1) = rinfinity (default-real 10.e32).
-template <bool FAST>
 __device__ __forceinline__ void src2_cell(double h, double& hu, double& hv, double b,
                                           double dt, const Params& P)
 {
@@ -444,22 +444,121 @@ __device__ __forceinline__ void src2_cell(double h, double& hu, double& hv, doub
         hv = 0.0;
     } else if (h <= P.friction_depth) {
         const double coeff = (b < (double)10.e32f) ? P.manning_n : 0.0;
-        const double c2 = coeff * coeff;
-        const double sq = hu * hu + hv * hv;
-        const double pw = pow_7_3(h);
-        // momenta above 2^-300 and a friction term of ordinary size, or none
-        const double num = root<FAST>(sq) * P.grav * c2;
-        const double lo = vmin<true>(hu == 0.0 ? 1.0 : fabs(hu), hv == 0.0 ? 1.0 : fabs(hv));
-        const Recip d = recip<FAST>(1.0 + dt * quot<FAST>(num, pw));
-        if (FAST && sq < 0x1p600 && lo >= 0x1p-300 && (num >= 0x1p-400 || num == 0.0) && d.b < 0x1p300) {
-            hu = quot<FAST>(hu, d);
-            hv = quot<FAST>(hv, d);
-        } else {
-            const double gamma = sqrt(sq) * P.grav * c2 / pw;
-            const double dgamma = 1.0 + dt * gamma;
-            hu = hu / dgamma;
-            hv = hv / dgamma;
+        const double gamma = sqrt(hu * hu + hv * hv) * P.grav * (coeff * coeff) / pow_7_3(h);
+        const double dgamma = 1.0 + dt * gamma;
+        hu = hu / dgamma;
+        hv = hv / dgamma;
+    }
+}
+
+// Compressed f-waves of one face: wave 1 (3), normal momentum of wave 2 (1),
+// wave 3 (3).  The other two components of wave 2 are exact zeros
+// (geoclaw_riemann_utils.f:289-299: fw(1,2) = beta(2)*r(2,2) = 0, fw(3,2) = 0).
+__device__ __forceinline__ void compress(const double w[3][3], double c[7])
+{
+    c[0] = w[0][0]; c[1] = w[0][1]; c[2] = w[0][2];
+    c[3] = w[1][1];
+    c[4] = w[2][0]; c[5] = w[2][1]; c[6] = w[2][2];
+}
+
+// Dot product of two 3-vectors given in direction-local order (h, n, t),
+// summed in the reference's physical component order (h, hu, hv):
+// x-direction (h, n, t) = (h, hu, hv); y-direction (h, n, t) = (h, hv, hu).
+template <int DIR>
+__device__ __forceinline__ double pdot(const double* a, const double* b)
+{
+    if (DIR == 0) return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
+    return a[0] * b[0] + a[2] * b[2] + a[1] * b[1];
+}
+
+// Limiter, second-order correction and fluctuation split of one face
+// (geoclaw_flux2fw_fort.f:143-224 with geoclaw_limiter_fort.f:34-58 and
+// philim.f).  wc: own compressed unlimited waves; wn: for each wave that of the
+// face before along the sweep when it moves forwards, else of the face after.
+// Outputs in direction-local order: faddm,
+// faddp (flux increments) and amdq*, apdq* (fluctuations handed to rpt2).
+// DEF: the default method (order 2, transverse 2, MC limiter on all three
+// families) fixed at compile time; otherwise the method is read from P.
+template <int DIR, bool DEF>
+__device__ __forceinline__ void face_second_order(const double wc[7], const double s[3],
+                                                  const double wn[7],
+                                                  double dtdx, const Params& P,
+                                                  double faddm[3], double faddp[3],
+                                                  double amq[3], double apq[3])
+{
+    double w[3][3] = {{wc[0], wc[1], wc[2]}, {0.0, wc[3], 0.0}, {wc[4], wc[5], wc[6]}};
+    double amdq[3], apdq[3];
+    fluctuations(s, w, amdq, apdq);
+    const int order = DEF ? 2 : P.order;
+    const int lim0 = DEF ? 4 : P.mthlim[0], lim1 = DEF ? 4 : P.mthlim[1], lim2 = DEF ? 4 : P.mthlim[2];
+    if (order == 1) {
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            faddm[k] = amdq[k];
+            faddp[k] = -apdq[k];
+            amq[k] = amdq[k];
+            apq[k] = apdq[k];
         }
+        return;
+    }
+    // limiter on the three wave families with the unlimited neighbours
+    {
+        // wave 1
+        if (lim0 != 0) {
+            const double wnorm2 = pdot<DIR>(wc, wc);
+            if (wnorm2 != 0.0) {
+                const double lim = philim(wnorm2, pdot<DIR>(wn, wc), lim0);
+                w[0][0] = lim * w[0][0]; w[0][1] = lim * w[0][1]; w[0][2] = lim * w[0][2];
+            }
+        }
+        // wave 2 (only its normal-momentum component is non-zero)
+        if (lim1 != 0) {
+            const double wnorm2 = wc[3] * wc[3];
+            if (wnorm2 != 0.0) {
+                const double lim = philim(wnorm2, wn[3] * wc[3], lim1);
+                w[1][1] = lim * w[1][1];
+            }
+        }
+        // wave 3
+        if (lim2 != 0) {
+            const double wnorm2 = pdot<DIR>(wc + 4, wc + 4);
+            if (wnorm2 != 0.0) {
+                const double lim = philim(wnorm2, pdot<DIR>(wn + 4, wc + 4), lim2);
+                w[2][0] = lim * w[2][0]; w[2][1] = lim * w[2][1]; w[2][2] = lim * w[2][2];
+            }
+        }
+    }
+    double c[3];
+#pragma unroll
+    for (int mw = 0; mw < 3; mw++) c[mw] = copysign(1.0, s[mw]) * (1.0 - fabs(s[mw]) * dtdx);
+    double cq[3];
+    cq[0] = c[0] * w[0][0] + c[2] * w[2][0];
+    cq[1] = c[0] * w[0][1] + c[1] * w[1][1] + c[2] * w[2][1];
+    cq[2] = c[0] * w[0][2] + c[2] * w[2][2];
+    const bool fold = DEF ? true : (P.transverse == 2);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        faddm[k] = amdq[k] + 0.5 * cq[k];
+        faddp[k] = -apdq[k] + 0.5 * cq[k];
+        amq[k] = fold ? amdq[k] + cq[k] : amdq[k];
+        apq[k] = fold ? apdq[k] - cq[k] : apdq[k];
+    }
+}
+
+// Transverse increments of one cell from the two normal fluctuations that
+// its state splits (geoclaw_flux2fw_fort.f:232-265): G1 (below/left) and G2
+// (above/right), direction-local order, hd = dt/dx / 2.
+__device__ __forceinline__ void cell_transverse(const Rpt2Cell& C, const double am_next[3],
+                                                const double ap_own[3], double hd,
+                                                double G1[3], double G2[3])
+{
+    double bm1[3], bp1[3], bm2[3], bp2[3];
+    rpt2_apply(C, am_next, bm1, bp1);
+    rpt2_apply(C, ap_own, bm2, bp2);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        G1[k] = -(hd * bm1[k]) - hd * bm2[k];
+        G2[k] = -(hd * bp1[k]) - hd * bp2[k];
     }
 }
 

@@ -31,6 +31,7 @@
 #include "gf_ghost.h"
 #include "gf_inflow.h"
 #include "gf_launch.h"
+#include "gf_physics_fast.h"
 
 namespace gf {
 
@@ -81,16 +82,6 @@ __device__ __forceinline__ double wave_max_last(double v)
     return max_from<0x143, 0xc>(v);  // row_bcast:31
 }
 
-// Dot product of two 3-vectors given in direction-local order (h, n, t),
-// summed in the reference's physical component order (h, hu, hv):
-// x-direction (h, n, t) = (h, hu, hv); y-direction (h, n, t) = (h, hv, hu).
-template <int DIR>
-__device__ __forceinline__ double pdot(const double* a, const double* b)
-{
-    if (DIR == 0) return a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
-    return a[0] * b[0] + a[2] * b[2] + a[1] * b[1];
-}
-
 // A face's own waves (at) and, wave by wave, the neighbour's that the limiter
 // compares with: the face before (-step) when the wave moves forwards, else the
 // face after.
@@ -108,67 +99,6 @@ __device__ __forceinline__ void load_waves(const double* at, int step, const dou
         wn[4 + k] = n2[(4 + k) * NPOS];
     }
     wn[3] = n1[3 * NPOS];
-}
-
-// Limiter, second-order correction and fluctuation split of one face
-// (geoclaw_flux2fw_fort.f:143-224 with geoclaw_limiter_fort.f:34-58 and
-// philim.f).  w: own compressed unlimited waves; wn: for each wave that of the
-// face it comes from (load_waves).  Outputs in direction-local order: faddm,
-// faddp (flux increments) and amdq*, apdq* (fluctuations handed to rpt2).
-// DEF: the default method (order 2, transverse 2, MC limiter on all three
-// families) fixed at compile time; otherwise the method is read from P.
-template <int DIR, bool DEF, bool FAST>
-__device__ __forceinline__ void face_second_order(const double w[7], const double s[3],
-                                                  const double wn[7], double dtdx, const Params& P,
-                                                  double faddm[3], double faddp[3],
-                                                  double amq[3], double apq[3])
-{
-    double amdq[3], apdq[3];
-    fluctuations(s, w, amdq, apdq);
-    const int order = DEF ? 2 : P.order;
-    if (order == 1) {
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            faddm[k] = amdq[k];
-            faddp[k] = -apdq[k];
-            amq[k] = amdq[k];
-            apq[k] = apdq[k];
-        }
-        return;
-    }
-    // limiter on the three wave families (wave 2 has its normal momentum only):
-    // the ratios b / a of the dot products, then the factor of each family (1
-    // where the wave vanishes or its family is not limited)
-    const double a[3] = {pdot<DIR>(w, w), w[3] * w[3], pdot<DIR>(w + 4, w + 4)};
-    const double b[3] = {pdot<DIR>(wn, w), wn[3] * w[3], pdot<DIR>(wn + 4, w + 4)};
-    double r[3];
-#pragma unroll
-    for (int mw = 0; mw < 3; mw++) r[mw] = quot<FAST>(b[mw], a[mw]);
-    const double ab[6] = {a[0], a[1], a[2], b[0], b[1], b[2]};
-    if (FAST && quotients_tiny(ab)) {
-#pragma unroll
-        for (int mw = 0; mw < 3; mw++) r[mw] = b[mw] / a[mw];
-    }
-    double lim[3], c[3];
-#pragma unroll
-    for (int mw = 0; mw < 3; mw++) {
-        const int meth = DEF ? 4 : P.mthlim[mw];
-        lim[mw] = a[mw] != 0.0 && (DEF || meth != 0) ? philim<FAST>(r[mw], meth) : 1.0;
-        c[mw] = copysign(1.0, s[mw]) * (1.0 - fabs(s[mw]) * dtdx);
-    }
-    double cq[3];
-    cq[0] = c[0] * (lim[0] * w[0]) + c[2] * (lim[2] * w[4]);
-    cq[1] = c[0] * (lim[0] * w[1]) + c[1] * (lim[1] * w[3]) + c[2] * (lim[2] * w[5]);
-    cq[2] = c[0] * (lim[0] * w[2]) + c[2] * (lim[2] * w[6]);
-    const bool fold = DEF ? true : (P.transverse == 2);
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const double hq = 0.5 * cq[k];
-        faddm[k] = amdq[k] + hq;
-        faddp[k] = -apdq[k] + hq;
-        amq[k] = fold ? amdq[k] + cq[k] : amdq[k];
-        apq[k] = fold ? apdq[k] - cq[k] : apdq[k];
-    }
 }
 
 // Maximum over a workgroup of NT threads; the result is valid in thread 0.
@@ -220,7 +150,8 @@ using gint = __attribute__((address_space(1))) int;
 
 // The step of one tile in LDS (T: h, hu, hv, b after b4step2, at least one
 // cell wet), by a group of NT threads; arguments as in step_patch.  FAST: every
-// cell and parameter lies in the range of gf_exact.h.
+// cell and parameter lies in the range of gf_exact.h, and the step takes the
+// forms of gf_physics_fast.h; otherwise the general ones of gf_physics.h.
 template <int MX, int MY, int TX, int TY, int NT, bool DEF, bool FREG, bool FAST, typename Ahead>
 __device__ __forceinline__ void step_tile(const double* T, double* E, double* F, double* red, int ox, int oy,
                                           gdouble* dst, double dtdx, double dtdy, double dt, const Params& P,
@@ -242,12 +173,25 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         pj[s] = p / PX;
     }
 
-    double smax = 0.0;  // largest |s| of the direction's faces: max |s| dt/dx = (max |s|) dt/dx, rounded too
+    double cfl = 0.0;
+    double smax = 0.0;  // FAST: largest |s| of the direction's faces: max |s| dt/dx = (max |s|) dt/dx, rounded too
+    const auto fold_speeds = [&](const double sw[3], double dtd) {
+#pragma unroll
+        for (int mw = 0; mw < 3; mw++) {
+            if constexpr (FAST) {
+                smax = fast::vmax(smax, fabs(sw[mw]));
+            } else {
+                const double v = dtd * sw[mw];
+                cfl = fmaxf64(cfl, v);
+                cfl = fmaxf64(cfl, -v);
+            }
+        }
+    };
     // A face's own compressed waves go to LDS for its neighbours' limiter and
     // are read back from there by the face itself, so that they do not stay
     // in registers while the other slots solve their Riemann problems.
     double Sr[SLOTS][3];
-    // Each cell's velocities, sqrt(g h) and reciprocal depth, once: a position
+    // FAST: each cell's velocities, sqrt(g h) and reciprocal depth, once: a position
     // keeps its own cell's (the right-hand cell of its two faces and the cell of
     // both transverse splits) and hands them to the face on its right and the
     // one above, whose left-hand cell it is.  (Values of dry cells are garbage
@@ -255,31 +199,33 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
     // increments' place, which is free until the limiter, or in the waves'.
     constexpr bool LF = !FREG && 4 * NPOS <= 6 * G::NF;
     double* const LC = LF ? F : E;
-    const auto put_cell = [&](double* at, const CellVel& c) {
+    const auto put_cell = [&](double* at, const fast::CellVel& c) {
         at[0] = c.u;
         at[NPOS] = c.v;
         at[2 * NPOS] = c.sg;
         at[3 * NPOS] = c.y;
     };
-    const auto get_cell = [&](const double* at) { return CellVel{at[0], at[NPOS], at[2 * NPOS], at[3 * NPOS]}; };
-    const auto cell_of = [&](int k) { return cell_velocity<FAST>(T[k], T[NP2 + k], T[2 * NP2 + k], g); };
+    const auto get_cell = [&](const double* at) { return fast::CellVel{at[0], at[NPOS], at[2 * NPOS], at[3 * NPOS]}; };
+    const auto cell_of = [&](int k) { return fast::cell_velocity(T[k], T[NP2 + k], T[2 * NP2 + k], g); };
     // the cells left of column 0 and below row 0 belong to no position: lanes of
     // the last wave, which has the fewest positions, form them
     const int edge = tid - (NT - 64);
     static_assert(G::PY <= 64 && PX <= 64, "one wave forms an edge's cells");
-    CellVel C[SLOTS], CL[SLOTS];
+    fast::CellVel C[SLOTS], CL[SLOTS];
+    if constexpr (FAST) {
 #pragma unroll
-    for (int s = 0; s < SLOTS; s++)
-        if (in[s]) {
-            C[s] = cell_of(G::ti(pi[s], pj[s]));
-            if (pi[s] < PX - 1) put_cell(LC + tid + s * NT + 1, C[s]);
-        }
-    if (edge >= 0 && edge < G::PY) put_cell(LC + edge * PX, cell_of(G::ti(-1, edge)));
-    __syncthreads();
+        for (int s = 0; s < SLOTS; s++)
+            if (in[s]) {
+                C[s] = cell_of(G::ti(pi[s], pj[s]));
+                if (pi[s] < PX - 1) put_cell(LC + tid + s * NT + 1, C[s]);
+            }
+        if (edge >= 0 && edge < G::PY) put_cell(LC + edge * PX, cell_of(G::ti(-1, edge)));
+        __syncthreads();
 #pragma unroll
-    for (int s = 0; s < SLOTS; s++)
-        if (in[s]) CL[s] = get_cell(LC + tid + s * NT);
-    if (!LF) __syncthreads();
+        for (int s = 0; s < SLOTS; s++)
+            if (in[s]) CL[s] = get_cell(LC + tid + s * NT);
+        if (!LF) __syncthreads();
+    }
     double AP[SLOTS][3], AM[SLOTS][3], GA[SLOTS][3], GB[SLOTS][3];
     double FX[FREG ? SLOTS : 1][6];  // FREG: the position's x-face increments (faddm, faddp)
 
@@ -291,10 +237,16 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         double wc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         if (in[s] && j <= TY + 1) {
             const int kL = G::ti(i - 1, j), kR = G::ti(i, j);
-            rpn2_face<FAST>(T[kL], T[NP2 + kL], T[2 * NP2 + kL], T[3 * NP2 + kL],
-                            T[kR], T[NP2 + kR], T[2 * NP2 + kR], T[3 * NP2 + kR], CL[s], C[s], P, sw, wc);
-#pragma unroll
-            for (int mw = 0; mw < 3; mw++) smax = vmax<FAST>(smax, fabs(sw[mw]));
+            if constexpr (FAST) {
+                fast::rpn2_face(T[kL], T[NP2 + kL], T[2 * NP2 + kL], T[3 * NP2 + kL],
+                                T[kR], T[NP2 + kR], T[2 * NP2 + kR], T[3 * NP2 + kR], CL[s], C[s], P, sw, wc);
+            } else {
+                double w[3][3];
+                rpn2_face(T[kL], T[NP2 + kL], T[2 * NP2 + kL], T[3 * NP2 + kL],
+                          T[kR], T[NP2 + kR], T[2 * NP2 + kR], T[3 * NP2 + kR], P, sw, w);
+                compress(w, wc);
+            }
+            fold_speeds(sw, dtdx);
         }
         Sr[s][0] = sw[0]; Sr[s][1] = sw[1]; Sr[s][2] = sw[2];
         if (in[s]) {
@@ -305,8 +257,10 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
     }
     __syncthreads();
 
-    double cfl = dtdx * smax;
-    smax = 0.0;
+    if constexpr (FAST) {
+        cfl = dtdx * smax;
+        smax = 0.0;
+    }
 
     // ================= x-faces: limiter + corrections =================
 #pragma unroll
@@ -317,7 +271,8 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
             double wc[7], wn[7];
             load_waves<NPOS>(E + p, 1, Sr[s], wc, wn);
             double fxm[3], fxp[3];
-            face_second_order<0, DEF, FAST>(wc, Sr[s], wn, dtdx, P, fxm, fxp, AM[s], AP[s]);
+            if constexpr (FAST) fast::face_second_order<0, DEF>(wc, Sr[s], wn, dtdx, P, fxm, fxp, AM[s], AP[s]);
+            else face_second_order<0, DEF>(wc, Sr[s], wn, dtdx, P, fxm, fxp, AM[s], AP[s]);
             if constexpr (FREG) {
 #pragma unroll
                 for (int k = 0; k < 3; k++) {
@@ -358,23 +313,30 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         for (int k = 0; k < 3; k++) { GA[s][k] = 0.0; GB[s][k] = 0.0; }
         if (transverse && in[s] && i >= 1 && i <= TX && j <= TY + 1) {
             const int kc = G::ti(i, j);
-            const Rpt2Cell R = rpt2_setup<FAST>(T[kc], C[s].u, C[s].v, C[s].sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i, j - 1)],
-                                          T[3 * NP2 + G::ti(i, j + 1)], drytol);
+            const double b = T[3 * NP2 + kc], below = T[3 * NP2 + G::ti(i, j - 1)], above = T[3 * NP2 + G::ti(i, j + 1)];
             const double amn[3] = {E[p + 1], E[NPOS + p + 1], E[2 * NPOS + p + 1]};
-            cell_transverse<FAST>(R, amn, AP[s], hdx, GA[s], GB[s]);  // GA = G1 (below), GB = G2 (above)
+            // GA = G1 (below), GB = G2 (above)
+            if constexpr (FAST)
+                fast::cell_transverse(fast::rpt2_setup(T[kc], C[s].u, C[s].v, C[s].sg, b, below, above, drytol), amn, AP[s],
+                                      hdx, GA[s], GB[s]);
+            else
+                cell_transverse(rpt2_setup(T[kc], T[NP2 + kc], T[2 * NP2 + kc], b, below, above, g, drytol), amn, AP[s], hdx,
+                                GA[s], GB[s]);
         }
     }
     __syncthreads();
-    // (with the increments, the cell below each position for the y-faces)
+    // (with the increments, FAST, the cell below each position for the y-faces)
 #pragma unroll
     for (int s = 0; s < SLOTS; s++)
         if (in[s]) {
             const int p = tid + s * NT;
 #pragma unroll
             for (int k = 0; k < 3; k++) E[k * NPOS + p] = GB[s][k];
-            if (pj[s] < G::PY - 1) put_cell(E + 3 * NPOS + p + PX, C[s]);
+            if constexpr (FAST)
+                if (pj[s] < G::PY - 1) put_cell(E + 3 * NPOS + p + PX, C[s]);
         }
-    if (edge >= 0 && edge < PX) put_cell(E + 3 * NPOS + edge, cell_of(G::ti(edge, -1)));
+    if constexpr (FAST)
+        if (edge >= 0 && edge < PX) put_cell(E + 3 * NPOS + edge, cell_of(G::ti(edge, -1)));
     __syncthreads();
     // GT(i, J) = GX2(i, J-1) + GX1(i, J): the x-sweep part of gm and gp at y-face (i, J)
     double GT[SLOTS][3];
@@ -389,7 +351,8 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
 #pragma unroll
             for (int k = 0; k < 3; k++) GT[s][k] = 0.0;
         }
-        if (in[s]) CL[s] = get_cell(E + 3 * NPOS + p);
+        if constexpr (FAST)
+            if (in[s]) CL[s] = get_cell(E + 3 * NPOS + p);
     }
     __syncthreads();
 
@@ -402,12 +365,18 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         if (in[s] && i <= TX + 1) {
             const int kL = G::ti(i, j - 1), kR = G::ti(i, j);
             // direction-local order for y: (h, hv, hu)
-            rpn2_face<FAST>(T[kL], T[2 * NP2 + kL], T[NP2 + kL], T[3 * NP2 + kL],
-                            T[kR], T[2 * NP2 + kR], T[NP2 + kR], T[3 * NP2 + kR],
-                            CellVel{CL[s].v, CL[s].u, CL[s].sg, CL[s].y}, CellVel{C[s].v, C[s].u, C[s].sg, C[s].y},
-                            P, sw, wc);
-#pragma unroll
-            for (int mw = 0; mw < 3; mw++) smax = vmax<FAST>(smax, fabs(sw[mw]));
+            if constexpr (FAST) {
+                fast::rpn2_face(T[kL], T[2 * NP2 + kL], T[NP2 + kL], T[3 * NP2 + kL],
+                                T[kR], T[2 * NP2 + kR], T[NP2 + kR], T[3 * NP2 + kR],
+                                fast::CellVel{CL[s].v, CL[s].u, CL[s].sg, CL[s].y},
+                                fast::CellVel{C[s].v, C[s].u, C[s].sg, C[s].y}, P, sw, wc);
+            } else {
+                double w[3][3];
+                rpn2_face(T[kL], T[2 * NP2 + kL], T[NP2 + kL], T[3 * NP2 + kL],
+                          T[kR], T[2 * NP2 + kR], T[NP2 + kR], T[3 * NP2 + kR], P, sw, w);
+                compress(w, wc);
+            }
+            fold_speeds(sw, dtdy);
         }
         Sr[s][0] = sw[0]; Sr[s][1] = sw[1]; Sr[s][2] = sw[2];
         if (in[s]) {
@@ -429,7 +398,8 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         if (in[s] && i <= TX + 1 && j >= 1 && j <= TY + 1) {
             double wc[7], wn[7], fm[3], fp[3];
             load_waves<NPOS>(E + p, PX, Sr[s], wc, wn);
-            face_second_order<1, DEF, FAST>(wc, Sr[s], wn, dtdy, P, fm, fp, AM[s], AP[s]);
+            if constexpr (FAST) fast::face_second_order<1, DEF>(wc, Sr[s], wn, dtdy, P, fm, fp, AM[s], AP[s]);
+            else face_second_order<1, DEF>(wc, Sr[s], wn, dtdy, P, fm, fp, AM[s], AP[s]);
             // gm = GT + faddm in physical order (h, hu, hv) = local (0, 2, 1)
             GMr[s][0] = GT[s][0] + fm[0];
             GMr[s][1] = GT[s][1] + fm[2];
@@ -461,10 +431,15 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
         for (int k = 0; k < 3; k++) { GA[s][k] = 0.0; GB[s][k] = 0.0; }
         if (transverse && in[s] && i <= TX + 1 && j >= 1 && j <= TY) {
             const int kc = G::ti(i, j);
-            const Rpt2Cell R = rpt2_setup<FAST>(T[kc], C[s].v, C[s].u, C[s].sg, T[3 * NP2 + kc], T[3 * NP2 + G::ti(i - 1, j)],
-                                          T[3 * NP2 + G::ti(i + 1, j)], drytol);
+            const double b = T[3 * NP2 + kc], left = T[3 * NP2 + G::ti(i - 1, j)], right = T[3 * NP2 + G::ti(i + 1, j)];
             const double amn[3] = {E[p + PX], E[NPOS + p + PX], E[2 * NPOS + p + PX]};
-            cell_transverse<FAST>(R, amn, AP[s], hdy, GA[s], GB[s]);  // GA = left (side 1), GB = right (side 2)
+            // GA = left (side 1), GB = right (side 2)
+            if constexpr (FAST)
+                fast::cell_transverse(fast::rpt2_setup(T[kc], C[s].v, C[s].u, C[s].sg, b, left, right, drytol), amn, AP[s], hdy,
+                                      GA[s], GB[s]);
+            else
+                cell_transverse(rpt2_setup(T[kc], T[2 * NP2 + kc], T[NP2 + kc], b, left, right, g, drytol), amn, AP[s], hdy,
+                                GA[s], GB[s]);
         }
     }
     __syncthreads();
@@ -530,7 +505,10 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
                 const double gmt = E[(3 + m) * NPOS + p + PX];
                 qn[m] = T[m * NP2 + k] - dtdx * (fmr - FPr[s][m]) - dtdy * (gmt - GPr[s][m]);
             }
-            if (P.src_term > 0) src2_cell<FAST>(qn[0], qn[1], qn[2], T[3 * NP2 + k], dt, P);
+            if (P.src_term > 0) {
+                if constexpr (FAST) fast::src2_cell(qn[0], qn[1], qn[2], T[3 * NP2 + k], dt, P);
+                else src2_cell(qn[0], qn[1], qn[2], T[3 * NP2 + k], dt, P);
+            }
             dst[pk] = qn[0];
             dst[PNP2 + pk] = qn[1];
             dst[2 * PNP2 + pk] = qn[2];
@@ -542,7 +520,7 @@ __device__ __forceinline__ void step_tile(const double* T, double* E, double* F,
     // ================= CFL and depth reductions =================
     // (the per-patch MAXCFL_CAP is applied by the caller, once per patch; a
     // non-finite new state makes the CFL number NaN, which the cap keeps)
-    cfl = fmaxf64(cfl, dtdy * smax);
+    if constexpr (FAST) cfl = fmaxf64(cfl, dtdy * smax);
     double v = bad ? quiet_nan() : cfl, hmx = hm;
     group_max2<NT>(v, hmx, red, tid);
     if (tid == 0) {
@@ -724,7 +702,7 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
             const int k = G::ti(i, j);
             const int pk = GP::ti(ox + i, oy + j);
             double h = T[k], hu = T[NP2 + k], hv = T[2 * NP2 + k];
-            if (P.src_term > 0) src2_cell<false>(h, hu, hv, T[3 * NP2 + k], dt, P);
+            if (P.src_term > 0) src2_cell(h, hu, hv, T[3 * NP2 + k], dt, P);
             if (valid) {
                 dst[pk] = h;
                 dst[PNP2 + pk] = hu;
@@ -1076,7 +1054,7 @@ __device__ __forceinline__ void dry_item(const BatchArgs* pa, int k, int next, i
         const double h = src[0];
         double hu = src[NP2], hv = src[2 * NP2];
         if (P.src_term > 0)
-            src2_cell<false>(h, hu, hv, a.aux[(size_t)pt * NP2 + G::ti(c % MX + 1, c / MX + 1)], sc->dt, P);
+            src2_cell(h, hu, hv, a.aux[(size_t)pt * NP2 + G::ti(c % MX + 1, c / MX + 1)], sc->dt, P);
         // a NaN depth lands here too: it sets the scenario's CFL maximum
         // to NaN, which stops the scenario at the controller
         if (!finite3(h, hu, hv))
