@@ -143,6 +143,23 @@ __device__ __forceinline__ void group_max2(double& a, double& b, double* red, in
     }
 }
 
+// The bits 0 and 1 that any of the workgroup's NB threads has set, in every
+// thread, past one barrier (LDS written before it is visible after it).
+// (__syncthreads_or tells only whether any value is not zero, and takes three
+// barriers.)  wave_bits: NB / 64 ints; the caller has a barrier between one
+// use's reads and the next one's writes.
+template <int NB>
+__device__ __forceinline__ int workgroup_bits(int bits, int* wave_bits)
+{
+    static_assert(NB % 64 == 0 && NB <= 1024, "whole waves");
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = (__ballot(bits & 1) ? 1 : 0) | (__ballot(bits & 2) ? 2 : 0);
+    if (lane == 0) wave_bits[threadIdx.x >> 6] = wave;
+    __syncthreads();
+    const int all = lane < NB / 64 ? wave_bits[lane] : 0;
+    return (__ballot(all & 1) ? 1 : 0) | (__ballot(all & 2) ? 2 : 0);
+}
+
 // Device memory named as such: an access through a pointer that was itself
 // read from memory would otherwise be a flat one, which also waits for LDS.
 using gdouble = __attribute__((address_space(1))) double;
@@ -636,7 +653,7 @@ __device__ __forceinline__ void load_tile(const RegionSrc* regions, int patch, i
         }
 }
 
-template <int MX, int MY, int TX, int TY, int NT, bool PULL, bool DEF, bool FREG, int LS, typename Hook, typename Ahead>
+template <int MX, int MY, int TX, int TY, int NT, int NPP, bool PULL, bool DEF, bool FREG, int LS, typename Hook, typename Ahead>
 __device__ __forceinline__ void step_patch(double* T, double* E, double* F, double* red, const RegionSrc* regions, int patch,
                            int ox, int oy, const gdouble* q_src, gdouble* q_dst, const gdouble* aux,
                            double dt, double dtdx, double dtdy, const Params& P, double& cfl_res, double& hmax_res,
@@ -688,7 +705,8 @@ __device__ __forceinline__ void step_patch(double* T, double* E, double* F, doub
             T[3 * NP2 + c] = 0.0;
         }
     }
-    const int flags = __syncthreads_or(wet);
+    __shared__ int wave_bits[NT * NPP / 64];
+    const int flags = workgroup_bits<NT * NPP>(wet, wave_bits);
     if (threadIdx.x / 64 == NT / 64 - 1) hook(threadIdx.x % 64);
 
     if (!(flags & 1)) {
@@ -787,7 +805,7 @@ __global__ void __launch_bounds__(NT) k_step(StepArgs a)
     double cfl = 0.0, hm = 0.0;
     const PatchDesc* d = a.desc + patch;
     TileCells<(G::NP2 + NT - 1) / NT> cells;
-    step_patch<MX, MY, TX, TY, NT, false, DEF, FREG>(T, E, F, red, nullptr, patch, ox, oy, src, dst, (const gdouble*)a.aux,
+    step_patch<MX, MY, TX, TY, NT, 1, false, DEF, FREG>(T, E, F, red, nullptr, patch, ox, oy, src, dst, (const gdouble*)a.aux,
                                                      a.dt, uniform(a.dt / d->dx), uniform(a.dt / d->dy), a.P, cfl, hm,
                                                      threadIdx.x, true, cells, false, NoHook(), [] {});
     if (threadIdx.x == 0) {
@@ -943,7 +961,7 @@ __device__ __forceinline__ void wet_item(const BatchArgs* pa, int idx, const Ite
             loaded = true;
         }
     };
-    step_patch<MX, MY, TX, TY, NT, true, DEF, FREG>(T + grp * 4 * G::NP2, E + grp * 7 * G::NPOS,
+    step_patch<MX, MY, TX, TY, NT, NPP, true, DEF, FREG>(T + grp * 4 * G::NP2, E + grp * 7 * G::NPOS,
                                                     F + (FREG ? 0 : grp * 6 * G::NF), red + grp * 2 * (NT / 64),
                                                     hd->region, patch, ox, oy, src, dst, aux,
                                                     uniform(hd->dt), uniform(hd->dtdx), uniform(hd->dtdy), P, cfl, hm,

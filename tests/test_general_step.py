@@ -17,8 +17,9 @@ INNER = (slice(2, -2), slice(2, -2))
 W = 20
 
 
-def special(kind, seed):
-    """(parameters, q, bed) of a 16x16 patch outside the range."""
+def special(kind, seed, W=W):
+    """(parameters, q, bed) of a patch (W cells wide with its ghost cells)
+    outside the range."""
     rng = np.random.default_rng(seed)
     h = 1.0 + rng.random((W, W))
     u = rng.normal(size=(2, W, W))
@@ -44,7 +45,7 @@ def special(kind, seed):
         b[9, 9] = -np.inf
     elif kind == "overflow":      # its square, and with it a wave, is infinite
         u[0][9, 9] = 1e155
-    elif kind.startswith("film"):  # depths down to 1e-200 or 1e-300, all of them wet
+    elif kind.startswith("film"):  # depths down to 1e-250 or 1e-300, all of them wet
         params = dict(dry_tolerance=0.0)
         h = 10.0 ** rng.uniform(-float(kind[5:]), 0.0, (W, W))
         u = u * h * np.sqrt(9.81 * h)
@@ -59,7 +60,7 @@ def special(kind, seed):
 
 
 SPECIAL = ["nan ghost", "nan depth", "nan bed", "inf ghost", "inf transverse ghost", "inf momentum", "inf depth", "inf bed",
-           "-inf bed", "overflow", "film 200", "film 300", "tolerance 1e-250"]
+           "-inf bed", "overflow", "film 250", "film 300", "tolerance 1e-250"]
 
 
 @pytest.fixture
