@@ -743,8 +743,11 @@ try {
         d.scen = -1;
         for (int k = 0; k < 8; k++) d.nbr[k] = GF_NB_STORED;
     }
+    // every slot has its halo sources from the start: a slot that is never
+    // described reads its own cells (gf_pool_describe can leave a gap below p->n)
     if (hipMemcpyAsync(p->desc, p->h_desc.data(), sizeof(PatchDesc) * capacity, hipMemcpyHostToDevice,
                        g.stream) != hipSuccess ||
+        gf::launch_regions(mx, my, p->desc, p->regions, 0, capacity, g.stream) != hipSuccess ||
         hipStreamSynchronize(g.stream) != hipSuccess) {
         fail(GF_EHIP, "descriptor upload failed");
         return nullptr;
