@@ -101,6 +101,7 @@ PROTOTYPES = {
     "gf_pool_autotune": (ct.c_int, [ct.c_void_p, ct.c_int, _ip, _dp]),
     "gf_synchronize": (ct.c_int, []),
     "gf_last_timing": (ct.c_int, [_dp, _dp, _ip]),
+    "gf_pool_graph_captures": (ct.c_longlong, [ct.c_void_p]),
     "gf_pool_stats": (ct.c_int, [ct.c_void_p, ct.POINTER(ct.c_longlong), ct.POINTER(ct.c_longlong),
                                  ct.POINTER(ct.c_longlong), ct.POINTER(ct.c_longlong)]),
     "gf_pool_write_frame": (ct.c_int, [ct.c_void_p, ct.c_int, ct.c_int, ct.c_int, ct.c_char_p, ct.c_int,

@@ -273,14 +273,22 @@ struct gf_pool {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     bool graph_dirty = true;
+    long long graph_captures = 0;          // see gf_pool_graph_captures
     // Resident AMR (gf_pool_set_levels, gf_pool_set_cf_links): every attempt
-    // starts with the multi-level ghost update, one launch per level that has
-    // patches with finer neighbours or a hydrograph side.  The items and links
-    // of the levels and their ranges live in device memory, so a regrid changes
-    // them without a new graph; it is captured again when the set of levels
-    // with a launch changes, which a regrid that keeps the occupied levels does
-    // not.
+    // starts with the multi-level ghost update, one launch for the averaging and
+    // one per pass over the patches with finer neighbours or a hydrograph side
+    // (ghost_passes).  The items of the passes, the links and their numbers live
+    // in device memory, so a regrid changes them without a new graph; it is
+    // captured again when the set of passes with items changes or the items
+    // outgrow their places.
     bool amr = false;
+    // The items are those of an earlier state of the links, scenarios, levels or
+    // descriptors.  They are built by the next call that uses them, not by each
+    // call that changes something: a regrid moves the scenario to its new slots
+    // and sets the links in two calls, and between them the old links lie
+    // outside the scenario, which has other passes (and had the graph captured
+    // twice per regrid).
+    bool ghost_stale = false;
     std::vector<int> h_level;              // [capacity] refinement level per slot (0 when not set)
     std::vector<int> h_links, h_link_level; // the links as given, [n][coarse, fine, side, igrid], and their coarse levels
     std::vector<int> h_inflow;             // the slots of inflow_list
@@ -623,7 +631,14 @@ static int rebuild_ghost_items(gf_pool* p)
     }
     HIPCHK(hipMemcpyAsync(p->d_amr, h.data(), sizeof(int) * h.size(), hipMemcpyHostToDevice, g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
+    p->ghost_stale = false;
     return GF_OK;
+}
+
+// Before any use of the items (outside a stream capture).
+static int current_ghost_items(gf_pool* p)
+{
+    return p->ghost_stale ? rebuild_ghost_items(p) : GF_OK;
 }
 
 // Rebuild the device list of patches with a hydrograph side, and check that
@@ -659,7 +674,8 @@ static int rebuild_inflow(gf_pool* p)
     HIPCHK(hipMemcpyAsync(p->inflow_n, &n, sizeof(int), hipMemcpyHostToDevice, g.stream));
     HIPCHK(hipStreamSynchronize(g.stream));
     p->h_inflow = std::move(list);
-    return p->amr ? rebuild_ghost_items(p) : GF_OK;
+    p->ghost_stale = p->amr;
+    return GF_OK;
 }
 
 gf_pool* gf_pool_create(int mx, int my, int mbc, int capacity)
@@ -1519,6 +1535,7 @@ static int any_active_flag(gf_pool* p, int* any_active)
 static int run_attempts(gf_pool* p, int substeps, int use_graph, int record = -1)
 {
     if (int r = sync_batch_args(p)) return r;
+    if (int r = current_ghost_items(p)) return r;
     const int variant = step_variant(p, p->n), grid = wet_grid(p, variant);
     if (use_graph) {
         if (p->graph_dirty || p->graph_variant != variant) {
@@ -1536,6 +1553,7 @@ static int run_attempts(gf_pool* p, int substeps, int use_graph, int record = -1
             HIPCHK(hipGraphInstantiate(&p->graph_exec, p->graph, nullptr, nullptr, 0));
             p->graph_dirty = false;
             p->graph_variant = variant;
+            p->graph_captures += 1;
         }
         HIPCHK(hipEventRecord(g.ev_begin, g.stream));
         for (int k = 0; k < substeps; k++) HIPCHK(hipGraphLaunch(p->graph_exec, g.stream));
@@ -1639,8 +1657,10 @@ try {
     std::vector<ScenCtrl>& hc = p->h_ctrl;
     HIPCHK(hipMemcpyAsync(hc.data(), p->ctrl, sizeof(ScenCtrl) * p->nscen, hipMemcpyDeviceToHost, g.stream));
     if (int r = reset_dry_age(p, 0, p->capacity)) return r;
-    if (p->amr)  // the ghost update reads the scenario count from them
+    if (p->amr) {  // the ghost update reads the scenario count from the arguments
         if (int r = sync_batch_args(p)) return r;
+        if (int r = current_ghost_items(p)) return r;
+    }
     HIPCHK(hipStreamSynchronize(g.stream));
     double total_ms = 0.0, step_ms = 0.0;
     int launches = 0;
@@ -1890,6 +1910,8 @@ try {
     return GF_OK;
 } GF_CATCH_STATUS
 
+long long gf_pool_graph_captures(const gf_pool* p) { return p ? p->graph_captures : 0; }
+
 int gf_pool_stats(gf_pool* p, long long* active_patches, long long* dry_patches, long long* attempts,
                   long long* steady_patches)
 try {
@@ -2029,6 +2051,7 @@ try {
     if (p->nscen == 0 || p->n == 0) return fail(GF_ESTATE, "no scenario registered");
     if (!p->inflow_error.empty()) return fail(GF_EINVAL, "%s", p->inflow_error.c_str());
     if (int r = sync_batch_args(p)) return r;
+    if (int r = current_ghost_items(p)) return r;
     const int nv = gf::num_variants(p->mx, p->my);
     // The active list of the current states (what the next attempt steps).
     // Each candidate steps it from the accepted buffer into the other one,
@@ -2390,12 +2413,12 @@ try {
 
 // ---- resident AMR ---------------------------------------------------------
 
-static int ensure_amr(gf_pool* p)
+static void ensure_amr(gf_pool* p)
 {
-    if (p->amr) return GF_OK;
+    if (p->amr) return;
     p->amr = true;
     p->graph_dirty = true;
-    return rebuild_ghost_items(p);
+    p->ghost_stale = true;
 }
 
 int gf_pool_set_levels(gf_pool* p, int first, int n, const int* level)
@@ -2406,7 +2429,7 @@ try {
     for (int k = 0; k < n; k++)
         if (level[k] < 0 || level[k] >= kMaxLevels) return fail(GF_EINVAL, "slot %d: level %d not in [0, %d)", first + k, level[k], kMaxLevels);
     const bool was_amr = p->amr;
-    if (int r = ensure_amr(p)) return r;
+    ensure_amr(p);
     bool in_scenario = false;
     for (int k = 0; k < n; k++) {
         in_scenario |= p->h_desc[first + k].scen >= 0;
@@ -2436,7 +2459,7 @@ try {
                             fine[l], p->h_level[fine[l]], coarse[l], p->h_level[coarse[l]]);
         }
     }
-    if (int r = ensure_amr(p)) return r;
+    ensure_amr(p);
     p->h_links.resize(4 * (size_t)n);
     p->h_link_level.resize(n);
     for (int l = 0; l < n; l++) {
@@ -2447,7 +2470,8 @@ try {
         k[3] = side[l] >= 4 ? 0 : igrid[l];
         p->h_link_level[l] = p->h_level[coarse[l]];
     }
-    return rebuild_ghost_items(p);
+    p->ghost_stale = true;
+    return GF_OK;
 } GF_CATCH_STATUS
 
 int gf_pool_ghost_update(gf_pool* p, int buf, double t)
@@ -2455,10 +2479,11 @@ try {
     if (!p) return fail(GF_EINVAL, "pool is NULL");
     if (buf < -1 || buf > 1) return fail(GF_EINVAL, "buffer must be 0, 1 or -1 (each scenario's current one)");
     if (!p->inflow_error.empty()) return fail(GF_EINVAL, "%s", p->inflow_error.c_str());
-    if (int r = ensure_amr(p)) return r;
+    ensure_amr(p);
     // stream-ordered: every call that reads the pool afterwards waits for it
     if (buf < 0)
         if (int r = sync_batch_args(p)) return r;
+    if (int r = current_ghost_items(p)) return r;
     return enqueue_ghost_update(p, buf, t, false);
 } GF_CATCH_STATUS
 

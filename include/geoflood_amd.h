@@ -449,6 +449,12 @@ int gf_last_timing(double *total_ms, double *step_ms, int *step_launches);
 int gf_pool_stats(gf_pool *pool, long long *active_patches, long long *dry_patches,
                   long long *attempts, long long *steady_patches);
 
+/* Times that gf_pool_run / gf_pool_advance captured this pool's attempt
+ * graph.  A captured graph is replayed until something that it
+ * holds changes: the parameters, the step variant, hydrograph sides where there
+ * were none, or the passes of a resident forest's ghost update. */
+long long gf_pool_graph_captures(const gf_pool *pool);
+
 /* ---- Output: ASCII frames and gauges --------------------------------------
  * Replaces fc2d_geoclaw_output_ascii (fc2d_geoclaw_output_ascii.c:39-114)
  * with its Fortran writers fc2d_geoclaw_fort_write_header / _write_file
