@@ -257,6 +257,7 @@ struct gf_pool {
     int* dry_age = nullptr;                // [capacity] steady dry patches (gf::DRY_STEADY)
     int variant = -1;                      // step variant chosen by the caller or the autotuner (-1: default_variant)
     int graph_variant = -1;                // variant of the captured graph
+    int grid_variant = -1, grid = 0;       // workgroups of the persistent step kernel (wet_grid) and their variant
     int* inflow_list = nullptr;            // [capacity] patches with a hydrograph side
     int* inflow_n = nullptr;               // [1] entries of inflow_list
     bool has_inflow = false;               // inflow_list is not empty (the graph launches k_inflow)
@@ -1442,10 +1443,14 @@ static int sync_batch_args(gf_pool* p)
 }
 
 // Workgroups of the persistent step kernel: every CU filled to the
-// variant's occupancy.
-static int wet_grid(const gf_pool* p, int variant)
+// variant's occupancy (kept: the runtime computes it anew at every question).
+static int wet_grid(gf_pool* p, int variant)
 {
-    return g.num_cu * gf::wet_occupancy(p->mx, p->my, variant);
+    if (p->grid_variant != variant) {
+        p->grid = g.num_cu * gf::wet_occupancy(p->mx, p->my, variant);
+        p->grid_variant = variant;
+    }
+    return p->grid;
 }
 
 // The multi-level ghost update of a resident AMR pool, which leaves what
