@@ -476,6 +476,11 @@ long long gf_pool_bytes(int mx, int my, int mbc, int capacity)
     return per * capacity + staging;
 }
 
+// The step's work tables, per patch, which gf_pool_bytes leaves out: halo
+// sources, the other queues' CFL maxima, tile folds and the hydrograph list.
+constexpr long long kTableBytes = gf::REGIONS * (long long)sizeof(gf::RegionSrc) + 8 * (gf::QUEUES - 1) + 8 + 8 + 4 + 4;
+static_assert(kTableBytes == 224, "the figure in geoflood_amd.h");
+
 // Forget the steady-dry history of slots [first, first + n) after a write
 // of their state, descriptors or parameters from outside the batched step.
 static int reset_dry_age(gf_pool* p, int first, int n)
@@ -751,7 +756,7 @@ try {
     if (!ok) {
         (void)hipGetLastError();
         fail(GF_ENOMEM, "pool allocation of %d patches (%lld bytes) failed", capacity,
-             gf_pool_bytes(mx, my, mbc, capacity));
+             gf_pool_bytes(mx, my, mbc, capacity) + kTableBytes * capacity);
         return nullptr;
     }
     p->h_desc.resize(capacity);

@@ -1,5 +1,5 @@
-// gf_exact.h -- correctly rounded quotients and square roots of the step's
-// inner loops, without the range handling of the general operations.
+// gf_exact.h -- quotients and square roots of the step's inner loops with the
+// bits of the general operations, without their range handling.
 //
 // The step kernel is bound by VALU issue, and its ~50 divisions and ~10
 // square roots per cell were a third of the instructions: `a / b` costs 11
@@ -12,16 +12,19 @@
 //  * quotients with one denominator share its reciprocal: each further one is
 //    a product and one residual correction (3 instructions).
 //
-// Correct rounding.  y is the reciprocal of b after two Newton steps from a
-// seed good to 20 bits or better: its error before the last rounding is below
-// 2^-80, so y is 1/b rounded (or a neighbour of a tie).  q0 = a y is then
-// within one ulp of a/b, the residual r = a - b q0 is exact in one FMA, and
-// q = q0 + r y rounds to the correctly rounded a/b (P. Markstein, "Computation
-// of elementary functions on the IBM RISC System/6000 processor", IBM J. Res.
-// Dev. 34, 1990; J.-M. Muller et al., Handbook of Floating-Point Arithmetic,
-// 2nd ed., 2018, sections 4.7 and 4.8, also for the square root: a Goldschmidt
-// step and two residual corrections).  The residual is exact when
-// |a| >= 2^-960 or a = 0.  A zero quotient loses the sign of its zero.
+// The same bits.  For `a / b` in double precision the compiler emits, between
+// the two scalings and the fixup, the reciprocal's seed, two Newton steps, the
+// product, its residual and the correction: the operations of recip and quot, in
+// that order; for sqrt, between two scalings, those of root.  Where nothing is
+// scaled or fixed up the results are therefore equal, whatever the seeds are.
+// (The sequences are the published ones: P. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990;
+// J.-M. Muller et al., Handbook of Floating-Point Arithmetic, 2nd ed., 2018,
+// sections 4.7 and 4.8.  With a seed good to 20 bits y is 1/b rounded unless 1/b
+// lies within 2^-80 of the midpoint of two doubles, and q then a/b rounded: the
+// residual is exact when |a| >= 2^-960 or a = 0.  Denominators one or two ulps
+// below a power of two have such reciprocals; there only the equality with `a / b`
+// is claimed.)  A zero quotient loses the sign of its zero.
 //
 // Range.  step_cell_in_range bounds a tile's cells, and
 // step_params_in_range bounds the parameters; a tile that holds anything else

@@ -141,6 +141,8 @@ class Pool:
 
     @staticmethod
     def bytes_for(mx, my, capacity, mbc=MBC) -> int:
+        """HBM of a pool's fields (gf_pool_bytes); the step's work tables take
+        224 bytes a patch more."""
         return int(load().gf_pool_bytes(mx, my, mbc, capacity))
 
     # -- layout ---------------------------------------------------------------
