@@ -9,8 +9,8 @@
 //
 // On the 4096^2 dam break a launch of the 32x32 step kernel (about 2,360 active
 // patches) fell from 1.275e8 to 1.019e8 VALU instructions and from 346 to
-// 284 us (with the other steps of the kernel since: 8.8e7 on 2,244 active
-// patches, 253 us).
+// 284 us (with the other steps of the kernel since: 8.85e7 on 2,244 active
+// patches, 250 us).
 #pragma once
 
 #include "gf_exact.h"

@@ -1102,8 +1102,8 @@ __device__ __forceinline__ void dry_item(const BatchArgs* pa, int k, int next, i
 // compute-bound active items leave when the list runs out.
 // step_waves: the waves per SIMD that the registers must allow.  The kernels
 // whose threads own one position each need 136-143 VGPRs when left to the
-// scheduler and 117-126 without a spill when held to four waves (8x8, 16,384
-// patches: 170-213 us, against 171-220 us before; three waves 171-220 us); 32x32
+// scheduler and 113-125 without a spill when held to four waves (8x8, 16,384
+// patches: 170-213 us, three waves 171-220 us); 32x32
 // tiles are alone on a CU by their LDS, and the two-position kernels spill.
 template <int TX, int TY, int NT>
 constexpr int step_waves()
@@ -2317,16 +2317,16 @@ bool get_variant(int mx, int my, int k, StepVariant* out)
 // Times below: one launch of the batched kernel, every cell wet, 256 CUs.
 //  * 32x32 and 64x64 patches: 16x16 tiles while there are at most two a CU
 //    (the chip is not full: a smaller tile's chain of phases is shorter).
-//    64 patches of 32x32: 18.4 against 27.7 us; 128: 25.5 against 28.2; 192:
-//    45 against 28.9.  16 patches of 64x64: 20.4 against 28.8 us; 32: 26.8
-//    against 30.2; 64: 48 against 32.4.  Else 32x32 tiles of 768 threads
-//    (2,304 patches of 32x32: 217 us; 16x16 tiles 323, 640 threads 262).
+//    64 patches of 32x32: 18.5 against 27.4 us; 128: 24.9 against 28.4; 192:
+//    45 against 29.0.  16 patches of 64x64: 20.1 against 28.5 us; 32: 26.9
+//    against 29.4; 64: 48 against 31.6.  Else 32x32 tiles of 768 threads
+//    (2,304 patches of 32x32: 217 us; 16x16 tiles 322, 640 threads 263).
 //  * 16x16 patches: 384 threads, one position each, until there are six a
-//    CU; then 192 and two, three workgroups a CU more (4,096 patches: 122
-//    against 147 us; 256: 19.5 against 17.2; 1,600: 68.6 against 70.1, and
-//    27.8 against 25.1 where two thirds of them are dry).
-//  * 8x8 patches: the increments in registers (10,000 patches: 101 against
-//    103.5 us).
+//    CU; then 192 and two, three workgroups a CU more (4,096 patches: 120
+//    against 144 us; 256: 19.2 against 16.9; 1,600: 69.8 both, and 27.9 against
+//    25.7 where two thirds of them are dry).
+//  * 8x8 patches: the increments in registers (10,000 patches: 99.8 against
+//    101.8 us).
 // The population on the device is not known here: the patches described bound
 // it.  whole: one tile per patch, for a step in place.
 int default_variant(int mx, int my, int patches, int num_cu, bool whole)
